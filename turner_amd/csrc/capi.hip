@@ -182,9 +182,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     float* __restrict__ out_r, float* __restrict__ out_s, float* __restrict__ out_t,
     uint8_t* __restrict__ occ, unsigned long long* counters, uint32_t* status, uint32_t* work) {
     constexpr bool TIE = REF && !ANY;
-    using WL = std::conditional_t<TIE, CoopLdsTie, CoopLds>;
     __shared__ uint2 stk[kStack * kBlock];
-    __shared__ WL wl[kBlock / 64];
+    __shared__ CoopLds wl[kBlock / 64];
     __shared__ uint32_t red[8];  // [0..6] sums, [7] longest traversal in leaves
     if (COUNT && threadIdx.x < 8) red[threadIdx.x] = 0;
     if (COUNT) __syncthreads();
@@ -208,8 +207,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
             if (ANY) tm = __builtin_nontemporal_load(tmax + k);
             if (COUNT) nrays++;
         },
-        [&](uint32_t k, const Trav& T, bool traversed) {
-            const bool hit = traversed && T.best_id != kInvalidId;
+        [&](uint32_t k, const CoopHit& T) {
+            const bool hit = T.id != kInvalidId;
             if (COUNT) atomicMax(&red[7], T.visits);  // leaves of the longest traversal
             if (REF && (needs_reference(T.d) || (TIE && T.tie))) {
                 if (ANY) occ[k] = 2;
@@ -219,10 +218,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
             if (ANY) {
                 __builtin_nontemporal_store((uint8_t)(hit ? 1 : 0), occ + k);
             } else {
-                __builtin_nontemporal_store(hit ? T.best_id : kInvalidId, out_id + k);
-                __builtin_nontemporal_store(hit ? T.best_r : FLT_MAX, out_r + k);
-                __builtin_nontemporal_store(hit ? T.best_s : 0.f, out_s + k);
-                __builtin_nontemporal_store(hit ? T.best_t : 0.f, out_t + k);
+                __builtin_nontemporal_store(T.id, out_id + k);
+                __builtin_nontemporal_store(T.r, out_r + k);
+                __builtin_nontemporal_store(T.s, out_s + k);
+                __builtin_nontemporal_store(T.t, out_t + k);
             }
         },
         cnt);

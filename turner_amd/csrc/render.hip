@@ -388,7 +388,7 @@ __device__ __forceinline__ void shadow_lit(const RenderArgs& A, const Queues& Q,
 // on the level's fix list.
 template <bool EXH, bool REF>
 __device__ __forceinline__ void trace_body(const RenderArgs& A, const Queues& Q, int level, int buf, uint2* stk,
-                                           std::conditional_t<REF, CoopLdsTie, CoopLds>* wl) {
+                                           CoopLds* wl) {
     const uint32_t n = min(Q.cnt[level], Q.cap);  // overflow is reported, never read
     const float4* qo = Q.o[buf];
     const float4* qd = Q.d[buf];
@@ -403,16 +403,14 @@ __device__ __forceinline__ void trace_body(const RenderArgs& A, const Queues& Q,
             d = make_float3(b.x, b.y, b.z);
             scene = scene_of_pixel(A, __float_as_uint(a.w));
         },
-        [&](uint32_t k, const Trav& T, bool traversed) {
+        [&](uint32_t k, const CoopHit& T) {
             if (REF && (T.tie || needs_reference(T.d))) {
                 hit[k] = make_uint4(kFixId, 0u, 0u, 0u);
                 const uint32_t slot = atomicAdd(Q.cnt + kFixHits + level, 1u);
                 if (slot < kFixCap) Q.fix[slot] = k;
                 return;
             }
-            const bool h = traversed && T.best_id != kInvalidId;
-            hit[k] = make_uint4(h ? T.best_id : kInvalidId, __float_as_uint(h ? T.best_r : FLT_MAX),
-                                __float_as_uint(h ? T.best_s : 0.f), __float_as_uint(h ? T.best_t : 0.f));
+            hit[k] = make_uint4(T.id, __float_as_uint(T.r), __float_as_uint(T.s), __float_as_uint(T.t));
         },
         cnt);
     if (cnt.incomplete) atomicAdd(A.status + 2, 1u);
@@ -422,7 +420,7 @@ template <bool EXH, bool REF>
 __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_trace(
     RenderArgs A, Queues Q, int level, int buf) {
     __shared__ uint2 stk[kRStack * kRBlock];
-    __shared__ std::conditional_t<REF, CoopLdsTie, CoopLds> wl[kRBlock / 64];
+    __shared__ CoopLds wl[kRBlock / 64];
     trace_body<EXH, REF>(A, Q, level, buf, stk, wl);
 }
 
@@ -472,7 +470,7 @@ __device__ __forceinline__ void shadow_body(const RenderArgs& A, const Queues& Q
             tmax = b.w;
             scene = scene_of_pixel(A, __float_as_uint(a.w));
         },
-        [&](uint32_t k, const Trav& T, bool traversed) {
+        [&](uint32_t k, const CoopHit& T) {
             if (REF && needs_reference(T.d)) {
                 float* w = reinterpret_cast<float*>(Q.sd[sb] + k) + 3;
                 *w = __uint_as_float(__float_as_uint(*w) | 0x80000000u);
@@ -480,7 +478,7 @@ __device__ __forceinline__ void shadow_body(const RenderArgs& A, const Queues& Q
                 if (slot < kFixCap) Q.fix[(1 + sb) * kFixCap + slot] = k;
                 return;
             }
-            if (!traversed || T.best_id == kInvalidId) shadow_lit(A, Q, sb, k);
+            if (T.id == kInvalidId) shadow_lit(A, Q, sb, k);
         },
         cnt);
     if (cnt.incomplete) atomicAdd(A.status + 2, 1u);
@@ -712,9 +710,9 @@ __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) vo
             tmax = b.w;
             scene = scene_of_pixel(A, __float_as_uint(a.w));
         },
-        [&](uint32_t k, const Trav& T, bool traversed) {
+        [&](uint32_t k, const CoopHit& T) {
             float4 c = Q.sc[sb][k];
-            if (traversed && T.best_id != kInvalidId) {
+            if (T.id != kInvalidId) {
                 const float si = A.shadow_si;
                 c = make_float4(c.x - c.x * si, c.y - c.y * si, c.z - c.z * si, c.w - c.w * si);
                 const uint32_t child = __float_as_uint(Q.sx[sb][k].x);

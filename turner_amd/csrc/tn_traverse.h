@@ -87,7 +87,6 @@ struct Trav {
     int head, count, restarts;
     uint32_t visits;  // leaves visited
     bool lost;
-    bool tie;  // another triangle was hit at exactly best_r (tie detection only)
     uint32_t best_id;
     float best_r, best_s, best_t;
 };
@@ -193,28 +192,27 @@ __device__ __forceinline__ int leaf_test_mt(const float4* __restrict__ pa, const
 __device__ __forceinline__ bool needs_reference(float3 d) { return d.x == 0.f || d.y == 0.f || d.z == 0.f; }
 
 // Fixes the direction and clips the ray to the root box (kdtree.cpp:519-535)
-// of its scene (the tree of `scene` in a forest).  Returns false when the root
-// box is missed.
-__device__ __forceinline__ bool trav_init(Trav& T, const SceneView& sc, float3 o, float3 d,
-                                          uint32_t scene = 0) {
-    T.o = o;
-    T.d = d;
+// of its scene (the tree of `scene` in a forest): the reciprocal direction,
+// the root node and the parameters [lo, hi] inside the box.  Returns false
+// when the root box is missed.
+__device__ __forceinline__ bool root_clip(const SceneView& sc, float3 o, float3 d, uint32_t scene, float3& dinv,
+                                          uint32_t& root, float& tlo, float& thi) {
     float3 fd = d;
     if (fd.x == 0.f) fd.x = kDirEps;
     if (fd.y == 0.f) fd.y = kDirEps;
     if (fd.z == 0.f) fd.z = kDirEps;
-    T.dinv = make_float3(1 / fd.x, 1 / fd.y, 1 / fd.z);
-    const float3 di = T.dinv;
+    dinv = make_float3(1 / fd.x, 1 / fd.y, 1 / fd.z);
+    const float3 di = dinv;
     float b0[3], b1[3];
     if (sc.roots) {
         const SceneRoot& R = sc.roots[scene];
-        T.root = R.node;
+        root = R.node;
         for (int k = 0; k < 3; ++k) {
             b0[k] = R.bmin[k];
             b1[k] = R.bmax[k];
         }
     } else {
-        T.root = 0;
+        root = 0;
         for (int k = 0; k < 3; ++k) {
             b0[k] = sc.bmin[k];
             b1[k] = sc.bmax[k];
@@ -228,6 +226,18 @@ __device__ __forceinline__ bool trav_init(Trav& T, const SceneView& sc, float3 o
     const float tz1 = (b0[2] - o.z) * di.z, tz2 = (b1[2] - o.z) * di.z;
     lo = fmaxf(lo, fminf(tz1, tz2));
     hi = fminf(hi, fmaxf(tz1, tz2));
+    tlo = lo;
+    thi = hi;
+    return !(hi < lo);
+}
+
+// Starts one ray of a per-lane traversal.  Returns false when the root box is
+// missed.
+__device__ __forceinline__ bool trav_init(Trav& T, const SceneView& sc, float3 o, float3 d) {
+    T.o = o;
+    T.d = d;
+    float lo, hi;
+    const bool inside = root_clip(sc, o, d, 0, T.dinv, T.root, lo, hi);
     T.tenter = lo;
     T.texit = hi;
     T.root_exit = hi;
@@ -239,84 +249,11 @@ __device__ __forceinline__ bool trav_init(Trav& T, const SceneView& sc, float3 o
     T.restarts = 0;
     T.visits = 0;
     T.lost = false;
-    T.tie = false;
     T.best_id = kInvalidId;
     T.best_r = FLT_MAX;
     T.best_s = 0.f;
     T.best_t = 0.f;
-    return !(hi < lo);
-}
-
-// Descends from T.node to the next leaf (T.texit becomes the leaf's exit).
-// Returns the leaf node.
-template <int S, bool COUNT>
-__device__ __forceinline__ uint2 trav_descend(Trav& T, const SceneView& sc, uint2* stk, int stride,
-                                              TraversalCounters& cnt) {
-    static_assert(S > 0 && (S & (S - 1)) == 0, "the circular stack index wraps with & (S - 1)");
-    uint32_t node = T.node;
-    const float tenter = T.tenter;
-    float texit = T.texit;
-    uint2 nd = sc.nodes[node];
-    while ((nd.y & 3u) != 3u) {
-        if (COUNT) cnt.inner++;
-        const uint32_t ax = nd.y & 3u;
-        const float tt = (__uint_as_float(nd.x) - pick(T.o, ax)) * pick(T.dinv, ax);
-        uint32_t nearn = node + 1, farn = nd.y >> 2;
-        if (pick(T.d, ax) < 0.f) {  // fixed direction <= 0 (zeros become +1e-5)
-            const uint32_t tmp = nearn;
-            nearn = farn;
-            farn = tmp;
-        }
-        if (texit < tt) {
-            node = nearn;
-        } else if (tt < tenter) {
-            node = farn;
-        } else {
-            stk[T.head * stride] = make_uint2(farn, __float_as_uint(texit));
-            T.head = (T.head + 1) & (S - 1);
-            if (T.count < S) ++T.count;
-            else T.lost = true;
-            node = nearn;
-            texit = tt;
-        }
-        nd = sc.nodes[node];
-    }
-    if (COUNT) cnt.leaves++;
-    T.node = node;
-    T.texit = texit;
-    return nd;
-}
-
-// After a leaf: early exit, next stack entry or restart.  Returns true when
-// the traversal is complete.
-template <int S, bool EXH, bool ANY>
-__device__ __forceinline__ bool trav_after_leaf(Trav& T, float tmax_any, const uint2* stk,
-                                                int stride, TraversalCounters& cnt) {
-    static_assert(S > 0 && (S & (S - 1)) == 0, "the circular stack index wraps with & (S - 1)");
-    const float texit = T.texit;
-    if (!EXH) {
-        if (!ANY && T.best_id != kInvalidId && T.best_r * kExitMargin < texit) return true;
-        if (ANY && tmax_any * kExitMargin < texit) return true;
-    }
-    if (T.count == 0) {
-        if (!T.lost || !(texit < T.root_exit)) return true;
-        if (++T.restarts > kMaxRestarts) {
-            cnt.incomplete = true;
-            return true;
-        }
-        T.node = T.root;
-        T.tenter = texit;
-        T.texit = T.root_exit;
-        T.lost = false;
-        return false;
-    }
-    T.head = (T.head - 1) & (S - 1);
-    --T.count;
-    const uint2 e = stk[T.head * stride];
-    T.node = e.x;
-    T.tenter = texit;
-    T.texit = __uint_as_float(e.y);
-    return false;
+    return inside;
 }
 
 // One leaf per step: descend to the next leaf, test all of its triangles,
@@ -568,171 +505,300 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
     return x;
 }
 
-// LDS of one wave for the cooperative loop: the closest-hit key of each lane's
-// leaf and the start markers of the pooled pairs of one round.
+// LDS of one wave for the cooperative loop, one entry per lane: the key of
+// the closest hit in the lane's leaf, the start markers of the pooled pairs of
+// one round, the distance at which a second pair of the leaf was hit, and the
+// barycentrics of the best hit so far.
 struct CoopLds {
     unsigned long long slot[64];
     uint32_t mark[64];
+    uint32_t tie[64];
+    float2 st[64];
 };
 
-// With tie detection: per lane also the largest key (~r bits, pair index) of
-// the candidates, i.e. the last pair among those at the smallest distance,
-// and so a second hit at exactly the winner's distance when it differs from
-// the winner.
-struct CoopLdsTie : CoopLds {
-    unsigned long long slot2[64];
+// What a cooperative traversal hands to its caller for one ray: the closest
+// hit (id kInvalidId, r FLT_MAX, s = t = 0 on a miss), or with ANY whether
+// some triangle was hit (id).
+struct CoopHit {
+    float3 d;
+    uint32_t id;
+    float r, s, t;
+    bool tie;         // another triangle was hit at exactly r (TIE)
+    uint32_t visits;  // leaves visited
 };
 
+// One ray of the cooperative loop.  Its stack holds the entries base .. head-1
+// of a circular array of S; base > 0 tells that entries were overwritten.
+struct CoopRay {
+    float3 o, d, dinv;
+    float tenter, texit, root_exit;
+    uint32_t node, root;
+    int head, base, restarts;
+    uint32_t visits;
+    float best_r;
+    uint32_t best_ref;  // reference slot of the best hit
+    bool tie;
+};
 
-// Wave-cooperative traversal loop.  Every round, each lane with a ray
-// descends to its next leaf; then the wave pools the (ray, triangle
-// reference) pairs of all its lanes' leaves and tests them 64 at a time, so a
-// round costs ceil(sum of leaf sizes / 64) tests instead of the largest leaf.
-// Pair p belongs to the lane whose range [excl, incl) of the prefix sum of
-// leaf sizes holds it.  In the round of pairs base..base+63 every lane whose
-// range meets the round writes a marker (round stamp, lane) at its first pair
-// of the round; a prefix maximum of the markers over the lanes gives each
-// pair its owner, whose ray is fetched with ds_bpermute.  A hit is folded
-// into the owner's 64-bit LDS slot with atomicMin on (r, pair index): the
-// minimum is the first of the leaf's closest hits in leaf order, i.e. the
-// reference's strict-< scan (kdtree.cpp:587-605); the owner re-tests that
-// triangle to recover r, s, t.
-// Finished lanes take the next rays of the wave's chunk.
+// Wave-cooperative traversal loop.  Every round, the lanes with a ray descend
+// towards their next leaf; then the wave pools the (ray, triangle reference)
+// pairs of the leaves its lanes have reached and tests them 64 at a time, so
+// a round costs ceil(sum of leaf sizes / 64) tests instead of the largest
+// leaf.  Pair p belongs to the lane whose range [excl, incl) of the prefix
+// sum of leaf sizes holds it.  In the round of pairs base..base+63 every lane
+// whose range meets the round writes a marker (round stamp, lane) at its
+// first pair of the round; a prefix maximum of the markers over the lanes
+// gives each pair its owner, whose ray is fetched with ds_bpermute.  A hit is
+// folded into the owner's 64-bit LDS slot with atomicMin on (r, pair index):
+// the minimum is the first of the leaf's closest hits in leaf order, i.e. the
+// reference's strict-< scan (kdtree.cpp:587-605).  The lane whose key stands
+// after its round's atomics leaves the barycentrics in the owner's entry, so
+// the owner reads nothing but its slot.
+//
+// The loop is bound by the chain of dependent node and record reads a round
+// waits for and by instruction issue (with every lane descending to its leaf
+// each round and refilled at once it issued 12.9 k VALU instructions per 64
+// rays of the 2^24-ray batch, 19 of 64 lanes active on average).  Two rules
+// raise the share of lanes that work:
+//   * a round's descent stops when at most a third of the wave's rays are
+//     still on their way (they go on in the next round): the last lanes of a
+//     round take most of its dependent node reads.  2^24 rays, 1.31 M
+//     triangles: 8.03 ms with no limit, 6.76 (1/8), 6.65 (1/4), 6.68 (1/3),
+//     6.72 (1/2); small and ragged launches are fastest at 1/3;
+//   * finished rays are written out and replaced once kRefill lanes wait: a
+//     ray's start (three divisions) and end run for that many lanes at once
+//     (2^24 rays: 7.39 ms at 1, 6.91 at 8, 6.80 at 16, 6.79 at 24; renders
+//     lose 2 % at 24).
 //   chunk(begin, end): called by all lanes of the wave; returns false when no
 //                      work is left (may update begin/end);
-//   load(k, o, d, tmax, scene), store(k, T, traversed): per-ray I/O (scene:
-//                      the ray's tree in a forest, 0 otherwise).
-// TIE (closest hit, reference leaf test, WL = CoopLdsTie): T.tie tells at the
-// end whether a second triangle was hit at exactly the final best distance
-// (in the same leaf, or in a later leaf at the earlier best); the winner among
-// such ties depends on the tree's visit order.
-template <int S, bool EXH, bool MT, bool ANY, bool COUNT, bool TIE = false, class WL = CoopLds, class Chunk,
-          class Load, class Store>
-__device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int stride,
-                                          WL* wl, Chunk chunk, Load load,
-                                          Store store, TraversalCounters& cnt) {
+//   load(k, o, d, tmax, scene), store(k, hit): per-ray I/O (scene: the ray's
+//                      tree in a forest, 0 otherwise).
+// TIE (closest hit, reference leaf test): hit.tie tells whether a second
+// triangle was hit at exactly the final best distance (in the same leaf, or
+// in a later leaf at the earlier best); the winner among such ties depends on
+// the tree's visit order.
+constexpr int kRefill = 16;
+constexpr int kDescendTail = 3;
+
+template <int S, bool EXH, bool MT, bool ANY, bool COUNT, bool TIE = false, class Chunk, class Load, class Store>
+__device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int stride, CoopLds* wl, Chunk chunk,
+                                          Load load, Store store, TraversalCounters& cnt) {
     static_assert(!TIE || (!ANY && !MT), "tie detection is for the reference leaf test's closest hit");
+    static_assert(S > 0 && (S & (S - 1)) == 0, "the circular stack index wraps with & (S - 1)");
     const uint32_t lane = threadIdx.x & 63u;
     constexpr uint32_t kNone = 0xFFFFFFFFu;
     uint32_t next = 0, end = 0, ray = kNone;
     bool more = true;
-    Trav T;
+    bool live = false;  // the lane's ray is still being traversed
+    CoopRay R;
     float tmx = 0.f;
     for (;;) {
-        const uint64_t idle = __ballot(ray == kNone);
-        if (idle && next >= end && more) more = chunk(next, end);
-        if (idle && next < end) {
-            const uint32_t k = next + lanes_below(idle);
-            next += (uint32_t)__popcll(idle);
-            if (ray == kNone && k < end) {
-                float3 o, d;
-                uint32_t scene = 0;
-                load(k, o, d, tmx, scene);
-                if (trav_init(T, sc, o, d, scene)) ray = k;
-                else store(k, T, false);
+        const uint64_t act = __ballot(live);
+        int nact = __popcll(act);
+        if (nact == 0 || (64 - nact >= kRefill && (more || next < end))) {
+            if (ray != kNone && !live) {
+                CoopHit h;
+                h.d = R.d;
+                h.visits = R.visits;
+                h.tie = TIE && R.tie;
+                h.id = kInvalidId;
+                h.r = FLT_MAX;
+                h.s = h.t = 0.f;
+                if (R.best_ref != kNone) {
+                    h.id = ANY ? 0u : sc.refs[R.best_ref];
+                    if (!ANY) {
+                        const float2 st = wl->st[lane];
+                        h.r = R.best_r;
+                        h.s = st.x;
+                        h.t = st.y;
+                    }
+                }
+                store(ray, h);
+                ray = kNone;
+            }
+            if (next >= end && more) more = chunk(next, end);
+            if (next < end) {
+                const uint32_t k = next + lanes_below(~act);
+                if (!live && k < end) {
+                    float3 o, d;
+                    uint32_t scene = 0;
+                    load(k, o, d, tmx, scene);
+                    R.o = o;
+                    R.d = d;
+                    float lo, hi;
+                    live = root_clip(sc, o, d, scene, R.dinv, R.root, lo, hi);
+                    // node steps take the direction's sign from the reciprocal
+                    // (d = -inf, NaN: as d < 0 decides)
+                    R.dinv.x = copysignf(R.dinv.x, d.x < 0.f ? -1.f : 1.f);
+                    R.dinv.y = copysignf(R.dinv.y, d.y < 0.f ? -1.f : 1.f);
+                    R.dinv.z = copysignf(R.dinv.z, d.z < 0.f ? -1.f : 1.f);
+                    R.tenter = lo;
+                    R.texit = hi;
+                    R.root_exit = hi;
+                    R.node = R.root;
+                    R.head = R.base = R.restarts = 0;
+                    R.visits = 0;
+                    R.best_r = FLT_MAX;
+                    R.best_ref = kNone;
+                    R.tie = false;
+                    ray = k;  // a ray that misses the root box is written out by the next refill
+                }
+                next = min(next + (uint32_t)(64 - nact), end);
+            } else if (nact == 0 && !more) {
+                break;
+            }
+            nact = __popcll(__ballot(live));
+            if (nact == 0) continue;
+        }
+        // phase 1: descend towards the next leaf
+        uint32_t loff = 0, lcnt = 0;
+        bool go = live;
+        const int tail = nact / kDescendTail;
+        for (;;) {
+            const int left = __popcll(__ballot(go));
+            if (left <= tail) break;
+            if (go) {
+                const uint2 nd = sc.nodes[R.node];
+                const uint32_t ax = nd.y & 3u;
+                if (ax == 3u) {
+                    loff = nd.x;
+                    lcnt = nd.y >> 2;
+                    go = false;
+                } else {
+                    if (COUNT) cnt.inner++;
+                    const float di = pick(R.dinv, ax);
+                    const float tt = (__uint_as_float(nd.x) - pick(R.o, ax)) * di;
+                    const bool neg = __float_as_int(di) < 0;  // fixed direction <= 0 (zeros become +1e-5)
+                    const uint32_t lo = R.node + 1u, hi = nd.y >> 2;
+                    const bool past = R.texit < tt;           // near child only
+                    const bool before = !past && tt < R.tenter;  // far child only
+                    const bool both = !past && !before;
+                    if (both) stk[(R.head & (S - 1)) * stride] = make_uint2(neg ? lo : hi, __float_as_uint(R.texit));
+                    R.head += both ? 1 : 0;
+                    R.base = max(R.base, R.head - S);
+                    R.texit = both ? tt : R.texit;
+                    R.node = neg != before ? hi : lo;
+                }
             }
         }
-        if (__ballot(ray != kNone) == 0) {
-            if (!more && next >= end) break;
-            continue;
-        }
-        // phase 1: every active lane descends to its next leaf
-        uint32_t loff = 0, lcnt = 0;
-        if (ray != kNone) {
-            const uint2 nd = trav_descend<S, COUNT>(T, sc, stk, stride, cnt);
-            loff = nd.x;
-            lcnt = nd.y >> 2;
-        }
+        const bool leaf = live && !go;
+        if (COUNT && leaf) cnt.leaves++;
         // phase 2: pooled leaf tests
         const uint32_t incl = wave_scan<false>(lcnt);
-        const uint32_t excl = incl - lcnt;
         const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-        const uint32_t rbase = loff - excl;  // refs index of pair p of this lane: rbase + p
-        const float bound_own = ANY ? tmx : T.best_r;
-        wl->slot[lane] = ~0ull;
-        wl->mark[lane] = 0u;
-        if constexpr (TIE) wl->slot2[lane] = 0ull;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        // owner of pair base + lane; called with all lanes active
-        uint32_t stamp = 0;
-        auto owner_of = [&](uint32_t base) {
-            stamp += 64u;  // above every marker of the earlier rounds
-            if (lcnt != 0 && excl < base + 64u && incl > base)
-                wl->mark[excl > base ? excl - base : 0u] = stamp | lane;
+        if (total) {
+            const uint32_t excl = incl - lcnt;
+            const uint32_t rbase = loff - excl;  // refs index of pair p of this lane: rbase + p
+            const float bound_own = ANY ? tmx : R.best_r;
+            wl->slot[lane] = ~0ull;
+            wl->mark[lane] = 0u;
+            if (TIE) wl->tie[lane] = ~0u;
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            return (int)(wave_scan<true>(wl->mark[lane]) & 63u);
-        };
-        for (uint32_t base = 0; base < total; base += 64) {
-            const uint32_t item = base + lane;
-            const int own = owner_of(base);
-            const uint32_t rb = __shfl(rbase, own, 64);
-            const float3 ro = make_float3(__shfl(T.o.x, own, 64), __shfl(T.o.y, own, 64),
-                                          __shfl(T.o.z, own, 64));
-            const float3 rd = make_float3(__shfl(T.d.x, own, 64), __shfl(T.d.y, own, 64),
-                                          __shfl(T.d.z, own, 64));
-            const float bnd = __shfl(bound_own, own, 64);
-            if (item < total) {
-                const size_t r = rb + item;  // reference slot of the pair
-                float rr, ss, tt;
-                int code = MT ? leaf_test_mt<ANY>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt)
-                              : leaf_test_ref<ANY, TIE>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt);
-                if (COUNT) {
-                    cnt.refs++;
-                    cnt.tests++;
-                    cnt.full += code >= 1 ? 1u : 0u;
+            uint32_t stamp = 0;
+            for (uint32_t base = 0; base < total; base += 64) {
+                stamp += 64u;  // above every marker of the earlier rounds
+                if (lcnt != 0 && excl < base + 64u && incl > base)
+                    wl->mark[excl > base ? excl - base : 0u] = stamp | lane;
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                const uint32_t item = base + lane;
+                const int own = (int)(wave_scan<true>(wl->mark[lane]) & 63u);
+                auto of_owner = [&](float x) {
+                    return __int_as_float(__builtin_amdgcn_ds_bpermute(own << 2, __float_as_int(x)));
+                };
+                const uint32_t rb = (uint32_t)__builtin_amdgcn_ds_bpermute(own << 2, (int)rbase);
+                const float3 ro = make_float3(of_owner(R.o.x), of_owner(R.o.y), of_owner(R.o.z));
+                const float3 rd = make_float3(of_owner(R.d.x), of_owner(R.d.y), of_owner(R.d.z));
+                const float bnd = of_owner(bound_own);
+                if (item < total) {
+                    const size_t r = rb + item;  // reference slot of the pair
+                    float rr, ss, tt;
+                    const int code = MT ? leaf_test_mt<ANY>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt)
+                                        : leaf_test_ref<ANY, TIE>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt);
+                    if (COUNT) {
+                        cnt.refs++;
+                        cnt.tests++;
+                        cnt.full += code >= 1 ? 1u : 0u;
+                    }
+                    if (code >= 2) {
+                        if (ANY) {
+                            wl->slot[own] = 0ull;
+                        } else {
+                            // r >= 0 here; -0 maps to +0 so the key orders like the reference's <
+                            const uint32_t rbits = __float_as_uint(rr + 0.0f);
+                            const unsigned long long key = ((unsigned long long)rbits << 32) | item;
+                            atomicMin(&wl->slot[own], key);
+                            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                            const unsigned long long now = wl->slot[own];
+                            if (now == key) {
+                                if (!TIE || code == 2) wl->st[own] = make_float2(ss, tt);
+                            } else if (TIE && (uint32_t)(now >> 32) == rbits) {
+                                wl->tie[own] = rbits;  // another pair at the smallest distance
+                            }
+                        }
+                    }
                 }
-                if (code >= 2) {
-                    // r >= 0 here; -0 maps to +0 so the key orders like the reference's <
-                    const uint32_t rbits = __float_as_uint(rr + 0.0f);
-                    atomicMin(&wl->slot[own], ((unsigned long long)rbits << 32) | item);
-                    if constexpr (TIE) atomicMax(&wl->slot2[own], ((unsigned long long)(~rbits) << 32) | item);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            const unsigned long long key = wl->slot[lane];
+            if (lcnt && key != ~0ull) {
+                const uint32_t r = rbase + (uint32_t)key, rbits = (uint32_t)(key >> 32);
+                if (ANY) {
+                    R.best_ref = 0u;
+                    live = false;
+                } else {
+                    const bool tied = TIE && wl->tie[lane] == rbits;
+                    if (TIE && R.best_ref != kNone && rbits == __float_as_uint(R.best_r + 0.0f)) {
+                        // The leaf's hits lie only at exactly the current best
+                        // distance: the best stays; tied iff one of them is
+                        // another triangle -- two or more of them (a triangle
+                        // occurs once per leaf), or one that is not the best's
+                        // (a triangle spanning several leaves is met again in
+                        // later ones).
+                        if (tied || sc.refs[r] != sc.refs[R.best_ref]) R.tie = true;
+                    } else {
+                        R.best_r = __uint_as_float(rbits);
+                        R.best_ref = r;
+                        R.tie = tied;
+                        if (rbits == 0u) {  // a distance of zero keeps its sign
+                            float rr, ss, tt;
+                            if (MT) leaf_test_mt<ANY>(sc.lra + 2 * (size_t)r, sc.lrb + 2 * (size_t)r, R.o, R.d, bound_own, rr, ss, tt);
+                            else leaf_test_ref<ANY>(sc.lra + 2 * (size_t)r, sc.lrb + 2 * (size_t)r, R.o, R.d, bound_own, rr, ss, tt);
+                            R.best_r = rr;
+                        }
+                    }
                 }
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const unsigned long long key = wl->slot[lane];
-        unsigned long long key2 = 0ull;
-        if constexpr (TIE) key2 = wl->slot2[lane];
-        // every active lane moves on after its leaf, empty leaves included
-        if (ray != kNone) {
-            // TIE: the leaf's hits lie only at exactly the current best distance
-            // (code 3): the best stays; tied iff one of them is another
-            // triangle -- two or more of them (a triangle occurs once per
-            // leaf), or one that is not the best's (a triangle spanning
-            // several leaves is met again in later ones)
-            if (TIE && lcnt && key != ~0ull && T.best_id != kInvalidId &&
-                (uint32_t)(key >> 32) == __float_as_uint(T.best_r + 0.0f)) {
-                if ((uint32_t)key != (uint32_t)key2 || sc.refs[rbase + (uint32_t)key] != T.best_id) T.tie = true;
-            } else if (lcnt && key != ~0ull) {
-                const size_t r = rbase + (uint32_t)key;
-                const uint32_t id = sc.refs[r];
-                float rr, ss, tt;
-                if (MT) leaf_test_mt<ANY>(sc.lra + 2 * r, sc.lrb + 2 * r, T.o, T.d, bound_own, rr, ss, tt);
-                else leaf_test_ref<ANY>(sc.lra + 2 * r, sc.lrb + 2 * r, T.o, T.d, bound_own, rr, ss, tt);
-                T.best_r = rr;
-                T.best_s = ss;
-                T.best_t = tt;
-                T.best_id = id;
-                // a new best: tied iff the last pair at its distance is another pair
-                if constexpr (TIE)
-                    T.tie = key2 != 0ull && (uint32_t)~(uint32_t)(key2 >> 32) == (uint32_t)(key >> 32) &&
-                            (uint32_t)key2 != (uint32_t)key;
-                if (ANY) {
-                    store(ray, T, true);
-                    ray = kNone;
+        // after the leaf (empty ones included): early exit, next stack entry or restart
+        if (leaf && live) {
+            const float texit = R.texit;
+            bool done = false;
+            if (!EXH) done = (ANY ? tmx : R.best_r) * kExitMargin < texit;  // no hit: FLT_MAX, never below
+            if (!done) {
+                if (R.head == R.base) {
+                    done = R.base == 0 || !(texit < R.root_exit);
+                    if (!done && ++R.restarts > kMaxRestarts) {
+                        cnt.incomplete = true;
+                        done = true;
+                    }
+                    R.node = R.root;
+                    R.texit = R.root_exit;
+                    R.head = R.base = 0;
+                } else {
+                    --R.head;
+                    const uint2 e = stk[(R.head & (S - 1)) * stride];
+                    R.node = e.x;
+                    R.texit = __uint_as_float(e.y);
                 }
-            }
-            if (ray != kNone) {
-                bool done = trav_after_leaf<S, EXH, ANY>(T, tmx, stk, stride, cnt);
-                if (!done && ++T.visits > kMaxLeafVisits) {
+                R.tenter = texit;
+                if (!done && ++R.visits > kMaxLeafVisits) {
                     cnt.incomplete = true;
                     done = true;
                 }
-                if (done) {
-                    if (COUNT) cnt.restarts += T.restarts;
-                    store(ray, T, true);
-                    ray = kNone;
-                }
+            }
+            if (done) {
+                if (COUNT) cnt.restarts += R.restarts;
+                live = false;
             }
         }
     }
