@@ -342,10 +342,12 @@ namespace {
 
 void free_device(tn_scene* sc) {
     (void)hipFree(sc->d_nodes);
+    (void)hipFree(sc->d_treelets);
     (void)hipFree(sc->d_refs);
     (void)hipFree(sc->d_tris);
     (void)hipFree(sc->d_lrec);
     (void)hipFree(sc->d_fnodes);
+    (void)hipFree(sc->d_ftreelets);
     (void)hipFree(sc->d_frefs);
     (void)hipFree(sc->d_flrec);
     (void)hipFree(sc->d_normals);
@@ -363,6 +365,12 @@ void free_device(tn_scene* sc) {
         if (e) (void)hipEventDestroy(e);
 }
 
+int upload_treelets(uint4** dst, const std::vector<DevNode>& nodes) {
+    std::vector<Treelet> t;
+    append_treelets(nodes, 0, t);
+    return dev_upload(dst, reinterpret_cast<const uint4*>(t.data()), 2 * t.size());
+}
+
 int finish_scene(tn_scene* sc, const float* verts9, const float* normals9, const float* albedo4,
                  const float* emission4) {
     const uint32_t n = sc->ntris;
@@ -376,6 +384,7 @@ int finish_scene(tn_scene* sc, const float* verts9, const float* normals9, const
     if ((rc = dev_upload(&sc->d_nodes, reinterpret_cast<const uint2*>(sc->tree.nodes.data()),
                          sc->tree.nodes.size())))
         return rc;
+    if ((rc = upload_treelets(&sc->d_treelets, sc->tree.nodes))) return rc;
     if ((rc = dev_upload(&sc->d_refs, sc->tree.refs.data(), sc->tree.refs.size()))) return rc;
     // device record: (v0, uv) (n, vv) (u, uu) (v, denom), one 64-byte line per triangle
     std::vector<float4> rec((size_t)n * 4);
@@ -395,6 +404,7 @@ int finish_scene(tn_scene* sc, const float* verts9, const float* normals9, const
                               sc->fnodes, sc->frefs, sc->fheight);
         if ((rc = dev_upload(&sc->d_fnodes, reinterpret_cast<const uint2*>(sc->fnodes.data()), sc->fnodes.size())))
             return rc;
+        if ((rc = upload_treelets(&sc->d_ftreelets, sc->fnodes))) return rc;
         if ((rc = dev_upload(&sc->d_frefs, sc->frefs.data(), sc->frefs.size()))) return rc;
         if ((rc = dev_upload<float4>(&sc->d_flrec, nullptr, 4 * sc->frefs.size()))) return rc;
         if ((rc = gather_leaf_records(sc->d_tris, sc->d_frefs, sc->frefs.size(), sc->d_flrec))) return rc;

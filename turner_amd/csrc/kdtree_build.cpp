@@ -833,4 +833,46 @@ bool flat_to_device(const std::vector<uint64_t>& flat, uint32_t ntris, std::vect
     return true;
 }
 
+uint32_t append_treelets(const std::vector<DevNode>& nodes, uint32_t root, std::vector<Treelet>& out) {
+    struct Item {
+        uint32_t node, treelet;
+    };
+    auto pair = [&] {
+        out.resize(out.size() + (out.size() & 1) + 2);
+        return (uint32_t)out.size() - 2;
+    };
+    const uint32_t first = pair();  // the second of the pair stays unused
+    std::vector<Item> todo{{root, first}};
+    while (!todo.empty()) {
+        const Item it = todo.back();
+        todo.pop_back();
+        const DevNode r = nodes[it.node];
+        Treelet t{};
+        t.root_x = r.x;
+        t.root_y = r.y;
+        if ((r.y & 3u) != 3u) {
+            t.root_y = r.y & 3u;
+            const uint32_t kids[2] = {it.node + 1, r.y >> 2};
+            uint32_t y[2];
+            // the right child's pair is pushed first: treelets then follow in
+            // depth-first order, left before right
+            for (int c = 1; c >= 0; --c) {
+                const DevNode k = nodes[kids[c]];
+                y[c] = k.y;
+                if ((k.y & 3u) == 3u) continue;
+                const uint32_t at = pair();
+                y[c] = at << 2 | (k.y & 3u);
+                todo.push_back({k.y >> 2, at + 1});
+                todo.push_back({kids[c] + 1, at});
+            }
+            t.left_x = nodes[kids[0]].x;
+            t.right_x = nodes[kids[1]].x;
+            t.left_y = y[0];
+            t.right_y = y[1];
+        }
+        out[it.treelet] = t;
+    }
+    return first;
+}
+
 }  // namespace tn

@@ -1867,6 +1867,7 @@ struct tn_batch {
     int device = 0, cus = 256;
     uint32_t nscenes = 0;
     uint2* nodes = nullptr;
+    uint4* treelets = nullptr;
     uint32_t* refs = nullptr;
     float4* tris = nullptr;
     float4* lrec = nullptr;  // records per reference (first halves, then second halves)
@@ -1893,6 +1894,7 @@ struct tn_batch {
     tn::RenderGeom geom() const {
         tn::RenderGeom g;
         g.sv.nodes = nodes;
+        g.sv.treelets = treelets;
         g.sv.refs = refs;
         g.sv.tris = tris;
         g.sv.lra = lrec;
@@ -1916,7 +1918,7 @@ namespace tn {
 namespace {
 
 void free_batch(tn_batch* b) {
-    for (void* p : {(void*)b->nodes, (void*)b->refs, (void*)b->tris, (void*)b->lrec, (void*)b->normals,
+    for (void* p : {(void*)b->nodes, (void*)b->treelets, (void*)b->refs, (void*)b->tris, (void*)b->lrec, (void*)b->normals,
                     (void*)b->albedo,
                     (void*)b->emission, (void*)b->emit_ids, (void*)b->emit_cdf, (void*)b->roots,
                     (void*)b->status})
@@ -2146,6 +2148,8 @@ int tn_batch_create(tn_scene* const* scenes, uint32_t n, tn_batch** out) {
             ecdf.insert(ecdf.end(), cdf.begin(), cdf.end());
         }
     }
+    std::vector<Treelet> treelets;
+    for (SceneRoot& r : roots) r.treelet = append_treelets(nodes, r.node, treelets);
     auto fail = [&](hipError_t e, const char* what) {
         free_batch(b);
         delete b;
@@ -2154,6 +2158,7 @@ int tn_batch_create(tn_scene* const* scenes, uint32_t n, tn_batch** out) {
     hipError_t e;
     const size_t nt = std::max<uint64_t>(ntri, 1);
     if ((e = hipMalloc(&b->nodes, std::max<size_t>(nodes.size(), 1) * 8)) != hipSuccess ||
+        (e = hipMalloc(&b->treelets, treelets.size() * sizeof(Treelet))) != hipSuccess ||
         (e = hipMalloc(&b->refs, std::max<size_t>(refs.size(), 1) * 4)) != hipSuccess ||
         (e = hipMalloc(&b->tris, nt * 64)) != hipSuccess || (e = hipMalloc(&b->normals, nt * 36)) != hipSuccess ||
         (e = hipMalloc(&b->albedo, nt * 16)) != hipSuccess || (e = hipMalloc(&b->emission, nt * 16)) != hipSuccess ||
@@ -2164,6 +2169,8 @@ int tn_batch_create(tn_scene* const* scenes, uint32_t n, tn_batch** out) {
         return fail(e, "hipMalloc");
     if ((e = hipMemset(b->status, 0, 4 * sizeof(uint32_t))) != hipSuccess) return fail(e, "hipMemset");
     if ((e = hipMemcpy(b->nodes, nodes.data(), nodes.size() * 8, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(b->treelets, treelets.data(), treelets.size() * sizeof(Treelet), hipMemcpyHostToDevice)) !=
+            hipSuccess ||
         (e = hipMemcpy(b->refs, refs.data(), refs.size() * 4, hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipMemcpy(b->roots, roots.data(), n * sizeof(SceneRoot), hipMemcpyHostToDevice)) != hipSuccess ||
         (!eids.empty() &&

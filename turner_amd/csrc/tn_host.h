@@ -16,6 +16,15 @@ struct DevNode {
     uint32_t x, y;
 };
 
+// Two levels of a tree in 32 bytes, read in one go by the cooperative
+// traversal: a root and, when it is an inner node, its two children.  Node
+// words are those of DevNode except that an inner child's y holds the index of
+// its own left child's treelet (its right child's is the next one) instead of
+// the right child's node index; an inner root's y holds its axis alone.
+struct Treelet {
+    uint32_t root_x, left_x, right_x, root_y, left_y, right_y, pad[2];
+};
+
 struct HostTree {
     std::vector<uint64_t> flat;     // reference FlatNode array (lib/kdtree.h:62-154)
     std::vector<DevNode> nodes;     // device layout
@@ -50,5 +59,10 @@ void refine_reference_tree(const float* verts9, const std::vector<DevNode>& rnod
 // device layout (no reference FlatNode array).
 void build_device_tree(const float* verts9, uint32_t n, bool parallel, std::vector<DevNode>& nodes,
                        std::vector<uint32_t>& refs, float box6[6], uint32_t& height);
+
+// Appends the treelets of the tree at nodes[root] (right children anywhere in
+// `nodes`) to `out` and returns the index of the first one.  Sibling treelets
+// share a 64-byte line.
+uint32_t append_treelets(const std::vector<DevNode>& nodes, uint32_t root, std::vector<Treelet>& out);
 
 }  // namespace tn

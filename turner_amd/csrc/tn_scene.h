@@ -24,6 +24,7 @@ struct tn_scene {
     float emit_area = 0.f;
     // device buffers (owned)
     uint2* d_nodes = nullptr;
+    uint4* d_treelets = nullptr;  // the same tree, two levels per 32 bytes
     uint32_t* d_refs = nullptr;
     float4* d_tris = nullptr;
     float4* d_lrec = nullptr;    // records per reference: 2 x nrefs first halves, then second halves
@@ -35,6 +36,7 @@ struct tn_scene {
     std::vector<uint32_t> frefs;
     uint32_t fheight = 0;
     uint2* d_fnodes = nullptr;
+    uint4* d_ftreelets = nullptr;
     uint32_t* d_frefs = nullptr;
     float4* d_flrec = nullptr;
     float* d_normals = nullptr;  // 9 per triangle
@@ -72,6 +74,7 @@ struct tn_scene {
     tn::SceneView fview() const {
         tn::SceneView v = view();
         v.nodes = d_fnodes;
+        v.treelets = d_ftreelets;
         v.refs = d_frefs;
         v.lra = d_flrec;
         v.lrb = d_flrec ? d_flrec + 2 * frefs.size() : nullptr;
@@ -81,6 +84,7 @@ struct tn_scene {
     tn::SceneView view() const {
         tn::SceneView v;
         v.nodes = d_nodes;
+        v.treelets = d_treelets;
         v.refs = d_refs;
         v.tris = d_tris;
         v.lra = d_lrec;

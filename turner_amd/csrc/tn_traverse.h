@@ -14,7 +14,8 @@
 //
 // GPU-specific machinery:
 //   * nodes are 8 bytes (see DevNode in tn_host.h); a leaf holds an offset
-//     and count into a 32-bit triangle-reference array;
+//     and count into a 32-bit triangle-reference array.  The cooperative
+//     traversal reads the same tree as 32-byte treelets of two levels;
 //   * triangle records are 64 bytes (4 x float4: v0|uv, n|vv, u|uu, v|denom),
 //     one L2 line per triangle for the per-lane gathers;
 //   * the stack is a circular short stack of S entries in LDS, 8 bytes per
@@ -50,16 +51,17 @@ constexpr int kMaxRestarts = 4096;
 constexpr uint32_t kMaxLeafVisits = 1u << 22;
 
 // Root of one tree in a packed forest (many scenes in one node / reference /
-// triangle allocation): its node index and root box.
+// triangle allocation): its node and treelet indices and root box.
 struct SceneRoot {
     uint32_t node;
     float bmin[3];
     float bmax[3];
-    uint32_t pad;
+    uint32_t treelet;
 };
 
 struct SceneView {
     const uint2* nodes;
+    const uint4* treelets;  // the same tree two levels at a time (Treelet of tn_host.h, 2 uint4 each)
     const uint32_t* refs;
     const float4* tris;  // 4 per triangle
     // The same records once per triangle reference, in reference order, as
@@ -192,11 +194,11 @@ __device__ __forceinline__ int leaf_test_mt(const float4* __restrict__ pa, const
 __device__ __forceinline__ bool needs_reference(float3 d) { return d.x == 0.f || d.y == 0.f || d.z == 0.f; }
 
 // Fixes the direction and clips the ray to the root box (kdtree.cpp:519-535)
-// of its scene (the tree of `scene` in a forest): the reciprocal direction,
-// the root node and the parameters [lo, hi] inside the box.  Returns false
-// when the root box is missed.
+// of its scene (the tree of `scene` in a forest): the reciprocal direction and
+// the parameters [tlo, thi] inside the box.  Returns false when the root box
+// is missed.
 __device__ __forceinline__ bool root_clip(const SceneView& sc, float3 o, float3 d, uint32_t scene, float3& dinv,
-                                          uint32_t& root, float& tlo, float& thi) {
+                                          float& tlo, float& thi) {
     float3 fd = d;
     if (fd.x == 0.f) fd.x = kDirEps;
     if (fd.y == 0.f) fd.y = kDirEps;
@@ -206,13 +208,11 @@ __device__ __forceinline__ bool root_clip(const SceneView& sc, float3 o, float3 
     float b0[3], b1[3];
     if (sc.roots) {
         const SceneRoot& R = sc.roots[scene];
-        root = R.node;
         for (int k = 0; k < 3; ++k) {
             b0[k] = R.bmin[k];
             b1[k] = R.bmax[k];
         }
     } else {
-        root = 0;
         for (int k = 0; k < 3; ++k) {
             b0[k] = sc.bmin[k];
             b1[k] = sc.bmax[k];
@@ -231,13 +231,14 @@ __device__ __forceinline__ bool root_clip(const SceneView& sc, float3 o, float3 
     return !(hi < lo);
 }
 
-// Starts one ray of a per-lane traversal.  Returns false when the root box is
-// missed.
+// Starts one ray of a per-lane traversal of a single tree.  Returns false when
+// the root box is missed.
 __device__ __forceinline__ bool trav_init(Trav& T, const SceneView& sc, float3 o, float3 d) {
     T.o = o;
     T.d = d;
     float lo, hi;
-    const bool inside = root_clip(sc, o, d, 0, T.dinv, T.root, lo, hi);
+    const bool inside = root_clip(sc, o, d, 0, T.dinv, lo, hi);
+    T.root = 0;
     T.tenter = lo;
     T.texit = hi;
     T.root_exit = hi;
@@ -529,16 +530,42 @@ struct CoopHit {
 
 // One ray of the cooperative loop.  Its stack holds the entries base .. head-1
 // of a circular array of S; base > 0 tells that entries were overwritten.
+// node: treelet << 2 | (0: its root, 1: the left child, 2: the right child), or
+// kDone.  Flags are bits of words, not bools: the compiler keeps a bool that
+// lives across the loop as a lane mask and spends scalar instructions on
+// merging it at every branch.
+constexpr uint32_t kDone = 0xFFFFFFFFu;
 struct CoopRay {
     float3 o, d, dinv;
     float tenter, texit, root_exit;
     uint32_t node, root;
     int head, base, restarts;
-    uint32_t visits;
+    uint32_t visits;  // leaves visited, kTied: another triangle was hit at exactly best_r
     float best_r;
     uint32_t best_ref;  // reference slot of the best hit
-    bool tie;
 };
+constexpr uint32_t kTied = 0x80000000u;
+
+// One node step of a lane's descent: near child = left iff the direction is
+// positive along the axis, then the three-way decision of kdtree.cpp:540-564;
+// when both children are crossed the far one (left / right as given) goes on
+// the stack.  Returns true for the right child.
+template <int S>
+__device__ __forceinline__ bool coop_step(CoopRay& R, uint32_t split, uint32_t ax, uint32_t left, uint32_t right,
+                                          uint2* stk, int stride) {
+    const float di = pick(R.dinv, ax);
+    const float tt = (__uint_as_float(split) - pick(R.o, ax)) * di;
+    const bool neg = __float_as_int(di) < 0;  // fixed direction <= 0 (zeros become +1e-5)
+    const bool past = R.texit < tt;           // near child only
+    const bool before = tt < R.tenter;        // far child only, unless past
+    if (!past && !before) {
+        stk[(R.head & (S - 1)) * stride] = make_uint2(neg ? left : right, __float_as_uint(R.texit));
+        ++R.head;
+        R.base = max(R.base, R.head - S);
+        R.texit = tt;
+    }
+    return neg != (before && !past);
+}
 
 // Wave-cooperative traversal loop.  Every round, the lanes with a ray descend
 // towards their next leaf; then the wave pools the (ray, triangle reference)
@@ -569,6 +596,10 @@ struct CoopRay {
 //     ray's start (three divisions) and end run for that many lanes at once
 //     (2^24 rays: 7.39 ms at 1, 6.91 at 8, 6.80 at 16, 6.79 at 24; renders
 //     lose 2 % at 24).
+// The descent reads two levels at a time (treelets, 32 bytes: a node and its
+// children), so a leaf is about 2.4 dependent reads away instead of 4.8:
+// 2^24 rays 6.67 -> 5.52 ms, a million visibility queries against 82 k
+// triangles 366 -> 298 us, a 512^2 one-sample pass 2.91 -> 2.63 ms.
 //   chunk(begin, end): called by all lanes of the wave; returns false when no
 //                      work is left (may update begin/end);
 //   load(k, o, d, tmax, scene), store(k, hit): per-ray I/O (scene: the ray's
@@ -577,8 +608,7 @@ struct CoopRay {
 // triangle was hit at exactly the final best distance (in the same leaf, or
 // in a later leaf at the earlier best); the winner among such ties depends on
 // the tree's visit order.
-constexpr int kRefill = 16;
-constexpr int kDescendTail = 3;
+constexpr uint32_t kRefill = 16, kDescendTail = 3;
 
 template <int S, bool EXH, bool MT, bool ANY, bool COUNT, bool TIE = false, class Chunk, class Load, class Store>
 __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int stride, CoopLds* wl, Chunk chunk,
@@ -587,20 +617,22 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
     static_assert(S > 0 && (S & (S - 1)) == 0, "the circular stack index wraps with & (S - 1)");
     const uint32_t lane = threadIdx.x & 63u;
     constexpr uint32_t kNone = 0xFFFFFFFFu;
-    uint32_t next = 0, end = 0, ray = kNone;
-    bool more = true;
-    bool live = false;  // the lane's ray is still being traversed
+    constexpr uint32_t kWalk = 0xFFFFFFFFu;  // leaf size of a lane that is still on its way
+    auto uniform = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+    uint32_t next = 0, end = 0, more = 1;  // the same in all lanes
+    uint32_t ray = kNone;
     CoopRay R;
+    R.node = kDone;
     float tmx = 0.f;
     for (;;) {
-        const uint64_t act = __ballot(live);
-        int nact = __popcll(act);
-        if (nact == 0 || (64 - nact >= kRefill && (more || next < end))) {
-            if (ray != kNone && !live) {
+        uint64_t act = __ballot(R.node != kDone);
+        uint32_t nact = uniform((uint32_t)__popcll(act));
+        if (nact == 0 || (nact <= 64 - kRefill && (more | (uint32_t)(next < end)))) {
+            if (ray != kNone && R.node == kDone) {
                 CoopHit h;
                 h.d = R.d;
-                h.visits = R.visits;
-                h.tie = TIE && R.tie;
+                h.visits = R.visits & ~kTied;
+                h.tie = TIE && (R.visits & kTied);
                 h.id = kInvalidId;
                 h.r = FLT_MAX;
                 h.s = h.t = 0.f;
@@ -616,17 +648,21 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                 store(ray, h);
                 ray = kNone;
             }
-            if (next >= end && more) more = chunk(next, end);
+            if (next >= end && more) {
+                more = uniform(chunk(next, end) ? 1u : 0u);
+                next = uniform(next);
+                end = uniform(end);
+            }
             if (next < end) {
                 const uint32_t k = next + lanes_below(~act);
-                if (!live && k < end) {
+                if (R.node == kDone && k < end) {
                     float3 o, d;
                     uint32_t scene = 0;
                     load(k, o, d, tmx, scene);
                     R.o = o;
                     R.d = d;
                     float lo, hi;
-                    live = root_clip(sc, o, d, scene, R.dinv, R.root, lo, hi);
+                    const bool inside = root_clip(sc, o, d, scene, R.dinv, lo, hi);
                     // node steps take the direction's sign from the reciprocal
                     // (d = -inf, NaN: as d < 0 decides)
                     R.dinv.x = copysignf(R.dinv.x, d.x < 0.f ? -1.f : 1.f);
@@ -635,53 +671,54 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                     R.tenter = lo;
                     R.texit = hi;
                     R.root_exit = hi;
-                    R.node = R.root;
+                    R.root = sc.roots ? sc.roots[scene].treelet << 2 : 0u;
+                    R.node = inside ? R.root : kDone;  // a miss is written out by the next refill
                     R.head = R.base = R.restarts = 0;
                     R.visits = 0;
                     R.best_r = FLT_MAX;
                     R.best_ref = kNone;
-                    R.tie = false;
-                    ray = k;  // a ray that misses the root box is written out by the next refill
+                    ray = k;
                 }
-                next = min(next + (uint32_t)(64 - nact), end);
+                next = min(next + (64u - nact), end);
             } else if (nact == 0 && !more) {
                 break;
             }
-            nact = __popcll(__ballot(live));
+            act = __ballot(R.node != kDone);
+            nact = uniform((uint32_t)__popcll(act));
             if (nact == 0) continue;
         }
-        // phase 1: descend towards the next leaf
-        uint32_t loff = 0, lcnt = 0;
-        bool go = live;
-        const int tail = nact / kDescendTail;
+        // phase 1: descend towards the next leaf, two levels per read
+        uint32_t loff = 0, lcnt = R.node != kDone ? kWalk : 0u;
+        const uint32_t tail = nact / kDescendTail;
         for (;;) {
-            const int left = __popcll(__ballot(go));
-            if (left <= tail) break;
-            if (go) {
-                const uint2 nd = sc.nodes[R.node];
-                const uint32_t ax = nd.y & 3u;
-                if (ax == 3u) {
-                    loff = nd.x;
-                    lcnt = nd.y >> 2;
-                    go = false;
+            if (uniform((uint32_t)__popcll(__ballot(lcnt == kWalk))) <= tail) break;
+            if (lcnt == kWalk) {
+                const uint4* t = sc.treelets + 2 * (size_t)(R.node >> 2);
+                const uint4 a = t[0];  // root_x, left_x, right_x, root_y
+                const uint2 b = *reinterpret_cast<const uint2*>(t + 1);  // left_y, right_y
+                bool right = (R.node & 2u) != 0;
+                uint32_t x = a.x, y = a.w;
+                if ((R.node & 3u) == 0 && (a.w & 3u) != 3u) {
+                    if (COUNT) cnt.inner++;
+                    right = coop_step<S>(R, a.x, a.w & 3u, R.node | 1u, R.node | 2u, stk, stride);
+                    R.node = 1u;  // below the root
+                }
+                if ((R.node & 3u) != 0) {
+                    x = right ? a.z : a.y;
+                    y = right ? b.y : b.x;
+                }
+                if ((y & 3u) == 3u) {
+                    loff = x;
+                    lcnt = y >> 2;
                 } else {
                     if (COUNT) cnt.inner++;
-                    const float di = pick(R.dinv, ax);
-                    const float tt = (__uint_as_float(nd.x) - pick(R.o, ax)) * di;
-                    const bool neg = __float_as_int(di) < 0;  // fixed direction <= 0 (zeros become +1e-5)
-                    const uint32_t lo = R.node + 1u, hi = nd.y >> 2;
-                    const bool past = R.texit < tt;           // near child only
-                    const bool before = !past && tt < R.tenter;  // far child only
-                    const bool both = !past && !before;
-                    if (both) stk[(R.head & (S - 1)) * stride] = make_uint2(neg ? lo : hi, __float_as_uint(R.texit));
-                    R.head += both ? 1 : 0;
-                    R.base = max(R.base, R.head - S);
-                    R.texit = both ? tt : R.texit;
-                    R.node = neg != before ? hi : lo;
+                    const uint32_t kid = y & ~3u;
+                    R.node = kid + (coop_step<S>(R, x, y & 3u, kid, kid + 4u, stk, stride) ? 4u : 0u);
                 }
             }
         }
-        const bool leaf = live && !go;
+        const bool leaf = R.node != kDone && lcnt != kWalk;
+        if (!leaf) lcnt = 0;
         if (COUNT && leaf) cnt.leaves++;
         // phase 2: pooled leaf tests
         const uint32_t incl = wave_scan<false>(lcnt);
@@ -744,7 +781,7 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                 const uint32_t r = rbase + (uint32_t)key, rbits = (uint32_t)(key >> 32);
                 if (ANY) {
                     R.best_ref = 0u;
-                    live = false;
+                    R.node = kDone;
                 } else {
                     const bool tied = TIE && wl->tie[lane] == rbits;
                     if (TIE && R.best_ref != kNone && rbits == __float_as_uint(R.best_r + 0.0f)) {
@@ -754,11 +791,11 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                         // occurs once per leaf), or one that is not the best's
                         // (a triangle spanning several leaves is met again in
                         // later ones).
-                        if (tied || sc.refs[r] != sc.refs[R.best_ref]) R.tie = true;
+                        if (tied || sc.refs[r] != sc.refs[R.best_ref]) R.visits |= kTied;
                     } else {
                         R.best_r = __uint_as_float(rbits);
                         R.best_ref = r;
-                        R.tie = tied;
+                        if (TIE) R.visits = (R.visits & ~kTied) | (tied ? kTied : 0u);
                         if (rbits == 0u) {  // a distance of zero keeps its sign
                             float rr, ss, tt;
                             if (MT) leaf_test_mt<ANY>(sc.lra + 2 * (size_t)r, sc.lrb + 2 * (size_t)r, R.o, R.d, bound_own, rr, ss, tt);
@@ -770,7 +807,7 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
             }
         }
         // after the leaf (empty ones included): early exit, next stack entry or restart
-        if (leaf && live) {
+        if (leaf && (!ANY || R.node != kDone)) {
             const float texit = R.texit;
             bool done = false;
             if (!EXH) done = (ANY ? tmx : R.best_r) * kExitMargin < texit;  // no hit: FLT_MAX, never below
@@ -791,14 +828,14 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                     R.texit = __uint_as_float(e.y);
                 }
                 R.tenter = texit;
-                if (!done && ++R.visits > kMaxLeafVisits) {
+                if (!done && (++R.visits & ~kTied) > kMaxLeafVisits) {
                     cnt.incomplete = true;
                     done = true;
                 }
             }
             if (done) {
                 if (COUNT) cnt.restarts += R.restarts;
-                live = false;
+                R.node = kDone;
             }
         }
     }
