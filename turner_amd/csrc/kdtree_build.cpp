@@ -847,9 +847,7 @@ uint32_t append_treelets(const std::vector<DevNode>& nodes, uint32_t root, std::
         const Item it = todo.back();
         todo.pop_back();
         const DevNode r = nodes[it.node];
-        Treelet t{};
-        t.root_x = r.x;
-        t.root_y = r.y;
+        Treelet t{r.x, r.x, r.x, r.y, r.y, r.y, {0, 0}};  // a leaf root repeats itself below
         if ((r.y & 3u) != 3u) {
             t.root_y = r.y & 3u;
             const uint32_t kids[2] = {it.node + 1, r.y >> 2};

@@ -20,7 +20,8 @@ struct DevNode {
 // traversal: a root and, when it is an inner node, its two children.  Node
 // words are those of DevNode except that an inner child's y holds the index of
 // its own left child's treelet (its right child's is the next one) instead of
-// the right child's node index; an inner root's y holds its axis alone.
+// the right child's node index; an inner root's y holds its axis alone; below a
+// leaf root both children repeat the leaf.
 struct Treelet {
     uint32_t root_x, left_x, right_x, root_y, left_y, right_y, pad[2];
 };

@@ -109,10 +109,9 @@ __device__ __forceinline__ bool certainly_negative(float num, float den) {
 // A candidate is also rejected when r is not below `bound` (closest hit: the
 // current best, which it must beat strictly) or, with ANY, above it.
 // Returns 2 on a hit, 1 for a miss decided after reading the whole record,
-// 0 for a miss decided from its first 32 bytes; with TIE (closest hit) 3 for
-// a hit at exactly r == bound, which does not replace the best.  pa: the
-// record's first half (v0, uv) (n, vv); pc: its second half (u, uu) (v, denom).
-template <bool ANY, bool TIE = false>
+// 0 for a miss decided from its first 32 bytes.  pa: the record's first half
+// (v0, uv) (n, vv); pc: its second half (u, uu) (v, denom).
+template <bool ANY>
 __device__ __forceinline__ int leaf_test_ref(const float4* __restrict__ pa, const float4* __restrict__ pc,
                                              float3 o, float3 d, float bound, float& r, float& s, float& t) {
     const float4 a = pa[0];  // v0, uv
@@ -130,7 +129,7 @@ __device__ __forceinline__ int leaf_test_ref(const float4* __restrict__ pa, cons
     }
     const float rr = nom / den;
     if (rr < 0) return 0;
-    if ((ANY || TIE) ? !(rr <= bound) : !(rr < bound)) return 0;
+    if (ANY ? !(rr <= bound) : !(rr < bound)) return 0;
     const float4 c = pc[0];  // u, uu
     const float4 e = pc[1];  // v, denom
     const float px = o.x + rr * d.x, py = o.y + rr * d.y, pz = o.z + rr * d.z;
@@ -157,6 +156,54 @@ __device__ __forceinline__ int leaf_test_ref(const float4* __restrict__ pa, cons
     r = rr;
     s = ss;
     t = tt;
+    return 2;
+}
+
+// The same test for the cooperative traversal, where a wave runs every stage
+// of it for whichever lanes are left, so a stage costs the same for one lane as
+// for 64.  It makes no rejection before the plane's division (some lane always
+// needs it) and hands out the numerators of s and t instead of the quotients:
+// s = snum / denom and t = tnum / denom are needed for the final hit of a ray
+// only.  The reference's verdict (s < 0, t < 0 or 1 < s + t reject) follows
+// from the numerators when a quotient is certainly negative (it cannot
+// underflow to -0) or the sum is above or below 1 by a 2^-18 margin, far beyond
+// the rounding of the divisions and of the sum; the divisions decide the rest.
+// (146 -> 100 VALU instructions per 64 pairs.)  With TIE (closest hit) returns
+// 3 for a hit at exactly r == bound, which does not replace the best.
+template <bool ANY, bool TIE>
+__device__ __forceinline__ int pair_test_ref(const float4* __restrict__ pa, const float4* __restrict__ pc,
+                                             float3 o, float3 d, float bound, float& r, float& snum,
+                                             float& tnum) {
+    const float4 a = pa[0];  // v0, uv
+    const float4 b = pa[1];  // n, vv
+    const float den = b.x * d.x + b.y * d.y + b.z * d.z;
+    const float nom = b.x * (a.x - o.x) + b.y * (a.y - o.y) + b.z * (a.z - o.z);
+    const float rr = nom / den;
+    float uv = a.w, vv = b.w;
+    asm volatile("" : "+v"(uv), "+v"(vv));  // read with the rest of their 16 bytes, not again below
+    // a ray along the plane (den 0) has no hit: the quotient is infinite or NaN
+    if (!(rr >= 0.f) || ((ANY || TIE) ? !(rr <= bound) : !(rr < bound)) || (ANY && den == 0.f)) return 0;
+    const float4 c = pc[0];  // u, uu
+    const float4 e = pc[1];  // v, denom
+    const float px = o.x + rr * d.x, py = o.y + rr * d.y, pz = o.z + rr * d.z;
+    const float wx = px - a.x, wy = py - a.y, wz = pz - a.z;
+    const float wv = wx * e.x + wy * e.y + wz * e.z;
+    const float wu = wx * c.x + wy * c.y + wz * c.z;
+    snum = uv * wv - vv * wu;
+    tnum = uv * wu - c.w * wv;
+    const uint32_t sign = __float_as_uint(e.w) & 0x80000000u;
+    const float s1 = __uint_as_float(__float_as_uint(snum) ^ sign), t1 = __uint_as_float(__float_as_uint(tnum) ^ sign);
+    const float size = fabsf(e.w), sum = s1 + t1, tiny = size * -0x1p-100f;
+    // NaN operands fail every comparison here and go on to the divisions
+    const float one = size >= 0x1p-99f ? size : __builtin_nanf("");
+    if (s1 < tiny || t1 < tiny || sum > one * (1.0f + 0x1p-18f)) return 1;
+    if (!(s1 >= 0.f && t1 >= 0.f && sum < one * (1.0f - 0x1p-18f))) {
+        const float ss = snum / e.w;
+        if (ss < 0) return 1;
+        const float tt = tnum / e.w;
+        if (tt < 0 || 1 < ss + tt) return 1;
+    }
+    r = rr;
     return (TIE && !ANY && rr == bound) ? 3 : 2;
 }
 
@@ -509,7 +556,7 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
 // LDS of one wave for the cooperative loop, one entry per lane: the key of
 // the closest hit in the lane's leaf, the start markers of the pooled pairs of
 // one round, the distance at which a second pair of the leaf was hit, and the
-// barycentrics of the best hit so far.
+// barycentrics (or their numerators) of the best hit so far.
 struct CoopLds {
     unsigned long long slot[64];
     uint32_t mark[64];
@@ -546,25 +593,23 @@ struct CoopRay {
 };
 constexpr uint32_t kTied = 0x80000000u;
 
-// One node step of a lane's descent: near child = left iff the direction is
-// positive along the axis, then the three-way decision of kdtree.cpp:540-564;
-// when both children are crossed the far one (left / right as given) goes on
-// the stack.  Returns true for the right child.
-template <int S>
-__device__ __forceinline__ bool coop_step(CoopRay& R, uint32_t split, uint32_t ax, uint32_t left, uint32_t right,
-                                          uint2* stk, int stride) {
+// The decision of one node step of a lane's descent (kdtree.cpp:540-564): the
+// near child is the left one iff the direction is positive along the axis;
+// past: the near child only, before: the far child only, else both, and the
+// far one goes on the stack.
+struct NodeStep {
+    float t;
+    bool both, right;  // right: the child to go on with
+};
+__device__ __forceinline__ NodeStep node_step(const CoopRay& R, uint32_t split, uint32_t ax) {
     const float di = pick(R.dinv, ax);
-    const float tt = (__uint_as_float(split) - pick(R.o, ax)) * di;
+    NodeStep n;
+    n.t = (__uint_as_float(split) - pick(R.o, ax)) * di;
     const bool neg = __float_as_int(di) < 0;  // fixed direction <= 0 (zeros become +1e-5)
-    const bool past = R.texit < tt;           // near child only
-    const bool before = tt < R.tenter;        // far child only, unless past
-    if (!past && !before) {
-        stk[(R.head & (S - 1)) * stride] = make_uint2(neg ? left : right, __float_as_uint(R.texit));
-        ++R.head;
-        R.base = max(R.base, R.head - S);
-        R.texit = tt;
-    }
-    return neg != (before && !past);
+    const bool past = R.texit < n.t, before = n.t < R.tenter;
+    n.both = !past && !before;
+    n.right = neg != (before && !past);
+    return n;
 }
 
 // Wave-cooperative traversal loop.  Every round, the lanes with a ray descend
@@ -573,33 +618,38 @@ __device__ __forceinline__ bool coop_step(CoopRay& R, uint32_t split, uint32_t a
 // a round costs ceil(sum of leaf sizes / 64) tests instead of the largest
 // leaf.  Pair p belongs to the lane whose range [excl, incl) of the prefix
 // sum of leaf sizes holds it.  In the round of pairs base..base+63 every lane
-// whose range meets the round writes a marker (round stamp, lane) at its
-// first pair of the round; a prefix maximum of the markers over the lanes
-// gives each pair its owner, whose ray is fetched with ds_bpermute.  A hit is
+// whose range meets the round writes its number at its first pair of the
+// round; a prefix maximum of these markers over the lanes gives each pair its
+// owner, whose ray is fetched with ds_bpermute.  A hit is
 // folded into the owner's 64-bit LDS slot with atomicMin on (r, pair index):
 // the minimum is the first of the leaf's closest hits in leaf order, i.e. the
 // reference's strict-< scan (kdtree.cpp:587-605).  The lane whose key stands
 // after its round's atomics leaves the barycentrics in the owner's entry, so
 // the owner reads nothing but its slot.
 //
-// The loop is bound by the chain of dependent node and record reads a round
-// waits for and by instruction issue (with every lane descending to its leaf
-// each round and refilled at once it issued 12.9 k VALU instructions per 64
-// rays of the 2^24-ray batch, 19 of 64 lanes active on average).  Two rules
-// raise the share of lanes that work:
+// What bounds the loop: on the 2^24-ray batch (1.31 M triangles) the lines it
+// reads (27 GB per launch, 5.2 TB/s against 4.7 of a large copy); elsewhere
+// VALU issue (SIMDs 96 % busy before the last of the changes below) and, for
+// launches that leave the chip idle, the chain of dependent reads of the
+// longest rays.  Four rules keep both short:
 //   * a round's descent stops when at most a third of the wave's rays are
 //     still on their way (they go on in the next round): the last lanes of a
-//     round take most of its dependent node reads.  2^24 rays, 1.31 M
-//     triangles: 8.03 ms with no limit, 6.76 (1/8), 6.65 (1/4), 6.68 (1/3),
-//     6.72 (1/2); small and ragged launches are fastest at 1/3;
+//     round take most of its dependent node reads.  2^24 rays: 8.03 ms with
+//     no limit, 6.76 (1/8), 6.65 (1/4), 6.68 (1/3), 6.72 (1/2); small and
+//     ragged launches are fastest at 1/3;
 //   * finished rays are written out and replaced once kRefill lanes wait: a
 //     ray's start (three divisions) and end run for that many lanes at once
 //     (2^24 rays: 7.39 ms at 1, 6.91 at 8, 6.80 at 16, 6.79 at 24; renders
-//     lose 2 % at 24).
-// The descent reads two levels at a time (treelets, 32 bytes: a node and its
-// children), so a leaf is about 2.4 dependent reads away instead of 4.8:
-// 2^24 rays 6.67 -> 5.52 ms, a million visibility queries against 82 k
-// triangles 366 -> 298 us, a 512^2 one-sample pass 2.91 -> 2.63 ms.
+//     lose 2 % at 24);
+//   * the descent reads two levels at a time (treelets, 32 bytes: a node and
+//     its children), so a leaf is about 2.4 dependent reads away instead of
+//     4.8: 6.67 -> 5.52 ms, a million visibility queries against 82 k
+//     triangles 366 -> 298 us, a 512^2 one-sample pass 2.91 -> 2.63 ms;
+//   * no branches where some lane always takes either side, loop exits and
+//     work ranges in scalar registers, no division for a pair that only needs
+//     a verdict (pair_test_ref): a two-level step takes 60 VALU instructions
+//     (was 90), a round of 64 pairs 95 (was 146); 298 -> 257 us, 2.63 -> 2.26
+//     ms, 4099 rays 195 -> 153 us, the 2^24 batch 5.50 -> 5.36 ms.
 //   chunk(begin, end): called by all lanes of the wave; returns false when no
 //                      work is left (may update begin/end);
 //   load(k, o, d, tmax, scene), store(k, hit): per-ray I/O (scene: the ray's
@@ -640,9 +690,10 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                     h.id = ANY ? 0u : sc.refs[R.best_ref];
                     if (!ANY) {
                         const float2 st = wl->st[lane];
+                        const float denom = MT ? 1.f : sc.lrb[2 * (size_t)R.best_ref + 1].w;
                         h.r = R.best_r;
-                        h.s = st.x;
-                        h.t = st.y;
+                        h.s = MT ? st.x : st.x / denom;
+                        h.t = MT ? st.y : st.y / denom;
                     }
                 }
                 store(ray, h);
@@ -690,33 +741,43 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
         // phase 1: descend towards the next leaf, two levels per read
         uint32_t loff = 0, lcnt = R.node != kDone ? kWalk : 0u;
         const uint32_t tail = nact / kDescendTail;
-        for (;;) {
-            if (uniform((uint32_t)__popcll(__ballot(lcnt == kWalk))) <= tail) break;
+        do {
             if (lcnt == kWalk) {
-                const uint4* t = sc.treelets + 2 * (size_t)(R.node >> 2);
-                const uint4 a = t[0];  // root_x, left_x, right_x, root_y
+                // No branches but around the stack writes: every path through
+                // them would be taken by some lane, and merging their results
+                // costs moves.
+                const uint32_t ref = R.node;
+                const uint4* t = sc.treelets + 2 * (size_t)(ref >> 2);
+                const uint4 a = t[0];                                    // root_x, left_x, right_x, root_y
                 const uint2 b = *reinterpret_cast<const uint2*>(t + 1);  // left_y, right_y
-                bool right = (R.node & 2u) != 0;
-                uint32_t x = a.x, y = a.w;
-                if ((R.node & 3u) == 0 && (a.w & 3u) != 3u) {
-                    if (COUNT) cnt.inner++;
-                    right = coop_step<S>(R, a.x, a.w & 3u, R.node | 1u, R.node | 2u, stk, stride);
-                    R.node = 1u;  // below the root
-                }
-                if ((R.node & 3u) != 0) {
-                    x = right ? a.z : a.y;
-                    y = right ? b.y : b.x;
-                }
-                if ((y & 3u) == 3u) {
-                    loff = x;
-                    lcnt = y >> 2;
-                } else {
-                    if (COUNT) cnt.inner++;
-                    const uint32_t kid = y & ~3u;
-                    R.node = kid + (coop_step<S>(R, x, y & 3u, kid, kid + 4u, stk, stride) ? 4u : 0u);
-                }
+                // the root, for lanes that enter there (a leaf root's children repeat it)
+                const uint32_t ax0 = a.w & 3u;
+                const bool root = (ref & 3u) == 0 && ax0 != 3u;
+                const NodeStep n0 = node_step(R, a.x, ax0);
+                const bool push0 = root && n0.both;
+                if (push0)
+                    stk[(R.head & (S - 1)) * stride] =
+                        make_uint2(ref | (n0.right ? 1u : 2u), __float_as_uint(R.texit));
+                R.head += push0 ? 1 : 0;
+                R.texit = push0 ? n0.t : R.texit;
+                // its child, or the child the lane enters at
+                const bool right = root ? n0.right : (ref & 2u) != 0;
+                const uint32_t x = right ? a.z : a.y, y = right ? b.y : b.x;
+                const uint32_t ax1 = y & 3u;
+                const bool inner = ax1 != 3u;
+                const NodeStep n1 = node_step(R, x, ax1);
+                const bool push1 = inner && n1.both;
+                R.node = (y & ~3u) | (n1.right ? 4u : 0u);  // the children's treelets are a pair
+                if (push1) stk[(R.head & (S - 1)) * stride] = make_uint2(R.node ^ 4u, __float_as_uint(R.texit));
+                R.head += push1 ? 1 : 0;
+                R.texit = push1 ? n1.t : R.texit;
+                R.base = max(R.base, R.head - S);
+                loff = x;
+                lcnt = inner ? kWalk : y >> 2;
+                if (COUNT) cnt.inner += (root ? 1u : 0u) + (inner ? 1u : 0u);
             }
-        }
+        } while (uniform((uint32_t)__popcll(__ballot(lcnt == kWalk))) > tail);
+        // R.node of a lane at its leaf is not kDone: its low bits come from a pair index
         const bool leaf = R.node != kDone && lcnt != kWalk;
         if (!leaf) lcnt = 0;
         if (COUNT && leaf) cnt.leaves++;
@@ -724,21 +785,20 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
         const uint32_t incl = wave_scan<false>(lcnt);
         const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         if (total) {
-            const uint32_t excl = incl - lcnt;
-            const uint32_t rbase = loff - excl;  // refs index of pair p of this lane: rbase + p
+            const uint32_t excl = lcnt ? incl - lcnt : ~0u;  // no pairs: meets no round
+            const uint32_t rbase = loff - excl;              // refs index of pair p of this lane: rbase + p
             const float bound_own = ANY ? tmx : R.best_r;
             wl->slot[lane] = ~0ull;
-            wl->mark[lane] = 0u;
             if (TIE) wl->tie[lane] = ~0u;
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            uint32_t stamp = 0;
-            for (uint32_t base = 0; base < total; base += 64) {
-                stamp += 64u;  // above every marker of the earlier rounds
-                if (lcnt != 0 && excl < base + 64u && incl > base)
-                    wl->mark[excl > base ? excl - base : 0u] = stamp | lane;
+            uint32_t base = 0;
+            do {
+                // the first pair of a round always has a marker, so 0 is free for "none"
+                wl->mark[lane] = 0u;
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                if (excl < base + 64u && incl > base) wl->mark[excl > base ? excl - base : 0u] = lane;
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 const uint32_t item = base + lane;
-                const int own = (int)(wave_scan<true>(wl->mark[lane]) & 63u);
+                const int own = (int)wave_scan<true>(wl->mark[lane]);
                 auto of_owner = [&](float x) {
                     return __int_as_float(__builtin_amdgcn_ds_bpermute(own << 2, __float_as_int(x)));
                 };
@@ -748,9 +808,9 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                 const float bnd = of_owner(bound_own);
                 if (item < total) {
                     const size_t r = rb + item;  // reference slot of the pair
-                    float rr, ss, tt;
+                    float rr, ss, tt;  // barycentrics, or their numerators (pair_test_ref)
                     const int code = MT ? leaf_test_mt<ANY>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt)
-                                        : leaf_test_ref<ANY, TIE>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt);
+                                        : pair_test_ref<ANY, TIE>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt);
                     if (COUNT) {
                         cnt.refs++;
                         cnt.tests++;
@@ -774,7 +834,8 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                         }
                     }
                 }
-            }
+                base += 64u;
+            } while (base < total);
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             const unsigned long long key = wl->slot[lane];
             if (lcnt && key != ~0ull) {
@@ -797,10 +858,10 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                         R.best_ref = r;
                         if (TIE) R.visits = (R.visits & ~kTied) | (tied ? kTied : 0u);
                         if (rbits == 0u) {  // a distance of zero keeps its sign
-                            float rr, ss, tt;
-                            if (MT) leaf_test_mt<ANY>(sc.lra + 2 * (size_t)r, sc.lrb + 2 * (size_t)r, R.o, R.d, bound_own, rr, ss, tt);
-                            else leaf_test_ref<ANY>(sc.lra + 2 * (size_t)r, sc.lrb + 2 * (size_t)r, R.o, R.d, bound_own, rr, ss, tt);
-                            R.best_r = rr;
+                            float ss, tt;
+                            const float4 *pa = sc.lra + 2 * (size_t)r, *pc = sc.lrb + 2 * (size_t)r;
+                            if (MT) leaf_test_mt<ANY>(pa, pc, R.o, R.d, bound_own, R.best_r, ss, tt);
+                            else pair_test_ref<ANY, TIE>(pa, pc, R.o, R.d, bound_own, R.best_r, ss, tt);
                         }
                     }
                 }
