@@ -495,11 +495,13 @@ int launch_rays(tn_scene* sc, const float* o3, const float* d3, const float* tma
     // Rays per wave.  The cooperative kernel refills its lanes from one range
     // per wave, so every resident wave (7 per SIMD) gets an equal share of the
     // batch and all finish together (fixed 512-ray chunks left the last of
-    // several generations of waves running on part of the chip); at least 64.
-    // The per-lane kernels take up to kChunk rays per wave.
-    const uint32_t slots = (sc->cus ? sc->cus : 256u) * 4u * kResidentWavesPerSimd;
+    // several generations of waves running on part of the chip); small
+    // batches by small_share.  The per-lane kernels take up to kChunk rays
+    // per wave.
+    const uint32_t simds = (sc->cus ? sc->cus : 256u) * 4u, slots = simds * kResidentWavesPerSimd;
     uint32_t chunk = (tick || leaf) ? rays_per_wave(n, sc->cus)
-                                    : std::max(64u, (uint32_t)(((uint64_t)n + slots - 1) / slots));
+                                    : std::max(small_share(n, simds * kSmallWavesPerSimd, slots),
+                                               (uint32_t)(((uint64_t)n + slots - 1) / slots));
     uint32_t waves = (uint32_t)(((uint64_t)n + chunk - 1) / chunk);
     // Large cooperative launches hand out chunks of about 1/32 of a wave's
     // share from a work slot of the scene, so waves that draw cheap

@@ -327,8 +327,9 @@ __global__ __launch_bounds__(kRBlock) void k_raygen_rays(RenderArgs A, Queues Q,
 }
 
 // Per-wave chunks of a device-counted queue.  The chunk shrinks with the
-// queue (rays_per_wave over a quarter of the grid's waves, so a wave takes
-// about four chunks) to keep every wave busy on short queues.  A queue of at
+// queue (a sixteenth of a wave's share, at least 64; queues of less than 64
+// paths for every second wave by small_share) to keep every wave busy on
+// short queues.  A queue of at
 // most one chunk per wave is dealt statically (wave w takes chunk w) with no
 // atomics: every wave hitting one device-wide counter at once serialises,
 // and on 1-spp passes (262 k paths) dropping those atomics made a pass 21 %
@@ -346,7 +347,7 @@ struct DynamicChunks {
         wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
         uint32_t c = (uint32_t)(((uint64_t)n + 16ull * nwaves - 1) / (16ull * nwaves));
         c = (c + 63u) & ~63u;
-        size = c < 64u ? 64u : (c > (uint32_t)kChunk ? (uint32_t)kChunk : c);
+        size = c <= 64u ? small_share(n, max(nwaves / 2u, 1u), nwaves) : (c > (uint32_t)kChunk ? (uint32_t)kChunk : c);
         nchunks = (n + size - 1) / size;
     }
     __device__ bool operator()(uint32_t& b, uint32_t& e) {

@@ -131,6 +131,22 @@ __host__ __device__ inline uint32_t rays_per_wave(uint32_t n, uint32_t cus) {
     return c < 64u ? 64u : (c > (uint32_t)kChunk ? (uint32_t)kChunk : c);
 }
 
+// Rays per wave (1..64) of a cooperative launch that does not give every wave
+// 64: a round lasts as long as the slowest of the wave's lanes, so a batch too
+// small to fill the chip runs fastest on many waves of few rays -- one each
+// while every ray can have a resident wave of its own (`slots`), then the batch
+// dealt over four waves per SIMD (`waves`), beyond which more waves only share
+// the SIMDs' issue.  Microseconds at 64 rays per wave / by this rule, 20 k
+// triangles, refined tree: 257 rays 108 / 76, 4099 149 / 89, 16384 150 / 114,
+// 65536 167 / 151, 131072 166 / 163; with the share dealt over seven waves per
+// SIMD instead 16384 119, 65536 169, 131072 192, 262144 244 (209).
+constexpr uint32_t kSmallWavesPerSimd = 4;
+__host__ __device__ inline uint32_t small_share(uint32_t n, uint32_t waves, uint32_t slots) {
+    if (n <= slots) return 1u;
+    const uint32_t c = (uint32_t)(((uint64_t)n + waves - 1) / waves);
+    return c < 64u ? c : 64u;
+}
+
 // Traversal over n rays (device arrays): closest hit into id/r/s/t, or with
 // occ != NULL visibility against tmax into occ.
 // fixed_work: zeroed work counters (16 x 9 words) the launch may use instead
