@@ -328,8 +328,11 @@ __global__ __launch_bounds__(kRBlock) void k_raygen_rays(RenderArgs A, Queues Q,
 
 // Per-wave chunks of a device-counted queue.  The chunk shrinks with the
 // queue (a sixteenth of a wave's share, at least 64; queues of less than 64
-// paths for every second wave by small_share) to keep every wave busy on
-// short queues.  A queue of at
+// paths for every fourth wave by small_share: a shadow launch and the other
+// pipeline usually share the chip) to keep every wave busy on short queues.
+// Guided 512x512x8 / raytracer 961x541x4 / one-sample 512^2 pass: 4.60 / 2.26 /
+// 2.24 ms with 64 at least, 4.67 / 2.04 / 2.23 for every second wave, 4.20 /
+// 2.04 / 2.21 for every fourth, 4.54 / 2.06 / 2.25 for every eighth.  A queue of at
 // most one chunk per wave is dealt statically (wave w takes chunk w) with no
 // atomics: every wave hitting one device-wide counter at once serialises,
 // and on 1-spp passes (262 k paths) dropping those atomics made a pass 21 %
@@ -347,7 +350,7 @@ struct DynamicChunks {
         wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
         uint32_t c = (uint32_t)(((uint64_t)n + 16ull * nwaves - 1) / (16ull * nwaves));
         c = (c + 63u) & ~63u;
-        size = c <= 64u ? small_share(n, max(nwaves / 2u, 1u), nwaves) : (c > (uint32_t)kChunk ? (uint32_t)kChunk : c);
+        size = c <= 64u ? small_share(n, max(nwaves / 4u, 1u), nwaves) : (c > (uint32_t)kChunk ? (uint32_t)kChunk : c);
         nchunks = (n + size - 1) / size;
     }
     __device__ bool operator()(uint32_t& b, uint32_t& e) {
