@@ -84,10 +84,10 @@ struct Queues {
     float4* sx[2];  // shadow: radiance at the segment (training records), slot (bits)
     uint32_t cap;   // capacity of each path queue (entries)
     uint32_t scap;  // capacity of the shadow queue
-    // device counters: [0..kMaxLevels) path counts, [kMaxLevels..2k) shadow
-    // counts, [2k..3k) trace work, [3k..4k) shadow work, [4k] overflow,
-    // [4k + 1] raycaster hits, [4k + 2..5k + 2) segments and [5k + 2..6k + 2)
-    // shadow rays a refined traversal handed to the reference tree
+    // device counters: [0..4k) path and shadow counts (path_count,
+    // shadow_count), [4k] overflow, [4k + 1] raycaster hits, [4k + 2..5k + 2)
+    // segments and [5k + 2..6k + 2) shadow rays a refined traversal handed to
+    // the reference tree (k = kMaxLevels)
     uint32_t* cnt;
     // lists of those rays: [0] the segments of the level being traced,
     // [1 + (level & 1)] the shadow rays of a level; kFixCap entries each (a
@@ -234,6 +234,56 @@ __device__ __forceinline__ void accumulate(float4* acc, uint32_t pixel, float4 c
     atomicAdd(p + 3, c.w);
 }
 
+// Paths queued at a level and shadow rays queued by shading it.  What shading
+// level k pushes -- paths of level k + 1 and shadow rays of level k -- is
+// counted in the two halves of one 64-bit word, so one atomic reserves both.
+__host__ __device__ __forceinline__ uint32_t path_count(int level) { return 2u * (uint32_t)level; }
+__host__ __device__ __forceinline__ uint32_t shadow_count(int level) { return 2u * (uint32_t)level + 3u; }
+
+// Queue slots of one block iteration of the shade kernels.  The counters of a
+// level are one address that every XCD's L2 takes in turn; an atomic per wave
+// and queue bound the shade kernels (about 10 ns each: 819,200 segments of the
+// Cornell box took 181 us at level 0), so a block reserves for all of its
+// waves at once: 54 us; 1080p m 4 pass 134.7 -> 121.2 ms, raytracer
+// 961x541x4 2.06 -> 1.82 ms, a batch of six small scenes 1.17 -> 0.96 ms,
+// 512^2 one-sample pass 2.22 -> 2.07 ms; guided 512^2x8 4.52 -> 4.37 ms
+// (a wave per block as before, on the packed word: 4.86).  Called by all
+// threads of the block; the two sets of words alternate by `turn`, so that a
+// wave may run ahead into the next iteration's counts.
+struct BlockSlots {
+    uint32_t n_[2][2][kRBlock / 64];  // [turn][paths, shadow rays][wave]
+    unsigned long long base_[2];
+    __device__ uint32_t& n(uint32_t turn, int kind, uint32_t wave) { return n_[turn][kind][wave]; }
+    __device__ unsigned long long& base(uint32_t turn) { return base_[turn]; }
+};
+template <class Slots>
+__device__ __forceinline__ void reserve_slots(Slots& S, uint32_t turn, uint32_t* cnt, int level, uint32_t paths,
+                                              uint32_t shadows, uint32_t& pbase, uint32_t& sbase) {
+    const uint32_t wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    if ((threadIdx.x & 63u) == 0) {
+        S.n(turn, 0, wave) = paths;
+        S.n(turn, 1, wave) = shadows;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t p = 0, q = 0;
+        for (uint32_t w = 0; w < waves; ++w) {
+            p += S.n(turn, 0, w);
+            q += S.n(turn, 1, w);
+        }
+        S.base(turn) = (p | q) ? atomicAdd(reinterpret_cast<unsigned long long*>(cnt + path_count(level + 1)),
+                                           (unsigned long long)q << 32 | p)
+                               : 0ull;
+    }
+    __syncthreads();
+    pbase = (uint32_t)S.base(turn);
+    sbase = (uint32_t)(S.base(turn) >> 32);
+    for (uint32_t w = 0; w < wave; ++w) {
+        pbase += S.n(turn, 0, w);
+        sbase += S.n(turn, 1, w);
+    }
+}
+
 // Starts the next chunk: [first, first + count) of the call's samples; zeroes
 // the level counters and sets the level-0 count.
 __global__ void k_chunk_begin(uint32_t* cnt, uint32_t* xwork, ChunkState* cs) {
@@ -264,8 +314,8 @@ __global__ void k_chunk_totals(const uint32_t* cnt, unsigned long long* totals, 
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         unsigned long long a = levels < 0 ? cnt[4 * kMaxLevels + 1] : 0, b = 0;
         for (int k = 0; k < levels; ++k) {
-            a += cnt[k];
-            b += cnt[kMaxLevels + k];
+            a += cnt[path_count(k)];
+            b += cnt[shadow_count(k)];
         }
         totals[0] += a;
         totals[1] += b;
@@ -393,7 +443,7 @@ __device__ __forceinline__ void shadow_lit(const RenderArgs& A, const Queues& Q,
 template <bool EXH, bool REF>
 __device__ __forceinline__ void trace_body(const RenderArgs& A, const Queues& Q, int level, int buf, uint2* stk,
                                            CoopLds* wl) {
-    const uint32_t n = min(Q.cnt[level], Q.cap);  // overflow is reported, never read
+    const uint32_t n = min(Q.cnt[path_count(level)], Q.cap);  // overflow is reported, never read
     const float4* qo = Q.o[buf];
     const float4* qd = Q.d[buf];
     uint4* hit = Q.hit;
@@ -438,7 +488,7 @@ __global__ __launch_bounds__(kRBlock) void k_fix_hits(RenderArgs A, Queues Q, in
     const uint32_t m = Q.cnt[kFixHits + level];
     if (m == 0) return;
     const bool scan = m > kFixCap;
-    const uint32_t n = scan ? min(Q.cnt[level], Q.cap) : m;
+    const uint32_t n = scan ? min(Q.cnt[path_count(level)], Q.cap) : m;
     TraversalCounters cnt;
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
         const uint32_t i = scan ? j : Q.fix[j];
@@ -461,7 +511,7 @@ __global__ __launch_bounds__(kRBlock) void k_fix_hits(RenderArgs A, Queues Q, in
 template <bool EXH, bool REF>
 __device__ __forceinline__ void shadow_body(const RenderArgs& A, const Queues& Q, int level, uint2* stk,
                                             CoopLds* wl) {
-    const uint32_t n = min(Q.cnt[kMaxLevels + level], Q.scap);
+    const uint32_t n = min(Q.cnt[shadow_count(level)], Q.scap);
     const int sb = level & 1;
     TraversalCounters cnt;
     coop_loop<kRStack, EXH, false, true, false>(
@@ -506,7 +556,7 @@ __global__ __launch_bounds__(kRBlock) void k_fix_shadows(RenderArgs A, Queues Q,
     if (m == 0) return;
     const bool scan = m > kFixCap;
     const int sb = level & 1;
-    const uint32_t n = scan ? min(Q.cnt[kMaxLevels + level], Q.scap) : m;
+    const uint32_t n = scan ? min(Q.cnt[shadow_count(level)], Q.scap) : m;
     TraversalCounters cnt;
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
         const uint32_t i = scan ? j : Q.fix[(1 + sb) * kFixCap + j];
@@ -550,7 +600,7 @@ __device__ __forceinline__ void push_shadow(const Queues& Q, int sb, uint32_t k,
 // clamp(1 - r / max_visibility, 0, 1).  Hits are counted in cnt[4 kMaxLevels + 1]
 // (the reference counts num_rays on hits only).
 __global__ __launch_bounds__(kRBlock) void k_cast(RenderArgs A, Queues Q, int level, int buf) {
-    const uint32_t n = min(Q.cnt[level], Q.cap);
+    const uint32_t n = min(Q.cnt[path_count(level)], Q.cap);
     uint32_t hits = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const float4 qo = Q.o[buf][i];
@@ -583,13 +633,12 @@ __global__ __launch_bounds__(kRBlock) void k_cast(RenderArgs A, Queues Q, int le
 // max_depth are counted (the reference counts the call that returns {})
 // but not queued.
 __global__ __launch_bounds__(kRBlock) void k_rt_shade(RenderArgs A, Queues Q, int level, int buf) {
-    const uint32_t n = min(Q.cnt[level], Q.cap);
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
+    const uint32_t n = min(Q.cnt[path_count(level)], Q.cap);
+    __shared__ BlockSlots slots;
     const int ob = buf ^ 1;
-    for (uint32_t base = wave * 64u; base < n; base += nwaves * 64u) {
-        const uint32_t i = base + lane;
+    uint32_t turn = 0;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x, turn ^= 1u) {
+        const uint32_t i = base + threadIdx.x;
         bool has_hit = false, spawn = false, shadow = false;
         float3 p2 = make_float3(0, 0, 0), rdir = p2, sdir = p2;
         float sdist = 0.f;
@@ -644,46 +693,37 @@ __global__ __launch_bounds__(kRBlock) void k_rt_shade(RenderArgs A, Queues Q, in
                 shadow = sdist > 0.f;
             }
         }
-        // children (mirror rays)
-        const uint64_t mc = __ballot(spawn);
+        // children (mirror rays) and shadow rays
+        const uint64_t mc = __ballot(spawn), ms = __ballot(shadow);
+        uint32_t cbase, sbase;
+        reserve_slots(slots, turn, Q.cnt, level, (uint32_t)__popcll(mc), (uint32_t)__popcll(ms), cbase, sbase);
         uint32_t child = ~0u;
-        if (mc) {
-            uint32_t cbase = 0;
-            if (lane == 0) cbase = atomicAdd(&Q.cnt[level + 1], (uint32_t)__popcll(mc));
-            cbase = __shfl(cbase, 0);
-            if (spawn && level < A.max_depth) {
-                const uint32_t k = cbase + lanes_below(mc);
-                if (k < Q.cap) {
-                    Q.o[ob][k] = make_float4(p2.x, p2.y, p2.z, __uint_as_float(pixel));
-                    Q.d[ob][k] = make_float4(rdir.x, rdir.y, rdir.z, pathbits);
-                    Q.w[ob][k] = cw;
-                    child = k;
-                } else {
-                    atomicOr(&Q.cnt[4 * kMaxLevels], 1u);
-                }
+        if (spawn && level < A.max_depth) {
+            const uint32_t k = cbase + lanes_below(mc);
+            if (k < Q.cap) {
+                Q.o[ob][k] = make_float4(p2.x, p2.y, p2.z, __uint_as_float(pixel));
+                Q.d[ob][k] = make_float4(rdir.x, rdir.y, rdir.z, pathbits);
+                Q.w[ob][k] = cw;
+                child = k;
+            } else {
+                atomicOr(&Q.cnt[4 * kMaxLevels], 1u);
             }
         }
         // lit test; a hit whose light sits at p2 itself is lit
         if (has_hit && !shadow) accumulate(A.accum, pixel, contrib);
-        const uint64_t ms = __ballot(shadow);
-        if (ms) {
-            uint32_t sbase = 0;
-            if (lane == 0) sbase = atomicAdd(&Q.cnt[kMaxLevels + level], (uint32_t)__popcll(ms));
-            sbase = __shfl(sbase, 0);
-            if (shadow) {
-                const uint32_t k = sbase + lanes_below(ms);
-                if (k < Q.scap) {
-                    // shadowed iff the closest hit is nearer than the light
-                    // (strict): any hit with r <= the float below sdist
-                    const float tmax = __uint_as_float(__float_as_uint(sdist) - 1u);
-                    const int sb = level & 1;
-                    Q.so[sb][k] = make_float4(p2.x, p2.y, p2.z, __uint_as_float(pixel));
-                    Q.sd[sb][k] = make_float4(sdir.x, sdir.y, sdir.z, tmax);
-                    Q.sc[sb][k] = contrib;
-                    Q.sx[sb][k] = make_float4(__uint_as_float(child), 0.f, 0.f, 0.f);
-                } else {
-                    atomicOr(&Q.cnt[4 * kMaxLevels], 1u);
-                }
+        if (shadow) {
+            const uint32_t k = sbase + lanes_below(ms);
+            if (k < Q.scap) {
+                // shadowed iff the closest hit is nearer than the light
+                // (strict): any hit with r <= the float below sdist
+                const float tmax = __uint_as_float(__float_as_uint(sdist) - 1u);
+                const int sb = level & 1;
+                Q.so[sb][k] = make_float4(p2.x, p2.y, p2.z, __uint_as_float(pixel));
+                Q.sd[sb][k] = make_float4(sdir.x, sdir.y, sdir.z, tmax);
+                Q.sc[sb][k] = contrib;
+                Q.sx[sb][k] = make_float4(__uint_as_float(child), 0.f, 0.f, 0.f);
+            } else {
+                atomicOr(&Q.cnt[4 * kMaxLevels], 1u);
             }
         }
     }
@@ -697,7 +737,7 @@ __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) vo
     RenderArgs A, Queues Q, int level, int buf) {
     __shared__ uint2 stk[kRStack * kRBlock];
     __shared__ CoopLds wl[kRBlock / 64];
-    const uint32_t n = min(Q.cnt[kMaxLevels + level], Q.scap);
+    const uint32_t n = min(Q.cnt[shadow_count(level)], Q.scap);
     const int ob = buf ^ 1;
     const int sb = level & 1;
     TraversalCounters cnt;
@@ -731,23 +771,22 @@ __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) vo
     if (cnt.incomplete) atomicAdd(A.status + 2, 1u);
 }
 
-// Shade one level.  GUIDED kernels run one wave per block (the guide's
-// forward pass is separated by block barriers).
-template <bool GUIDED>
+// Shade one level: the block's waves take 64 segments each per iteration.
+// glds: the calling wave's rows for the guide's network (GUIDED).
+template <bool GUIDED, class Slots>
 __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q, int level, int buf,
-                                           uint16_t* glds) {
-    const uint32_t n = min(Q.cnt[level], Q.cap);
+                                           uint16_t* glds, Slots& slots) {
+    const uint32_t n = min(Q.cnt[path_count(level)], Q.cap);
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
     const bool spawn = level < A.max_depth && A.mc > 0;
     const uint32_t m = (uint32_t)max(A.mc, 0);
     const bool cosine = A.flags & TN_RENDER_COSINE;
     const bool area_flag = (A.flags & TN_RENDER_AREA_LIGHTS) != 0;
     const bool records = GUIDED && A.rec_p != nullptr;
     const float inv_pi = 0.318309886183790671538f;
-    for (uint32_t base = wave * 64u; base < n; base += nwaves * 64u) {
-        const uint32_t i = base + lane;
+    uint32_t turn = 0;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+        const uint32_t i = base + threadIdx.x;
         const bool active = i < n;
         bool has_hit = false, has_point = false, has_area = false;
         float4 w = make_float4(0, 0, 0, 0), rho = w;
@@ -890,13 +929,14 @@ __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q,
                 }
             }
         }
-        // shadow rays: wave-aggregated push
+        // shadow rays and unguided children (guided ones are drawn later)
         const uint64_t mp = __ballot(has_point), ma = __ballot(has_area);
+        const uint64_t mh = spawn && !GUIDED ? __ballot(has_hit) : 0ull;
         const uint32_t tot = (uint32_t)(__popcll(mp) + __popcll(ma));
+        uint32_t hbase = 0, sbase = 0;
+        reserve_slots(slots, turn, Q.cnt, level, (uint32_t)__popcll(mh) * m, tot, hbase, sbase);
+        turn ^= 1u;
         if (tot) {
-            uint32_t sbase = 0;
-            if (lane == 0) sbase = atomicAdd(&Q.cnt[kMaxLevels + level], tot);
-            sbase = __shfl(sbase, 0);
             if (has_point) {
                 const uint32_t k = sbase + lanes_below(mp);
                 if (k < Q.scap) push_shadow(Q, level & 1, k, p2, pixel, ldir, ldist, lcontrib, llocal, slot, records);
@@ -917,13 +957,8 @@ __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q,
         onb(nn, b1, b2);
         if (!GUIDED) {
             // children: m per hit (pathtracer.cpp:72-85)
-            const uint64_t mc = __ballot(has_hit);
-            if (!mc) continue;
-            uint32_t cbase = 0;
-            if (lane == 0) cbase = atomicAdd(&Q.cnt[level + 1], (uint32_t)__popcll(mc) * m);
-            cbase = __shfl(cbase, 0);
             if (!has_hit) continue;
-            const uint32_t first = cbase + lanes_below(mc) * m;
+            const uint32_t first = hbase + lanes_below(mh) * m;
             for (uint32_t c = 0; c < m; ++c) {
                 const float u1 = rng_uniform(rng), u2 = rng_uniform(rng);
                 float lx, ly, lz, f;
@@ -961,7 +996,7 @@ __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q,
             guide_forward_wave(A.gv, p, nn, has_hit, gout, glds);
             Mixture M;
             mixture_from(gout + lane * kGOut, M);
-            __syncthreads();  // gout is overwritten by the next iteration's forward pass
+            guide_wave_sync();  // gout is overwritten by the next iteration's forward pass
             for (uint32_t c = 0; c < m; ++c) {
                 const float us = rng_uniform(rng), u0 = rng_uniform(rng), u1 = rng_uniform(rng),
                             u2 = rng_uniform(rng);
@@ -985,9 +1020,9 @@ __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q,
                     f = inv_pi * cos_pdf * invm;
                 }
                 const uint64_t mc = __ballot(ok);
-                uint32_t cbase = 0;
-                if (mc && lane == 0) cbase = atomicAdd(&Q.cnt[level + 1], (uint32_t)__popcll(mc));
-                cbase = __shfl(cbase, 0);
+                uint32_t cbase, none;
+                reserve_slots(slots, turn, Q.cnt, level, (uint32_t)__popcll(mc), 0u, cbase, none);
+                turn ^= 1u;
                 if (records && has_hit) {
                     A.rec_p[slot] = make_float4(p.x, p.y, p.z, cos_pdf);
                     A.rec_n[slot] = make_float4(nn.x, nn.y, nn.z, ok ? 1.f : 0.f);
@@ -1009,10 +1044,25 @@ __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q,
     }
 }
 
-template <bool GUIDED>
-__global__ __launch_bounds__(kRBlock) void k_shade(RenderArgs A, Queues Q, int level, int buf) {
-    __shared__ __align__(16) uint16_t glds[GUIDED ? 64 * (kGStrideIn + kGStrideHid) : 1];
-    shade_body<GUIDED>(A, Q, level, buf, glds);
+// Two waves per block, each with its own 20 KB of rows for the guide's network:
+// four blocks (two waves per SIMD, as the registers allow) fill a CU's 160 KB
+// exactly, so the block's slot words live in the padding behind the hidden
+// rows of its first wave, which nothing else touches.
+constexpr int kGuidedBlock = 128;
+struct RowSlots {
+    uint16_t* rows;  // 16-byte gaps at rows + kGHid, every kGStrideHid
+    __device__ uint32_t& n(uint32_t turn, int kind, uint32_t wave) {
+        return reinterpret_cast<uint32_t*>(rows + turn * kGStrideHid + kGHid)[2 * kind + wave];
+    }
+    __device__ unsigned long long& base(uint32_t turn) {
+        return *reinterpret_cast<unsigned long long*>(rows + (2 + turn) * kGStrideHid + kGHid);
+    }
+};
+static_assert(kGStrideHid - kGHid >= 8 && kGuidedBlock == 128, "two waves' counts fit a row's padding");
+__global__ __launch_bounds__(kGuidedBlock) void k_shade_guided(RenderArgs A, Queues Q, int level, int buf) {
+    __shared__ __align__(16) uint16_t glds[kGuidedBlock / 64][64 * (kGStrideIn + kGStrideHid)];
+    RowSlots slots{glds[0] + 64 * kGStrideIn};
+    shade_body<true>(A, Q, level, buf, glds[threadIdx.x >> 6], slots);
 }
 
 // The unguided shade capped at 72 VGPRs (7 waves per SIMD, 68 bytes of
@@ -1021,8 +1071,8 @@ __global__ __launch_bounds__(kRBlock) void k_shade(RenderArgs A, Queues Q, int l
 // VGPRs: 1157).
 __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_shade_plain(
     RenderArgs A, Queues Q, int level, int buf) {
-    __shared__ uint16_t glds[1];
-    shade_body<false>(A, Q, level, buf, glds);
+    __shared__ BlockSlots slots;
+    shade_body<false>(A, Q, level, buf, nullptr, slots);
 }
 
 // ---------------------------------------------------------- persistent
@@ -1109,7 +1159,7 @@ template <bool EXH>
 __global__ __launch_bounds__(kRBlock) void k_persist(RenderArgs A, Queues Q, int levels) {
     __shared__ uint2 stk[kRStack * kRBlock];
     __shared__ CoopLds wl[kRBlock / 64];
-    __shared__ uint16_t glds[1];
+    __shared__ BlockSlots slots;
     uint32_t gen = 0;
     for (;;) {
         if (blockIdx.x == 0) chunk_begin_block(Q.cnt, Q.xwork, A.cs);
@@ -1123,7 +1173,7 @@ __global__ __launch_bounds__(kRBlock) void k_persist(RenderArgs A, Queues Q, int
         for (int lv = 0; lv < levels; ++lv) {
             trace_body<EXH, false>(A, Q, lv, buf, stk, wl);
             if (!grid_sync(Q.bar, gen)) return;
-            shade_body<false>(A, Q, lv, buf, glds);
+            shade_body<false>(A, Q, lv, buf, nullptr, slots);
             if (!grid_sync(Q.bar, gen)) return;
             shadow_body<EXH, false>(A, Q, lv, stk, wl);
             if (!grid_sync(Q.bar, gen)) return;
@@ -1132,8 +1182,8 @@ __global__ __launch_bounds__(kRBlock) void k_persist(RenderArgs A, Queues Q, int
         if (blockIdx.x == 0 && threadIdx.x == 0) {  // k_chunk_totals
             unsigned long long a = 0, b = 0;
             for (int k = 0; k < levels; ++k) {
-                a += Q.cnt[k];
-                b += Q.cnt[kMaxLevels + k];
+                a += Q.cnt[path_count(k)];
+                b += Q.cnt[shadow_count(k)];
             }
             Q.totals[0] += a;
             Q.totals[1] += b;
@@ -1681,7 +1731,7 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
             const int dep = renderer == TN_RENDERER_RAYTRACER ? lv - 1 : lv - 2;
             if (dep >= 0) chk(hipStreamWaitEvent(s, rb.ev_shadow[dep], 0));
             if (renderer == TN_RENDERER_RAYTRACER) k_rt_shade<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-            else if (guided) k_shade<true><<<tgrid.x * (kRBlock / 64), 64, 0, s>>>(Ap, Qp, lv, buf);
+            else if (guided) k_shade_guided<<<tgrid.x * (kRBlock / kGuidedBlock), kGuidedBlock, 0, s>>>(Ap, Qp, lv, buf);
             else k_shade_plain<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
             chk(hipEventRecord(rb.ev_shade[lv], s));
             chk(hipStreamWaitEvent(side, rb.ev_shade[lv], 0));

@@ -383,8 +383,14 @@ __device__ __forceinline__ void load_guide_frags(const GuideView& G, GuideFrags&
     load_frags32(G.wbf + kGW4, F.w4);
 }
 
-// Runs the MLP for the 64 lanes' samples of one wave (the block must be that
-// one wave: the layers are separated by block barriers).  Leaves the 40
+// Separates a wave's writes of its LDS rows from its reads of other lanes' rows:
+// LDS serves a wave's accesses in order, so only the compiler has to keep them.
+__device__ __forceinline__ void guide_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Runs the MLP for the 64 lanes' samples of one wave.  Leaves the 40
 // outputs of lane l's sample at out[l * 40 ..] (out may alias the first
 // 64 * kGStrideIn uint16 of lds).  `lds` holds 64 * (kGStrideIn +
 // kGStrideHid) uint16 values.  Every forward evaluation of the guide (render,
@@ -396,15 +402,15 @@ __device__ __forceinline__ void guide_forward_wave32(const GuideView& G, const G
     uint16_t* a = lds;                    // [64][kGStrideIn]
     uint16_t* b = lds + 64 * kGStrideIn;  // [64][kGStrideHid]
     guide_features(G, p, n, active, a + l * kGStrideIn);
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32(F.w1, a, kGStrideIn, HiddenEpi{G.theta + kGOffB1, b, kGStrideHid});
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32(F.w2, b, kGStrideHid, HiddenEpi{G.theta + kGOffB2, a, kGStrideIn});
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32(F.w3, a, kGStrideIn, HiddenEpi{G.theta + kGOffB3, b, kGStrideHid});
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32(F.w4, b, kGStrideHid, OutputEpi{G.theta + kGOffB4, out});
-    __syncthreads();
+    guide_wave_sync();
 }
 
 // As guide_forward_wave32 with the weights read from memory layer by layer
@@ -415,15 +421,15 @@ __device__ __forceinline__ void guide_forward_wave(const GuideView& G, float3 p,
     uint16_t* a = lds;                    // [64][kGStrideIn]
     uint16_t* b = lds + 64 * kGStrideIn;  // [64][kGStrideHid]
     guide_features(G, p, n, active, a + l * kGStrideIn);
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32_mem<2, true, 4>(G.wbf + kGW1, a, kGStrideIn, HiddenEpi{G.theta + kGOffB1, b, kGStrideHid});
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32_mem<2, false, 4>(G.wbf + kGW2, b, kGStrideHid, HiddenEpi{G.theta + kGOffB2, a, kGStrideIn});
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32_mem<2, false, 4>(G.wbf + kGW3, a, kGStrideIn, HiddenEpi{G.theta + kGOffB3, b, kGStrideHid});
-    __syncthreads();
+    guide_wave_sync();
     mfma_wx32_mem<2, false, 3>(G.wbf + kGW4, b, kGStrideHid, OutputEpi{G.theta + kGOffB4, out});
-    __syncthreads();
+    guide_wave_sync();
 }
 
 }  // namespace tn
