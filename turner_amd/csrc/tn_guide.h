@@ -26,11 +26,25 @@ constexpr int kGOffW2 = kGOffB1 + 64, kGOffB2 = kGOffW2 + 64 * 64;
 constexpr int kGOffW3 = kGOffB2 + 64, kGOffB3 = kGOffW3 + 64 * 64;
 constexpr int kGOffW4 = kGOffB3 + 64, kGOffB4 = kGOffW4 + 40 * 64;
 constexpr int kGParams = kGOffB4 + 40;  // 15976
-// BF16 copies, padded: W_l as [out_pad][in_pad] (forward A operand) and
-// W_l^T as [in_pad][out_pad] (backward A operand)
+// BF16 copies of W_l (forward A operand, padded [out_pad][in_pad]) and W_l^T
+// (backward A operand, [in_pad][out_pad]) in fragment order (frag_at)
 constexpr int kGW1 = 0, kGW2 = kGW1 + 64 * kGInPad, kGW3 = kGW2 + 64 * 64, kGW4 = kGW3 + 64 * 64;
 constexpr int kGWT2 = kGW4 + kGOutPad * 64, kGWT3 = kGWT2 + 64 * 64, kGWT4 = kGWT3 + 64 * 64;
 constexpr int kGBf16 = kGWT4 + 64 * kGOutPad;
+
+// Position of element (row, col) of a padded [16 out_tiles][cols] matrix in
+// fragment order: for every 16-row tile the K = 32 fragments of its columns,
+// 64 lanes of 8 consecutive columns each, then (cols = 32 kt32 + 16) the K = 16
+// fragments of the last 16 columns, 64 lanes of 4.  A fragment load then reads
+// 1 KB (512 B) in a row; row-major it touched 16 cache lines per instruction, and
+// the products that read their weights from memory waited for nothing else
+// (a 64 x 64 product on 16 samples: 5,000 cycles).
+__host__ __device__ constexpr int frag_at(int row, int col, int kt32, int out_tiles) {
+    const int mt = row / 16, r = row % 16;
+    if (col < 32 * kt32) return ((mt * kt32 + col / 32) * 64 + col % 32 / 8 * 16 + r) * 8 + col % 8;
+    const int c = col - 32 * kt32;
+    return out_tiles * kt32 * 512 + (mt * 64 + c / 4 * 16 + r) * 4 + c % 4;
+}
 
 struct GuideView {
     const uint16_t* wbf;  // BF16 weight copies (layout above)
@@ -170,79 +184,24 @@ __device__ __forceinline__ void guide_features(const GuideView& G, float3 p, flo
     row[79] = 0;
 }
 
-// Y^T = W X^T on the wave's 64 samples (4 tiles of 16) with
-// mfma_f32_16x16x16bf16_1k.  A = W tile (lane: row 16mt + l%16, columns
-// 16kt + 4(l/16) .. +3 of a row-major [16 OUT_TILES][16 IN_TILES] matrix),
-// B = X^T tile read from the [sample][feature] LDS rows (lane: sample
-// 16nt + l%16, features 16kt + 4(l/16) .. +3).  The accumulator of lane l
-// holds outputs 16mt + 4(l/16) .. +3 of sample 16nt + l%16 -- four
-// consecutive features of one row -- handed to epi(first output, sample, v).
-template <int IN_TILES, int OUT_TILES, class Epi>
-__device__ __forceinline__ void mfma_wx(const uint16_t* __restrict__ W, const uint16_t* in, int in_stride,
-                                        Epi epi) {
-    const int l = threadIdx.x & 63;
-    const int row = l & 15, grp = l >> 4;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        g_s4 bfrag[IN_TILES];
-#pragma unroll
-        for (int kt = 0; kt < IN_TILES; ++kt)
-            bfrag[kt] = *reinterpret_cast<const g_s4*>(in + (16 * nt + row) * in_stride + 16 * kt + 4 * grp);
-#pragma unroll
-        for (int mt = 0; mt < OUT_TILES; ++mt) {
-            g_f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < IN_TILES; ++kt) {
-                const g_s4 a =
-                    *reinterpret_cast<const g_s4*>(W + (16 * mt + row) * (16 * IN_TILES) + 16 * kt + 4 * grp);
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bfrag[kt], acc, 0, 0, 0);
-            }
-            epi(16 * mt + 4 * grp, 16 * nt + row, acc);
-        }
-    }
-}
-
-// Same product with the A fragments already in registers (Wf[mt][kt]).
-template <int IN_TILES, int OUT_TILES, class Epi>
-__device__ __forceinline__ void mfma_wx_reg(const g_s4 (&Wf)[OUT_TILES][IN_TILES], const uint16_t* in,
-                                            int in_stride, Epi epi) {
-    const int l = threadIdx.x & 63;
-    const int row = l & 15, grp = l >> 4;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        g_s4 bfrag[IN_TILES];
-#pragma unroll
-        for (int kt = 0; kt < IN_TILES; ++kt)
-            bfrag[kt] = *reinterpret_cast<const g_s4*>(in + (16 * nt + row) * in_stride + 16 * kt + 4 * grp);
-#pragma unroll
-        for (int mt = 0; mt < OUT_TILES; ++mt) {
-            g_f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < IN_TILES; ++kt)
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Wf[mt][kt], bfrag[kt], acc, 0, 0, 0);
-            epi(16 * mt + 4 * grp, 16 * nt + row, acc);
-        }
-    }
-}
-
-// Loads the A fragments of a [16 OUT_TILES][16 IN_TILES] BF16 matrix.
-template <int IN_TILES, int OUT_TILES>
-__device__ __forceinline__ void load_frags(const uint16_t* __restrict__ W, g_s4 (&Wf)[OUT_TILES][IN_TILES]) {
-    const int l = threadIdx.x & 63;
-    const int row = l & 15, grp = l >> 4;
-#pragma unroll
-    for (int mt = 0; mt < OUT_TILES; ++mt)
-#pragma unroll
-        for (int kt = 0; kt < IN_TILES; ++kt)
-            Wf[mt][kt] = *reinterpret_cast<const g_s4*>(W + (16 * mt + row) * (16 * IN_TILES) + 16 * kt + 4 * grp);
-}
-
 typedef __attribute__((ext_vector_type(8))) __bf16 g_bf8;
 
 // K = 32 tiles with gfx950's mfma_f32_16x16x32_bf16: A lane holds row
 // 16mt + l%16, columns 32kt + 8(l/16) .. +7; B lane holds sample 16nt + l%16,
 // features 32kt + 8(l/16) .. +7; the accumulator layout is the 16x16x16 one.
-// KT32 tiles of 32 then, if TAIL, one 16x16x16 tile for columns 32 KT32 .. +15.
+// KT32 tiles of 32 then, if TAIL, one 16x16x16 tile for columns 32 KT32 .. +15
+// (A lane: row 16mt + l%16, columns 32 KT32 + 4(l/16) .. +3; B likewise).  The
+// matrix is in fragment order (frag_at): lane l's part of fragment f is at
+// 8 (64 f + l), of tail fragment f at 4 (64 f + l) behind the others.
+template <int KT32, int OUT_TILES>
+__device__ __forceinline__ g_bf8 frag32(const uint16_t* W, int mt, int kt, uint32_t l) {
+    return *reinterpret_cast<const g_bf8*>(reinterpret_cast<const char*>(W) + (16u * l + 1024u * (uint32_t)(mt * KT32 + kt)));
+}
+template <int KT32, int OUT_TILES>
+__device__ __forceinline__ g_s4 frag16(const uint16_t* W, int mt, uint32_t l) {
+    return *reinterpret_cast<const g_s4*>(reinterpret_cast<const char*>(W) +
+                                          (8u * l + 1024u * OUT_TILES * KT32 + 512u * (uint32_t)mt));
+}
 template <int KT32, bool TAIL, int OUT_TILES>
 struct Frags32 {
     g_bf8 a[OUT_TILES][KT32];
@@ -251,15 +210,12 @@ struct Frags32 {
 
 template <int KT32, bool TAIL, int OUT_TILES>
 __device__ __forceinline__ void load_frags32(const uint16_t* __restrict__ W, Frags32<KT32, TAIL, OUT_TILES>& F) {
-    constexpr int kCols = 32 * KT32 + (TAIL ? 16 : 0);
-    const int l = threadIdx.x & 63;
-    const int row = l & 15, grp = l >> 4;
+    const uint32_t l = threadIdx.x & 63;
 #pragma unroll
     for (int mt = 0; mt < OUT_TILES; ++mt) {
 #pragma unroll
-        for (int kt = 0; kt < KT32; ++kt)
-            F.a[mt][kt] = *reinterpret_cast<const g_bf8*>(W + (16 * mt + row) * kCols + 32 * kt + 8 * grp);
-        if (TAIL) F.t[mt][0] = *reinterpret_cast<const g_s4*>(W + (16 * mt + row) * kCols + 32 * KT32 + 4 * grp);
+        for (int kt = 0; kt < KT32; ++kt) F.a[mt][kt] = frag32<KT32, OUT_TILES>(W, mt, kt, l);
+        if (TAIL) F.t[mt][0] = frag16<KT32, OUT_TILES>(W, mt, l);
     }
 }
 
@@ -297,7 +253,6 @@ __device__ __forceinline__ void mfma_wx32(const Frags32<KT32, TAIL, OUT_TILES>& 
 template <int KT32, bool TAIL, int OUT_TILES, class Epi>
 __device__ __forceinline__ void mfma_wx32_mem(const uint16_t* __restrict__ W, const uint16_t* in, int in_stride,
                                               Epi epi) {
-    constexpr int kCols = 32 * KT32 + (TAIL ? 16 : 0);
     const int l = threadIdx.x & 63;
     const int row = l & 15, grp = l >> 4;
 #pragma unroll
@@ -310,16 +265,13 @@ __device__ __forceinline__ void mfma_wx32_mem(const uint16_t* __restrict__ W, co
         if (TAIL) bt = *reinterpret_cast<const g_s4*>(x + 32 * KT32 + 4 * grp);
 #pragma unroll
         for (int mt = 0; mt < OUT_TILES; ++mt) {
-            const uint16_t* w = W + (16 * mt + row) * kCols;
             g_f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kt = 0; kt < KT32; ++kt)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const g_bf8*>(w + 32 * kt + 8 * grp),
-                                                              b[kt], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag32<KT32, OUT_TILES>(W, mt, kt, l), b[kt], acc, 0, 0, 0);
             if (TAIL) {
                 g_f4 t = {0.f, 0.f, 0.f, 0.f};
-                t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*reinterpret_cast<const g_s4*>(w + 32 * KT32 + 4 * grp),
-                                                              bt, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(frag16<KT32, OUT_TILES>(W, mt, l), bt, t, 0, 0, 0);
                 acc += t;
             }
             epi(16 * mt + 4 * grp, 16 * nt + row, acc);
@@ -354,19 +306,6 @@ struct OutputEpi {
             make_float4(v[0] + b.x, v[1] + b.y, v[2] + b.z, v[3] + b.w);
     }
 };
-
-// Hidden layer: bias, ReLU, BF16 into the next [sample][feature] rows.
-template <int IN_TILES>
-__device__ __forceinline__ void guide_hidden(const uint16_t* W, const float* bias, const uint16_t* in,
-                                             int in_stride, uint16_t* out, int out_stride) {
-    mfma_wx<IN_TILES, 4>(W, in, in_stride, HiddenEpi{bias, out, out_stride});
-}
-
-// Output layer: 40 FP32 outputs per sample into out[sample * 40 + o].
-__device__ __forceinline__ void guide_output(const uint16_t* W, const float* bias, const uint16_t* in,
-                                             int in_stride, float* out) {
-    mfma_wx<4, 3>(W, in, in_stride, OutputEpi{bias, out});
-}
 
 // The A fragments of all four layers (K = 80 as 2 x 32 + 16, then 2 x 32):
 // 128 VGPRs, loaded once per wave and reused for every 64 samples.
@@ -437,11 +376,12 @@ __device__ __forceinline__ void guide_forward_wave(const GuideView& G, float3 p,
 // Guide state behind tn_guide* (device buffers owned).
 struct tn_guide {
     int device = 0;
+    int cus = 256;  // compute units of the device
     float* theta = nullptr;   // FP32 master parameters
     float* adam_m = nullptr;  // Adam moments
     float* adam_v = nullptr;
     uint16_t* wbf = nullptr;  // BF16 operand copies
-    float* partial = nullptr; // per-block gradient slices
+    float* partial = nullptr; // per-block gradient slices and sums
     uint32_t partial_blocks = 0;
     float* dloss = nullptr;   // [0] loss of the last batch, [1] its sum of weights
     float4* ts = nullptr;     // training set: 3 float4 per sample (p, c), (n, cos/pdf), (w, tag)
