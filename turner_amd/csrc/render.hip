@@ -117,7 +117,7 @@ struct SceneParams {
 };
 
 // Chunk bounds kept on the device, so that one captured launch sequence
-// serves every chunk: k_chunk_begin advances them.
+// serves every chunk: chunk_begin_block advances them.
 struct ChunkState {
     unsigned long long next, total, first;
     unsigned long long stride;  // samples from one chunk of this pipeline to its next
@@ -327,40 +327,72 @@ __device__ __forceinline__ void reserve_slots(Slots& S, uint32_t turn, uint32_t*
 
 // Starts the next chunk: [first, first + count) of the call's samples; zeroes
 // the level counters and sets the level-0 count.
-__global__ void k_chunk_begin(uint32_t* cnt, uint32_t* xwork, ChunkState* cs) {
-    const uint32_t i = threadIdx.x;
+// Words of the persistent kernel's grid barrier (grid_sync).
+constexpr uint32_t kBarGen = 0, kBarOut = 32, kBarGroups = 64, kBarGroup = 96;
+constexpr uint32_t kBarWords = kBarGroup + 32 * kXcds;
+
+// Starts the pipeline's next chunk (one block of any size): its bounds, and its
+// counters zeroed but for the overflow word, which lives for the whole render.
+__device__ __forceinline__ void chunk_begin_block(uint32_t* cnt, uint32_t* xwork, ChunkState* cs) {
     const unsigned long long first = cs->next;
     const unsigned long long left = cs->total > first ? cs->total - first : 0ull;
     const uint32_t count = (uint32_t)(left < cs->chunk ? left : cs->chunk);
-    // the overflow word [4 kMaxLevels] lives for the whole render
-    if (i < 4 * kMaxLevels || i == 4 * kMaxLevels + 1) cnt[i] = (i == 0) ? count : 0u;
-    for (uint32_t k = kFixHits + i; k < 6 * kMaxLevels + 2; k += blockDim.x) cnt[k] = 0u;
-    for (uint32_t k = i; k < 2 * kMaxLevels * kXcds; k += blockDim.x) xwork[16 * k] = 0u;
+    for (uint32_t i = threadIdx.x; i < 6 * kMaxLevels + 2; i += blockDim.x)
+        if (i != 4 * kMaxLevels) cnt[i] = (i == 0) ? count : 0u;
+    for (uint32_t k = threadIdx.x; k < 2 * kMaxLevels * kXcds; k += blockDim.x) xwork[16 * k] = 0u;
     __syncthreads();
-    if (i == 0) {
+    if (threadIdx.x == 0) {
         cs->first = first;
         cs->count = count;
         cs->next = first + cs->stride;
     }
 }
 
-__global__ void k_zero_totals(unsigned long long* totals, uint32_t* cnt, uint32_t* incomplete) {
-    if (threadIdx.x < 2) totals[threadIdx.x] = 0;
-    if (threadIdx.x == 2) cnt[4 * kMaxLevels] = 0;  // queue overflow
-    if (threadIdx.x == 3 && incomplete) *incomplete = 0;
-}
+// What a render reports, in pinned host memory: each pipeline writes its own
+// after every chunk, so that the call ends with a stream synchronisation alone.
+struct RenderReport {
+    unsigned long long rays, shadow_rays;
+    uint32_t overflow, incomplete, barrier_out;
+};
 
-// levels < 0: the raycaster, whose rays are its hits (cnt[4 kMaxLevels + 1])
-__global__ void k_chunk_totals(const uint32_t* cnt, unsigned long long* totals, int levels) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        unsigned long long a = levels < 0 ? cnt[4 * kMaxLevels + 1] : 0, b = 0;
-        for (int k = 0; k < levels; ++k) {
-            a += cnt[path_count(k)];
-            b += cnt[shadow_count(k)];
-        }
+// One wave.  Adds a chunk's rays to the pipeline's totals.  levels < 0: the
+// raycaster, whose rays are its hits (cnt[4 kMaxLevels + 1]).
+__device__ __forceinline__ void chunk_totals(const uint32_t* cnt, unsigned long long* totals, int levels) {
+    static_assert(kMaxLevels <= 64, "a lane per level");
+    const int k = (int)(threadIdx.x & 63u);
+    unsigned long long a = k < levels ? cnt[path_count(k)] : 0u, b = k < levels ? cnt[shadow_count(k)] : 0u;
+    if (k == 0 && levels < 0) a = cnt[4 * kMaxLevels + 1];
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_xor(a, off, 64);
+        b += __shfl_xor(b, off, 64);
+    }
+    if (k == 0) {
         totals[0] += a;
         totals[1] += b;
     }
+}
+
+// One thread.  `incomplete` counts both pipelines' abandoned traversals.
+__device__ __forceinline__ void write_report(const Queues& Q, const uint32_t* incomplete, bool barriers,
+                                             RenderReport* out) {
+    out->rays = Q.totals[0];
+    out->shadow_rays = Q.totals[1];
+    out->overflow = Q.cnt[4 * kMaxLevels];
+    out->incomplete = *incomplete;
+    out->barrier_out = barriers ? Q.bar[kBarOut] : 0u;
+}
+
+// End of a chunk: its counts are added up and reported, then the next begins.
+__global__ __launch_bounds__(512) void k_chunk_end(Queues Q, ChunkState* cs, const uint32_t* incomplete, int levels,
+                                                   RenderReport* out) {
+    if (threadIdx.x < 64) chunk_totals(Q.cnt, Q.totals, levels);
+    if (threadIdx.x == 0) write_report(Q, incomplete, false, out);
+    __syncthreads();
+    chunk_begin_block(Q.cnt, Q.xwork, cs);
+}
+
+__global__ void k_persist_end(Queues Q, const uint32_t* incomplete, RenderReport* out) {
+    if (threadIdx.x == 0) write_report(Q, incomplete, true, out);
 }
 
 // Primary samples: within a scene, j = (y * width + x) * spp + i
@@ -1209,8 +1241,6 @@ __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) vo
 // wait is bounded (2^22 polls of about 64 cycles): then [32] is set, and
 // every block stops at its next barrier (grid_sync returns false).
 constexpr uint32_t kBarrierPolls = 1u << 22;
-constexpr uint32_t kBarGen = 0, kBarOut = 32, kBarGroups = 64, kBarGroup = 96;
-constexpr uint32_t kBarWords = kBarGroup + 32 * kXcds;
 
 __device__ __forceinline__ bool grid_sync(uint32_t* bar, uint32_t& gen) {
     __shared__ uint32_t ok;
@@ -1254,23 +1284,6 @@ __device__ __forceinline__ bool grid_sync(uint32_t* bar, uint32_t& gen) {
     return ok != 0u;
 }
 
-// k_chunk_begin for one block of any size (block 0 of the persistent kernel).
-__device__ __forceinline__ void chunk_begin_block(uint32_t* cnt, uint32_t* xwork, ChunkState* cs) {
-    const unsigned long long first = cs->next;
-    const unsigned long long left = cs->total > first ? cs->total - first : 0ull;
-    const uint32_t count = (uint32_t)(left < cs->chunk ? left : cs->chunk);
-    for (uint32_t i = threadIdx.x; i < 4 * kMaxLevels + 2; i += blockDim.x)
-        if (i != 4 * kMaxLevels) cnt[i] = (i == 0) ? count : 0u;  // the overflow word lives for the whole render
-    for (uint32_t k = kFixHits + threadIdx.x; k < 6 * kMaxLevels + 2; k += blockDim.x) cnt[k] = 0u;
-    for (uint32_t k = threadIdx.x; k < 2 * kMaxLevels * kXcds; k += blockDim.x) xwork[16 * k] = 0u;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        cs->first = first;
-        cs->count = count;
-        cs->next = first + cs->stride;
-    }
-}
-
 // Plain path tracing (no guide, no training records, no refined tree) of
 // every chunk of a call in one cooperative launch: per chunk, raygen, then
 // per level the same trace, shade and shadow stages as the wavefront
@@ -1302,21 +1315,9 @@ __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(4))) vo
             if (!grid_sync(Q.bar, gen)) return;
             buf ^= 1;
         }
-        if (blockIdx.x == 0 && threadIdx.x == 0) {  // k_chunk_totals
-            unsigned long long a = 0, b = 0;
-            for (int k = 0; k < levels; ++k) {
-                a += Q.cnt[path_count(k)];
-                b += Q.cnt[shadow_count(k)];
-            }
-            Q.totals[0] += a;
-            Q.totals[1] += b;
-        }
+        if (blockIdx.x == 0 && threadIdx.x < 64) chunk_totals(Q.cnt, Q.totals, levels);
         __syncthreads();  // the counts are read before block 0 clears them for the next chunk
     }
-}
-
-__global__ void k_zero_bar(uint32_t* bar) {
-    for (uint32_t i = threadIdx.x; i < kBarWords; i += blockDim.x) bar[i] = 0u;
 }
 
 // Clears the training records of a chunk: valid flags and found radiance.
@@ -1396,7 +1397,7 @@ std::vector<float> reference_jitter(uint32_t width, uint32_t spp) {
         s ^= s << 25;
         s ^= s >> 27;
         const uint64_t out = s * 2685821657736338717ull;
-        v = std::ldexp((float)(out & 0xFFFFFFull), -24);
+        v = (float)(out & 0xFFFFFFull) * 0x1p-24f;
     }
     return j;
 }
@@ -1511,6 +1512,10 @@ struct RenderContext {
     hipEvent_t ev_fork = nullptr, ev_join[kPipes] = {};
     float* jitter = nullptr;  // reference pixel jitter (TN_RENDER_REF_JITTER)
     size_t jitter_cap = 0;
+    // pinned: the pipelines' reports, then scene table and jitter on their way to
+    // the device (free again when the call that wrote them returns)
+    char* host = nullptr;
+    size_t host_cap = 0;
     // graph replay (TN_RENDER_GRAPH): the capture stream and the executable
     // graph of the last captured chunk sequence, updated in place while the
     // topology stays the same
@@ -1519,20 +1524,74 @@ struct RenderContext {
     uint64_t graph_instantiations = 0, graph_updates = 0;
 };
 
+// Pinned jitter is at most this; a longer table takes a copy of its own.
+constexpr size_t kPinnedJitter = 1u << 20;
+
+int reserve_host(RenderContext& C, size_t bytes) {
+    if (C.host && C.host_cap >= bytes) return TN_OK;
+    if (C.host) (void)hipHostFree(C.host);
+    C.host = nullptr;
+    C.host_cap = 0;
+    bytes = std::max<size_t>(bytes, 1u << 16);
+    TN_HIP(hipHostMalloc((void**)&C.host, bytes, hipHostMallocDefault));
+    C.host_cap = bytes;
+    return TN_OK;
+}
+
 RenderContext& render_context(int device) {
     static RenderContext ctx[kMaxDevices];
     return ctx[device];
 }
 
-// Pipeline p of n renders chunks p, p + n, p + 2n, ... of the call's samples.
-__global__ void k_chunk_setup(ChunkState* cs, unsigned long long total, uint32_t chunk, uint32_t p, uint32_t n) {
-    if (threadIdx.x == 0) {
-        cs->next = (unsigned long long)p * chunk;
-        cs->total = total;
-        cs->first = 0;
-        cs->stride = (unsigned long long)n * chunk;
-        cs->chunk = chunk;
-        cs->count = 0;
+__global__ void k_scale(const float4* __restrict__ a, float4* __restrict__ out, uint32_t n, float f) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float4 v = a[i];
+    out[i] = make_float4(v.x * f, v.y * f, v.z * f, v.w * f);
+}
+
+// Start of a render in one launch.  Block 0: counters and totals of every
+// pipeline (pipeline p of n renders chunks p, p + n, p + 2n, ...) and, unless the
+// persistent kernel does that itself, their first chunks; all blocks: scene table
+// and jitter from pinned host memory.  With separate launches and copies here,
+// and a blocking copy per counter at the end, a 320 x 320 Cornell render took
+// 966 us (now 875), 512 x 512 x 1 at depth 6 2075 (2030), a batch of six small
+// scenes 900 (850).
+struct RenderStart {
+    Queues q[kPipes];
+    ChunkState* cs[kPipes];
+    uint32_t pipes, chunk;
+    unsigned long long total;
+    bool persistent;
+    uint32_t* incomplete;
+    const uint32_t* src[2];
+    uint32_t* dst[2];
+    uint32_t words[2];
+};
+__global__ __launch_bounds__(512) void k_render_start(RenderStart R) {
+    for (int k = 0; k < 2; ++k)
+        for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < R.words[k]; i += gridDim.x * blockDim.x)
+            R.dst[k][i] = R.src[k][i];
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x == 0) *R.incomplete = 0;
+    for (uint32_t p = 0; p < R.pipes; ++p) {
+        const Queues& Q = R.q[p];
+        if (threadIdx.x == 0) {
+            Q.totals[0] = Q.totals[1] = 0;
+            Q.cnt[4 * kMaxLevels] = 0;  // queue overflow
+            ChunkState c{};
+            c.next = (unsigned long long)p * R.chunk;
+            c.total = R.total;
+            c.stride = (unsigned long long)R.pipes * R.chunk;
+            c.chunk = R.chunk;
+            *R.cs[p] = c;
+        }
+        if (R.persistent) {
+            for (uint32_t i = threadIdx.x; i < kBarWords; i += blockDim.x) Q.bar[i] = 0u;
+            continue;
+        }
+        __syncthreads();
+        chunk_begin_block(Q.cnt, Q.xwork, R.cs[p]);
     }
 }
 
@@ -1732,9 +1791,16 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
     }
     for (int p = 0; p < npipes && training; ++p)
         if ((rc = alloc_records(C.recs[p], (size_t)chunk * ((uint32_t)P->max_depth + 1)))) return rc;
+    const size_t table_bytes = table.size() * sizeof(SceneParams);
+    const size_t jitter_bytes = jitter_host ? jitter_len * sizeof(float) : 0;
+    const bool pin_jitter = jitter_bytes <= kPinnedJitter;
+    static_assert(sizeof(RenderReport) * kPipes <= 256 && sizeof(SceneParams) % 4 == 0, "layout of the pinned memory");
+    if ((rc = reserve_host(C, 256 + table_bytes + (pin_jitter ? jitter_bytes : 0)))) return rc;
+    RenderReport* report = (RenderReport*)C.host;
+    std::memcpy(C.host + 256, table.data(), table_bytes);
+    if (pin_jitter && jitter_bytes) std::memcpy(C.host + 256 + table_bytes, jitter_host, jitter_bytes);
+    for (int p = 0; p < npipes; ++p) report[p] = RenderReport{};
     enqueued = true;
-    TN_RHIP(hipMemcpyAsync(rbs[0].sp, table.data(), table.size() * sizeof(SceneParams), hipMemcpyHostToDevice,
-                           stream));
 
     RenderArgs A0{};
     A0.sv = G.sv;
@@ -1787,12 +1853,14 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         A0.ts_cap = guide->ts_cap;
     }
     if (jitter_host) {
-        TN_RHIP(hipMemcpyAsync(C.jitter, jitter_host, jitter_len * sizeof(float), hipMemcpyHostToDevice, stream));
+        if (!pin_jitter)
+            TN_RHIP(hipMemcpyAsync(C.jitter, jitter_host, jitter_bytes, hipMemcpyHostToDevice, stream));
         A0.jitter = C.jitter;
     }
     RecordBuffers* recs = C.recs;
     RenderArgs A[kPipes];
     Queues Q[kPipes];
+    RenderStart R{};
     for (int p = 0; p < npipes; ++p) {
         A[p] = A0;
         A[p].cs = rbs[p].cs;
@@ -1805,9 +1873,22 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
             A[p].rec_g = recs[p].base + 3 * ns;
             A[p].rec_x = recs[p].base + 4 * ns;
         }
-        k_zero_totals<<<1, 64, 0, stream>>>(Q[p].totals, Q[p].cnt, p == 0 ? G.status + 2 : nullptr);
-        k_chunk_setup<<<1, 64, 0, stream>>>(rbs[p].cs, total, chunk, (uint32_t)p, (uint32_t)npipes);
+        R.q[p] = Q[p];
+        R.cs[p] = rbs[p].cs;
     }
+    R.pipes = (uint32_t)npipes;
+    R.chunk = chunk;
+    R.total = total;
+    R.persistent = persistent;
+    R.incomplete = G.status + 2;
+    R.src[0] = (const uint32_t*)(C.host + 256);
+    R.dst[0] = (uint32_t*)rbs[0].sp;
+    R.words[0] = (uint32_t)(table_bytes / 4);
+    R.src[1] = (const uint32_t*)(C.host + 256 + table_bytes);
+    R.dst[1] = (uint32_t*)C.jitter;
+    R.words[1] = pin_jitter ? (uint32_t)(jitter_bytes / 4) : 0u;
+    const uint32_t start_blocks = std::min<uint32_t>(64u, 1u + (R.words[0] + R.words[1]) / 512u);
+    k_render_start<<<start_blocks, 512, 0, stream>>>(R);
     const bool exh = P->flags & TN_RENDER_EXHAUSTIVE;
     const int levels = q.max_depth + 1;
     const uint32_t bpc = std::max(1u, shape.blocks_per_cu);
@@ -1829,7 +1910,6 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         const RenderArgs& Ap = A[p];
         const Queues& Qp = Q[p];
         const hipStream_t side = rb.side;
-        k_chunk_begin<<<1, 4 * kMaxLevels + 64, 0, s>>>(Qp.cnt, Qp.xwork, rb.cs);
         if (training) k_rec_clear<<<(uint32_t)(((size_t)chunk * Ap.rstride + 255) / 256), 256, 0, s>>>(Ap);
         if (rays) k_raygen_rays<<<rgrid, kRBlock, 0, s>>>(Ap, Qp, ray_o, ray_d);
         else k_raygen<<<rgrid, kRBlock, 0, s>>>(Ap, Qp);
@@ -1879,11 +1959,12 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         if (shadows) chk(hipStreamWaitEvent(s, rb.ev_shadow[levels - 1], 0));
         // the raytracer also counts the mirror rays of its last level
         // (trace() is entered and returns {} beyond max_depth)
-        k_chunk_totals<<<1, 64, 0, s>>>(Qp.cnt, Qp.totals,
-                                          renderer == TN_RENDERER_RAYCASTER   ? -1
-                                          : renderer == TN_RENDERER_RAYTRACER ? levels + 1
-                                                                              : levels);
         if (training) k_collect<<<rgrid, kRBlock, 0, s>>>(Ap, P->max_depth);
+        k_chunk_end<<<1, 512, 0, s>>>(Qp, rb.cs, Ap.status + 2,
+                                      renderer == TN_RENDERER_RAYCASTER   ? -1
+                                      : renderer == TN_RENDERER_RAYTRACER ? levels + 1
+                                                                          : levels,
+                                      report + p);
         return e;
     };
     // One round: pipeline 0 on s0, pipeline 1 forked onto its own stream and
@@ -1904,7 +1985,6 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
     const uint64_t nchunks = (total + chunk - 1) / chunk;
     const uint64_t rounds = (nchunks + npipes - 1) / npipes;
     auto t0 = std::chrono::steady_clock::now();
-    uint32_t barrier_out = 0;
     if (persistent) {
         // every block resident at once: the occupancy the kernel allows, at
         // most the shape's blocks per CU
@@ -1913,14 +1993,13 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         TN_RHIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, kRBlock, 0));
         if (per_cu < 1) return fail(set_error(TN_ERR_LIMIT, "the persistent kernel does not fit a CU"));
         const dim3 pgrid((uint32_t)G.cus * std::min<uint32_t>((uint32_t)per_cu, bpc));
-        k_zero_bar<<<1, 256, 0, stream>>>(Q[0].bar);
         TN_RHIP(hipGetLastError());
         RenderArgs pa = A[0];
         Queues pq = Q[0];
         int plevels = levels;
         void* args[] = {&pa, &pq, &plevels};
         TN_RHIP(hipLaunchCooperativeKernel(kfn, pgrid, dim3(kRBlock), args, 0, stream));
-        TN_RHIP(hipMemcpyAsync(&barrier_out, Q[0].bar + kBarOut, 4, hipMemcpyDeviceToHost, stream));
+        k_persist_end<<<1, 64, 0, stream>>>(Q[0], G.status + 2, report);
     } else if (shape.graph && rounds > 1) {
         // The chunk sequence is captured on every call (host-side recording;
         // its kernel arguments change from call to call) and applied to the
@@ -1967,26 +2046,22 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         else if ((rc = guide_train_from_set(guide, train_samples, stream))) return fail(rc);
     }
     if (deferred) TN_RHIP(hipStreamWaitEvent(stream, guide->ev_join, 0));
-    unsigned long long tot[kPipes][2] = {};
-    uint32_t overflow[kPipes] = {}, incomplete = 0;
-    for (int p = 0; p < npipes; ++p) {
-        TN_RHIP(hipMemcpyAsync(tot[p], Q[p].totals, 16, hipMemcpyDeviceToHost, stream));
-        TN_RHIP(hipMemcpyAsync(&overflow[p], Q[p].cnt + 4 * kMaxLevels, 4, hipMemcpyDeviceToHost, stream));
-    }
-    TN_RHIP(hipMemcpyAsync(&incomplete, G.status + 2, 4, hipMemcpyDeviceToHost, stream));
     TN_RHIP(hipStreamSynchronize(stream));
 #undef TN_RHIP
     const double ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     for (int p = 0; p < npipes; ++p)
-        if (overflow[p]) return set_error(TN_ERR_QUEUE, "a ray queue overflowed");
-    if (barrier_out) return set_error(TN_ERR_INCOMPLETE, "a grid barrier wait of the persistent kernel ran out");
+        if (report[p].overflow) return set_error(TN_ERR_QUEUE, "a ray queue overflowed");
+    if (report[0].barrier_out) return set_error(TN_ERR_INCOMPLETE, "a grid barrier wait of the persistent kernel ran out");
+    // counted by both pipelines in one word: the later report has them all
+    uint32_t incomplete = 0;
+    for (int p = 0; p < npipes; ++p) incomplete = std::max(incomplete, report[p].incomplete);
     if (incomplete) return set_error(TN_ERR_INCOMPLETE, "%u render traversals hit the visit cap", incomplete);
     if (st) {
         st->rays = st->shadow_rays = 0;
         for (int p = 0; p < npipes; ++p) {
-            st->rays += tot[p][0];
-            st->shadow_rays += tot[p][1];
+            st->rays += report[p].rays;
+            st->shadow_rays += report[p].shadow_rays;
         }
         st->primary_rays = rays ? 0 : total;
         st->ms = ms;
@@ -2259,11 +2334,10 @@ int tn_render(tn_scene* sc, const tn_camera* cam, const tn_light* lights, uint32
     if (!rc) rc = render_into(sc, cam, lights, nl, P, acc, st, nullptr);
     const float inv = 1.0f / (float)P->pixel_samples;
     if (!rc && linear) {  // mean over pixel samples (main.cpp:216)
-        std::vector<float> tmp(np * 4);
-        if (!rc && (e = hipMemcpy(tmp.data(), acc, np * 16, hipMemcpyDeviceToHost)) != hipSuccess)
+        k_scale<<<(uint32_t)((np + 255) / 256), 256, 0, nullptr>>>((const float4*)acc, (float4*)out, (uint32_t)np, inv);
+        if ((e = hipGetLastError()) != hipSuccess) rc = hip_error(e, "k_scale");
+        if (!rc && (e = hipMemcpy(linear, out, np * 16, hipMemcpyDeviceToHost)) != hipSuccess)
             rc = hip_error(e, "hipMemcpy");
-        if (!rc)
-            for (size_t k = 0; k < np * 4; ++k) linear[k] = tmp[k] * inv;
     }
     if (!rc && display) {
         rc = tn_tonemap(acc, out, (uint32_t)np, inv, P->exposure, P->inverse_gamma, P->gamma_enabled,

@@ -67,8 +67,16 @@ struct tn_scene {
     size_t stage_cap = 0;
     std::mutex stage_mu;
 
-    // Device memory of at least `bytes` in d_stage (caller holds stage_mu).
+    // Pinned host memory through which small host-pointer calls exchange rays and
+    // hits with the kernels, likewise (at most kPinnedRays rays, 2.6 MB).
+    static constexpr uint32_t kPinnedRays = 1u << 16;
+    char* h_stage = nullptr;
+    size_t h_cap = 0;
+
+    // Device memory of at least `bytes` in d_stage, pinned memory in h_stage
+    // (caller holds stage_mu).
     int reserve_stage(size_t bytes);
+    int reserve_pinned(size_t bytes);
 
     // the refined tree (TN_SCENE_REFINED scenes only)
     tn::SceneView fview() const {
