@@ -1402,6 +1402,8 @@ std::vector<float> reference_jitter(uint32_t width, uint32_t spp) {
     return j;
 }
 
+constexpr uint32_t kLeastQueueAlloc = 1u << 22;  // entries: small renders of growing sizes share one allocation
+
 struct RenderBuffers {
     Queues q{};
     size_t bytes = 0;
@@ -1466,26 +1468,65 @@ size_t carve(Queues& q, ChunkState** cs, char* base, uint32_t cap) {
     return off;
 }
 
-int alloc_queues(RenderBuffers& rb, uint32_t cap, uint32_t nscenes) {
-    if (!rb.sp || rb.sp_cap < nscenes) {
-        if (rb.sp) (void)hipFree(rb.sp);
-        rb.sp = nullptr;
-        rb.sp_cap = 0;
-        const uint32_t want = std::max(nscenes, 64u);
-        TN_HIP(hipMalloc(&rb.sp, (size_t)want * sizeof(SceneParams)));
-        rb.sp_cap = want;
-    }
+int reserve_scenes(RenderBuffers& rb, uint32_t nscenes) {
+    if (rb.sp && rb.sp_cap >= nscenes) return TN_OK;
+    if (rb.sp) (void)hipFree(rb.sp);
+    rb.sp = nullptr;
+    rb.sp_cap = 0;
+    const uint32_t want = std::max(nscenes, 64u);
+    TN_HIP(hipMalloc(&rb.sp, (size_t)want * sizeof(SceneParams)));
+    rb.sp_cap = want;
+    return TN_OK;
+}
+
+size_t queue_bytes(uint32_t cap) {
     Queues probe{};
     ChunkState* pcs = nullptr;
-    const size_t need = carve(probe, &pcs, nullptr, cap);
-    if (rb.base && rb.bytes >= need && rb.q.cap >= cap) return TN_OK;
-    if (rb.base) (void)hipFree(rb.base);
-    rb.base = nullptr;
-    rb.bytes = 0;
-    TN_HIP(hipMalloc(&rb.base, need));
-    rb.bytes = need;
-    const size_t used = carve(rb.q, &rb.cs, rb.base, cap);
-    return used <= need ? TN_OK : set_error(TN_ERR_INVALID, "queue layout exceeds its allocation");
+    return carve(probe, &pcs, nullptr, cap);
+}
+
+// Queues of `cap` entries for the first npipes pipelines.  share > 0: refused with
+// TN_ERR_OOM, before anything is touched, if what has to be allocated exceeds
+// 1/share of the memory that is free or held by the queues it replaces.
+int reserve_queues(RenderBuffers* rbs, int npipes, uint32_t cap, size_t share) {
+    const uint32_t least = std::max(cap, kLeastQueueAlloc);
+    size_t grow = 0, held = 0;
+    for (int p = 0; p < npipes; ++p)
+        if (!rbs[p].base || rbs[p].q.cap < cap) {
+            grow += queue_bytes(least);
+            held += rbs[p].bytes;
+        }
+    if (!grow) return TN_OK;
+    if (share) {
+        size_t free_bytes = 0, all = 0;
+        TN_HIP(hipMemGetInfo(&free_bytes, &all));
+        if (grow > (free_bytes + held) / share)
+            return set_error(TN_ERR_OOM, "queues of %zu bytes, %zu are free", grow, free_bytes);
+    }
+    for (int p = 0; p < npipes; ++p) {
+        RenderBuffers& rb = rbs[p];
+        if (rb.base && rb.q.cap >= cap) continue;
+        if (rb.base) (void)hipFree(rb.base);
+        rb.base = nullptr;
+        rb.bytes = 0;
+        uint32_t take = least;
+        size_t need = queue_bytes(take);
+        hipError_t e = hipMalloc(&rb.base, need);
+        if (e != hipSuccess && take > cap) {  // no room for more than this call needs
+            (void)hipGetLastError();
+            take = cap;
+            need = queue_bytes(take);
+            e = hipMalloc(&rb.base, need);
+        }
+        if (e != hipSuccess) {
+            rb.base = nullptr;
+            (void)hipGetLastError();  // reported here
+            return hip_error(e, "hipMalloc(ray queues)");
+        }
+        rb.bytes = need;
+        carve(rb.q, &rb.cs, rb.base, take);
+    }
+    return TN_OK;
 }
 
 struct RecordBuffers {
@@ -1677,16 +1718,67 @@ int check_render_params(const tn_render_params* P) {
     return TN_OK;
 }
 
-// Chunk size for a render: the queue of a chunk's deepest level holds
-// chunk * m^max_depth segments; the default keeps it near 2^23.
-int chunk_size(const tn_render_params* P, uint32_t requested, uint32_t& chunk, uint32_t& cap) {
-    const uint32_t m = (uint32_t)P->mc_samples;
+// Queue entries a pipeline's deepest level may take by default (404 bytes each):
+// larger chunks are fewer launches, and fewer levels that only part of the chip
+// works on.  1920 x 1080 x 2, depth 3, m 4 at 2^23 entries 100.3 ms, 2^24 90.8,
+// 2^25 85.8, 2^26 83.7; m 2 18.1, 16.6, 16.5, 16.5; m 1 (8 samples) at 2^22 paths
+// per chunk 19.0, 2^23 17.7, 2^24 17.6.  2^25 entries are 13.6 GB a pipeline;
+// where that is more than a share of the free memory, half, down to the least.
+constexpr uint32_t kQueueEntries = 1u << 25, kLeastQueueEntries = 1u << 23;
+constexpr size_t kFreeShare = 4;  // new queues take at most a quarter of the free memory
+
+double path_fan(const tn_render_params* P) {
     double fan = 1;
-    for (int k = 0; k < P->max_depth; ++k) fan *= std::max(1u, m);
+    for (int k = 0; k < P->max_depth; ++k) fan *= std::max(1u, (uint32_t)P->mc_samples);
+    return fan;
+}
+
+// Chunk size for a render: the queue of a chunk's deepest level holds
+// chunk * m^max_depth segments, by default `entries` at most.
+int chunk_size(const tn_render_params* P, uint32_t requested, uint32_t entries, uint32_t& chunk, uint32_t& cap) {
+    const double fan = path_fan(P);
     chunk = requested ? requested : P->chunk_paths;
-    if (chunk == 0) chunk = (uint32_t)std::max(1.0, std::min((double)(1u << 23) / fan, 1.0 * (1u << 22)));
+    if (chunk == 0)
+        chunk = (uint32_t)std::max(1.0, std::min((double)entries / fan, (double)std::max(entries / 4, 1u << 22)));
     if (fan * chunk > 2147483647.0) return set_error(TN_ERR_LIMIT, "queue would exceed 2^31 entries");
     cap = (uint32_t)std::max(1.0, fan * chunk);
+    return TN_OK;
+}
+
+// Chunks of a call: samples per chunk, queue entries of a pipeline, pipelines.
+struct ChunkPlan {
+    uint32_t chunk = 0, cap = 0;
+    int npipes = 1;
+};
+
+// Two pipelines, each with its own queues and streams, render alternate chunks
+// concurrently, so that one's launch tails (the slowest rays of a level) overlap
+// the other's work.  A render of one chunk is split evenly between them when the
+// halves are large enough to fill the chip: 2^19 paths each (m 1, depth 6: 2^18
+// samples 2.00 ms whole, 2.16 split; 2^20 3.69, 3.70), or 2^22 entries at the
+// deepest level (m 4, depth 3: 65,536 samples 2.47 ms whole, 2.63 split; 259,200
+// 7.16, 6.62).  Several chunks are made equal, with `even`, so that both
+// pipelines end together.
+int plan_chunks(const tn_render_params* P, uint32_t requested, uint32_t entries, uint64_t total, int npipes,
+                bool even, ChunkPlan& plan) {
+    int rc = chunk_size(P, requested, entries, plan.chunk, plan.cap);
+    if (rc) return rc;
+    even = even && !requested && P->chunk_paths == 0;
+    uint64_t parts = 0;
+    if (npipes > 1 && total <= plan.chunk) {
+        if (total >= (uint64_t)npipes << 19 || (even && path_fan(P) * (double)total >= 8388608.0)) parts = npipes;
+        else npipes = 1;
+    } else if (npipes > 1 && even) {
+        const uint64_t round = (uint64_t)npipes * plan.chunk;
+        parts = (total + round - 1) / round * npipes;
+    }
+    plan.npipes = npipes;
+    if (parts) {
+        const uint64_t part = std::min<uint64_t>(plan.chunk, ((total + parts - 1) / parts + 255) & ~255ull);
+        return chunk_size(P, (uint32_t)part, entries, plan.chunk, plan.cap);
+    }
+    // a call of less than one chunk needs no more queue than its samples do
+    if (total && total < plan.chunk) return chunk_size(P, (uint32_t)total, entries, plan.chunk, plan.cap);
     return TN_OK;
 }
 
@@ -1721,27 +1813,17 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
     tn_render_params q = *P;
     if (renderer == TN_RENDERER_RAYCASTER) q.max_depth = 0;
     if (renderer != TN_RENDERER_PATHTRACER) q.mc_samples = 1;
-    uint32_t chunk = 0, cap = 0;
-    if ((rc = chunk_size(&q, shape.chunk, chunk, cap))) return rc;
-    // Two pipelines, each with its own queues and streams, render alternate
-    // chunks concurrently, so that one's launch tails (the slowest rays of a
-    // level) overlap the other's work.  A render of one chunk is split evenly
-    // between them when each half keeps at least 2^19 paths (smaller halves
-    // measured slower than one pipeline).  A graph-replayed render uses one
-    // pipeline: capturing the second pipeline's stream, which itself forks
-    // its shadow stream, crashed the host process, so that combination
-    // stays off.
     // the persistent kernel serves plain path tracing of camera samples
     const bool persistent = shape.persistent && renderer == TN_RENDERER_PATHTRACER && !guided && !rays && !G.refined;
-    int npipes = (shape.graph || persistent) ? 1 : kPipes;
-    if (npipes > 1 && total <= chunk) {
-        if (total >= (uint64_t)npipes << 19) {
-            const uint64_t part = ((total + npipes - 1) / npipes + 255) & ~255ull;
-            if ((rc = chunk_size(&q, (uint32_t)part, chunk, cap))) return rc;
-        } else {
-            npipes = 1;
-        }
-    }
+    // A graph-replayed render uses one pipeline: capturing the second
+    // pipeline's stream, which itself forks its shadow stream, crashed the host
+    // process, so that combination stays off.
+    const int most_pipes = (shape.graph || persistent) ? 1 : kPipes;
+    // Which records a training render keeps depends on its chunks: they stay as
+    // small as their five records per bounce make advisable.
+    uint32_t entries = training ? kLeastQueueEntries : kQueueEntries;
+    ChunkPlan plan;
+    if ((rc = plan_chunks(&q, shape.chunk, entries, total, most_pipes, !training, plan))) return rc;
     if (st) *st = tn_render_stats{};
     if (total == 0) return TN_OK;
 
@@ -1771,8 +1853,15 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         hipError_t e_ = (call);                                          \
         if (e_ != hipSuccess) return fail(::tn::hip_error(e_, #call));   \
     } while (0)
+    while ((rc = reserve_queues(rbs, plan.npipes, plan.cap, entries > kLeastQueueEntries ? kFreeShare : 0))) {
+        if (rc != TN_ERR_OOM || entries <= kLeastQueueEntries) return rc;
+        entries /= 2;
+        if ((rc = plan_chunks(&q, shape.chunk, entries, total, most_pipes, !training, plan))) return rc;
+    }
+    const uint32_t chunk = plan.chunk;
+    const int npipes = plan.npipes;
     for (int p = 0; p < npipes; ++p) {
-        if ((rc = alloc_queues(rbs[p], cap, (uint32_t)table.size()))) return rc;
+        if ((rc = reserve_scenes(rbs[p], (uint32_t)table.size()))) return rc;
         if ((rc = ensure_side_stream(rbs[p]))) return rc;
     }
     if (!C.ev_fork) {
@@ -2215,7 +2304,7 @@ int autotune(tn_batch* b, const std::vector<SceneParams>& table, uint64_t total,
     int rc = TN_OK;
     for (uint32_t c : chunks) {
         uint32_t ch = 0, cap = 0;
-        if (chunk_size(P, c, ch, cap) != TN_OK || cap > (1u << 24)) continue;  // queue budget
+        if (chunk_size(P, c, kLeastQueueEntries, ch, cap) != TN_OK || cap > (1u << 24)) continue;  // queue budget
         if (c > 2 * probe && c != chunks[0]) continue;
         for (uint32_t g : grids) {
             // graph replay (one pipeline) or direct launches (two
