@@ -67,77 +67,97 @@ __device__ __forceinline__ float3 load3(const float* a, uint32_t i) {
     return make_float3(a[3 * (size_t)i], a[3 * (size_t)i + 1], a[3 * (size_t)i + 2]);
 }
 
-// mode 0: raw outputs (40 per point) into out
-// mode 1: q(w) into pdf
-// mode 2: w ~ q from u3 into w3out, q(w) into pdf
-__global__ __launch_bounds__(64) void k_guide_eval(GuideView G, const float* __restrict__ p3,
-                                                   const float* __restrict__ n3,
-                                                   const float* __restrict__ w3,
-                                                   const float* __restrict__ u3, uint32_t n, int mode,
-                                                   float* __restrict__ out, float* __restrict__ pdf,
-                                                   float* __restrict__ w3out) {
-    __shared__ __align__(16) uint16_t lds[64 * (kGStrideIn + kGStrideHid)];
-    const uint32_t l = threadIdx.x;
-    const uint32_t base = blockIdx.x * 64u;
-    const uint32_t i = base + l;
+// w3 given: q(w) into pdf; else w ~ q from u3 into w3out, q(w) into pdf.  64 points
+// per block: one wave for all (NT = 4 tiles of 16) or a wave per tile (NT = 1).
+template <int NT>
+__global__ __launch_bounds__(256 / NT) void k_guide_eval(GuideView G, const float* __restrict__ p3,
+                                                         const float* __restrict__ n3,
+                                                         const float* __restrict__ w3,
+                                                         const float* __restrict__ u3, uint32_t n,
+                                                         float* __restrict__ pdf, float* __restrict__ w3out) {
+    __shared__ __align__(16) float rows[64 * kGOut];
+    constexpr uint32_t kPoints = 16 * NT;  // of a wave
+    const uint32_t first = threadIdx.x / 64u * kPoints, l = threadIdx.x % kPoints;
+    const uint32_t i = blockIdx.x * 64u + first + l;
+    float* o = rows + first * kGOut;
     const bool act = i < n;
     float3 p = make_float3(0.f, 0.f, 0.f), nn = p;
     if (act) {
         p = load3(p3, i);
         nn = load3(n3, i);
     }
-    float* o = reinterpret_cast<float*>(lds);
-    guide_forward_wave(G, p, nn, act, o, lds);
-    if (mode == 0) {
-        const uint32_t rows = min(64u, n - base);
-        for (uint32_t k = l; k < rows * kGOut; k += 64) out[(size_t)base * kGOut + k] = o[k];
-        return;
-    }
-    if (!act) return;
+    guide_forward_wave<NT>(G, p, nn, act, o);
+    if (!act || threadIdx.x % 64u >= kPoints) return;
     Mixture M;
     mixture_from(o + l * kGOut, M);
     float3 w;
-    if (mode == 2) {
+    if (w3) {
+        w = load3(w3, i);
+    } else {
         w = mixture_sample(M, u3[3 * (size_t)i], u3[3 * (size_t)i + 1], u3[3 * (size_t)i + 2]);
         w3out[3 * (size_t)i] = w.x;
         w3out[3 * (size_t)i + 1] = w.y;
         w3out[3 * (size_t)i + 2] = w.z;
-    } else {
-        w = load3(w3, i);
     }
     pdf[i] = mixture_pdf(M, w);
 }
 
-// MLP outputs for n points with persistent waves: each wave (block) loads
-// every BF16 weight fragment into registers once and then runs groups of 64
-// points, so weights are not re-read per group; the products use gfx950's
-// K = 32 BF16 MFMA (half the instructions of the K = 16 form).
-__global__ __launch_bounds__(64) void k_guide_forward(GuideView G, const float* __restrict__ p3,
-                                                      const float* __restrict__ n3, uint32_t n,
-                                                      float* __restrict__ out) {
-    __shared__ __align__(16) uint16_t lds[64 * (kGStrideIn + kGStrideHid)];
-    GuideFrags F;  // register-resident for every group this wave takes
-    load_guide_frags(G, F);
-    const uint32_t l = threadIdx.x;
-    float* o = reinterpret_cast<float*>(lds);
-    const uint32_t groups = (n + 63) / 64;
-    for (uint32_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {
-        const uint32_t base = grp * 64u, i = base + l;
-        const bool act = i < n;
-        float3 p = make_float3(0.f, 0.f, 0.f), nn = p;
-        if (act) {
+int launch_eval(tn_guide* g, const float* p3, const float* n3, const float* w3, const float* u3, uint32_t n, float* pdf,
+                float* w3out, hipStream_t stream) {
+    const uint32_t blocks = (n + 63) / 64;
+    // A wave per tile while a compute unit has at most two blocks: latency is all
+    // there is (density of 4,099 points 10.6 us per call against 11.8, of 32,768
+    // 11.2 against 12.4); beyond, its idle lanes in the mixture cost more (65,536
+    // points 18.4 us against 12.9, 1,048,576 212 against 98).
+    if (blocks <= (uint32_t)std::max(g->cus, 1) * 2u) k_guide_eval<1><<<blocks, 256, 0, stream>>>(g->view(), p3, n3, w3, u3, n, pdf, w3out);
+    else k_guide_eval<4><<<blocks, 64, 0, stream>>>(g->view(), p3, n3, w3, u3, n, pdf, w3out);
+    TN_HIP(hipGetLastError());
+    return TN_OK;
+}
+
+// four floats at any float's address (callers' arrays need no more)
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// Network outputs for n points with persistent waves: each wave (block) loads
+// every weight fragment into registers once and then takes tiles of 16 points
+// (points and normals of the next tile in flight), whose outputs it stores from
+// the accumulators.  1,048,576 points: 90 us with features, activations and
+// outputs in LDS rows, 68 without (54 without the stores, 41 to move the bytes);
+// what is left is instruction issue: about 250 vector instructions and 20 sines
+// and cosines per tile against 34 matrix ones.  Two to four tiles at a time,
+// three waves per SIMD or biases in LDS gave 68 to 71.
+__global__ __launch_bounds__(64, 2) void k_guide_forward(GuideView G, const float* __restrict__ p3,
+                                                         const float* __restrict__ n3, uint32_t n,
+                                                         float* __restrict__ out) {
+    const GuideRegs net(G);
+    const GuideLane L = guide_lane();
+    const uint32_t s = threadIdx.x & 15u;
+    const uint32_t tiles = (n + 15) / 16;
+    uint32_t tile = blockIdx.x;
+    if (tile >= tiles) return;
+    uint32_t i = min(tile * 16u + s, n - 1u);
+    float3 p = load3(p3, i), nn = load3(n3, i);
+    for (;;) {
+        const uint32_t next = tile + gridDim.x;
+        GuideIn in[1] = {guide_features(G, L, p, nn)};
+        if (next < tiles) {
+            i = min(next * 16u + s, n - 1u);
             p = load3(p3, i);
             nn = load3(n3, i);
         }
-        guide_forward_wave32(G, F, p, nn, act, o, lds);
-        const uint32_t rows = min(64u, n - base);
-        for (uint32_t k = l; k < rows * kGOut; k += 64) out[(size_t)base * kGOut + k] = o[k];
-        __syncthreads();
+        const uint32_t k = tile * 16u + s;
+        guide_network<1>(net, in, [&](int, int o, float4 v) {
+            if (k < n) *reinterpret_cast<f4_any*>(out + (size_t)k * kGOut + o) = (f4_any){v.x, v.y, v.z, v.w};
+        });
+        if (next >= tiles) break;
+        tile = next;
     }
 }
 
 constexpr int kTrainWaves = 8, kTrainBlock = 64 * kTrainWaves;
 constexpr uint32_t kTrainBlocksPerCu = 2;
+constexpr int kGStrideIn = kGInPad + 8;  // LDS row strides (u16), padded against bank conflicts
+constexpr int kGStrideHid = kGHid + 8;
 constexpr int kTStride = 64 + 8;  // row stride (u16) of the transposed [feature][sample] arrays
 
 // d(c * -log q(w)) / d(out) of one of a sample's eight lobes, FP32 in log space:
@@ -199,7 +219,7 @@ struct TrainSrc {
     uint64_t subset_seed;  // fixes which ones
 };
 
-// Two output tiles, mt0 and mt0 + 1, of Y^T = W X^T for 16 samples (mfma_wx32's
+// Two output tiles, mt0 and mt0 + 1, of Y^T = W X^T for 16 samples (guide_layer's
 // sequence): B fragments from their rows (stride in u16), epi(0 or 1, first
 // output, accumulator).
 template <int KT32, bool TAIL, int OUT_TILES, class Epi>
@@ -848,8 +868,7 @@ int tn_guide_forward(tn_guide* g, const float* p3, const float* n3, uint32_t n, 
     if (n && (!p3 || !n3 || !out)) return set_error(TN_ERR_INVALID, "NULL argument");
     if (n > (1u << 30)) return set_error(TN_ERR_LIMIT, "too many points");
     if (!n) return TN_OK;
-    const uint32_t groups = (n + 63) / 64;
-    const uint32_t grid = std::min<uint32_t>(groups, (uint32_t)std::max(g->cus, 1) * 8);  // resident: 8 one-wave blocks per CU
+    const uint32_t grid = std::min<uint32_t>((n + 15) / 16, (uint32_t)std::max(g->cus, 1) * 8);  // resident: 8 one-wave blocks per CU
     k_guide_forward<<<grid, 64, 0, (hipStream_t)stream>>>(g->view(), p3, n3, n, out);
     TN_HIP(hipGetLastError());
     return TN_OK;
@@ -862,10 +881,7 @@ int tn_guide_pdf(tn_guide* g, const float* p3, const float* n3, const float* w3,
     if (n && (!p3 || !n3 || !w3 || !pdf)) return set_error(TN_ERR_INVALID, "NULL argument");
     if (n > (1u << 30)) return set_error(TN_ERR_LIMIT, "too many points");
     if (!n) return TN_OK;
-    k_guide_eval<<<(n + 63) / 64, 64, 0, (hipStream_t)stream>>>(g->view(), p3, n3, w3, nullptr, n, 1, nullptr,
-                                                                pdf, nullptr);
-    TN_HIP(hipGetLastError());
-    return TN_OK;
+    return launch_eval(g, p3, n3, w3, nullptr, n, pdf, nullptr, (hipStream_t)stream);
 }
 
 int tn_guide_sample(tn_guide* g, const float* p3, const float* n3, const float* u3, uint32_t n, float* w3,
@@ -875,10 +891,7 @@ int tn_guide_sample(tn_guide* g, const float* p3, const float* n3, const float* 
     if (n && (!p3 || !n3 || !u3 || !w3 || !pdf)) return set_error(TN_ERR_INVALID, "NULL argument");
     if (n > (1u << 30)) return set_error(TN_ERR_LIMIT, "too many points");
     if (!n) return TN_OK;
-    k_guide_eval<<<(n + 63) / 64, 64, 0, (hipStream_t)stream>>>(g->view(), p3, n3, nullptr, u3, n, 2, nullptr,
-                                                                pdf, w3);
-    TN_HIP(hipGetLastError());
-    return TN_OK;
+    return launch_eval(g, p3, n3, nullptr, u3, n, pdf, w3, (hipStream_t)stream);
 }
 
 int tn_guide_loss_grad(tn_guide* g, const float* p3, const float* n3, const float* w3, const float* c,

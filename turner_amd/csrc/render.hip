@@ -292,41 +292,36 @@ __host__ __device__ __forceinline__ uint32_t shadow_count(int level) { return 2u
 // threads of the block; the two sets of words alternate by `turn`, so that a
 // wave may run ahead into the next iteration's counts.
 struct BlockSlots {
-    uint32_t n_[2][2][kRBlock / 64];  // [turn][paths, shadow rays][wave]
-    unsigned long long base_[2];
-    __device__ uint32_t& n(uint32_t turn, int kind, uint32_t wave) { return n_[turn][kind][wave]; }
-    __device__ unsigned long long& base(uint32_t turn) { return base_[turn]; }
+    uint32_t n[2][2][kRBlock / 64];  // [turn][paths, shadow rays][wave]
+    unsigned long long base[2];
 };
-template <class Slots>
-__device__ __forceinline__ void reserve_slots(Slots& S, uint32_t turn, uint32_t* cnt, int level, uint32_t paths,
+__device__ __forceinline__ void reserve_slots(BlockSlots& S, uint32_t turn, uint32_t* cnt, int level, uint32_t paths,
                                               uint32_t shadows, uint32_t& pbase, uint32_t& sbase) {
     const uint32_t wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     if ((threadIdx.x & 63u) == 0) {
-        S.n(turn, 0, wave) = paths;
-        S.n(turn, 1, wave) = shadows;
+        S.n[turn][0][wave] = paths;
+        S.n[turn][1][wave] = shadows;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t p = 0, q = 0;
         for (uint32_t w = 0; w < waves; ++w) {
-            p += S.n(turn, 0, w);
-            q += S.n(turn, 1, w);
+            p += S.n[turn][0][w];
+            q += S.n[turn][1][w];
         }
-        S.base(turn) = (p | q) ? atomicAdd(reinterpret_cast<unsigned long long*>(cnt + path_count(level + 1)),
+        S.base[turn] = (p | q) ? atomicAdd(reinterpret_cast<unsigned long long*>(cnt + path_count(level + 1)),
                                            (unsigned long long)q << 32 | p)
                                : 0ull;
     }
     __syncthreads();
-    pbase = (uint32_t)S.base(turn);
-    sbase = (uint32_t)(S.base(turn) >> 32);
+    pbase = (uint32_t)S.base[turn];
+    sbase = (uint32_t)(S.base[turn] >> 32);
     for (uint32_t w = 0; w < wave; ++w) {
-        pbase += S.n(turn, 0, w);
-        sbase += S.n(turn, 1, w);
+        pbase += S.n[turn][0][w];
+        sbase += S.n[turn][1][w];
     }
 }
 
-// Starts the next chunk: [first, first + count) of the call's samples; zeroes
-// the level counters and sets the level-0 count.
 // Words of the persistent kernel's grid barrier (grid_sync).
 constexpr uint32_t kBarGen = 0, kBarOut = 32, kBarGroups = 64, kBarGroup = 96;
 constexpr uint32_t kBarWords = kBarGroup + 32 * kXcds;
@@ -917,10 +912,10 @@ __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) vo
 }
 
 // Shade one level: the block's waves take 64 segments each per iteration.
-// glds: the calling wave's rows for the guide's network (GUIDED).
-template <bool GUIDED, class Slots>
+// gout: the calling wave's outputs of the guide's network (GUIDED).
+template <bool GUIDED>
 __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q, int level, int buf,
-                                           uint16_t* glds, Slots& slots) {
+                                           float* gout, BlockSlots& slots) {
     const uint32_t n = min(Q.cnt[path_count(level)], Q.cap);
     const uint32_t lane = threadIdx.x & 63u;
     const bool spawn = level < A.max_depth && A.mc > 0;
@@ -1147,8 +1142,7 @@ __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q,
             }
         } else {
             // guided: the wave's 64 hits through the guide MLP
-            float* gout = reinterpret_cast<float*>(glds);
-            guide_forward_wave(A.gv, p, nn, has_hit, gout, glds);
+            guide_forward_wave<4>(A.gv, p, nn, has_hit, gout);
             Mixture M;
             mixture_from(gout + lane * kGOut, M);
             guide_wave_sync();  // gout is overwritten by the next iteration's forward pass
@@ -1199,25 +1193,15 @@ __device__ __forceinline__ void shade_body(const RenderArgs& A, const Queues& Q,
     }
 }
 
-// Two waves per block, each with its own 20 KB of rows for the guide's network:
-// four blocks (two waves per SIMD, as the registers allow) fill a CU's 160 KB
-// exactly, so the block's slot words live in the padding behind the hidden
-// rows of its first wave, which nothing else touches.
+// Two waves per block, each with 10 KB for the outputs of the guide's network:
+// guided 512^2x8 at depth 6 4.21 ms with its features and activations in LDS rows
+// (20 KB), 4.06 without; three or four waves per SIMD (16 or 32 samples at a time)
+// 4.07 to 4.14.
 constexpr int kGuidedBlock = 128;
-struct RowSlots {
-    uint16_t* rows;  // 16-byte gaps at rows + kGHid, every kGStrideHid
-    __device__ uint32_t& n(uint32_t turn, int kind, uint32_t wave) {
-        return reinterpret_cast<uint32_t*>(rows + turn * kGStrideHid + kGHid)[2 * kind + wave];
-    }
-    __device__ unsigned long long& base(uint32_t turn) {
-        return *reinterpret_cast<unsigned long long*>(rows + (2 + turn) * kGStrideHid + kGHid);
-    }
-};
-static_assert(kGStrideHid - kGHid >= 8 && kGuidedBlock == 128, "two waves' counts fit a row's padding");
 __global__ __launch_bounds__(kGuidedBlock) void k_shade_guided(RenderArgs A, Queues Q, int level, int buf) {
-    __shared__ __align__(16) uint16_t glds[kGuidedBlock / 64][64 * (kGStrideIn + kGStrideHid)];
-    RowSlots slots{glds[0] + 64 * kGStrideIn};
-    shade_body<true>(A, Q, level, buf, glds[threadIdx.x >> 6], slots);
+    __shared__ __align__(16) float gout[kGuidedBlock / 64][64 * kGOut];
+    __shared__ BlockSlots slots;
+    shade_body<true>(A, Q, level, buf, gout[threadIdx.x >> 6], slots);
 }
 
 // The unguided shade capped at 72 VGPRs (7 waves per SIMD, 68 bytes of

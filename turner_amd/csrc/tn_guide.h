@@ -150,40 +150,6 @@ __host__ __device__ __forceinline__ uint16_t to_bf16(float x) {
 }
 __device__ __forceinline__ float from_bf16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-constexpr int kGStrideIn = kGInPad + 8;  // LDS row strides (u16), padded against bank conflicts
-constexpr int kGStrideHid = kGHid + 8;
-
-// Features of one sample (lane) into an LDS row of kGInPad BF16 values.
-__device__ __forceinline__ void guide_features(const GuideView& G, float3 p, float3 n, bool active,
-                                               uint16_t* row) {
-    float u[3] = {(p.x - G.bmin[0]) * G.inv_ext[0], (p.y - G.bmin[1]) * G.inv_ext[1],
-                  (p.z - G.bmin[2]) * G.inv_ext[2]};
-    if (!active) u[0] = u[1] = u[2] = 0.f;
-    row[0] = to_bf16(u[0]);
-    row[1] = to_bf16(u[1]);
-    row[2] = to_bf16(u[2]);
-    // sin / cos of 2^q pi u = of 2 pi (2^(q-1) u): the hardware sine and
-    // cosine take revolutions; the argument's fraction (exact, as is the
-    // power-of-two scaling) keeps them in range.  Absolute error about
-    // 1.3e-7 (sincospif: 5e-8), far below the BF16 step.
-    int k = 3;
-    for (int c = 0; c < 3; ++c) {
-        float f = 0.5f;
-        for (int q = 0; q < kGFreq; ++q) {
-            const float r = __builtin_amdgcn_fractf(f * u[c]);
-            const uint32_t sc = pack_bf16x2(__builtin_amdgcn_sinf(r), __builtin_amdgcn_cosf(r));
-            row[k++] = (uint16_t)sc;
-            row[k++] = (uint16_t)(sc >> 16);
-            f *= 2.0f;
-        }
-    }
-    row[75] = to_bf16(active ? n.x : 0.f);
-    row[76] = to_bf16(active ? n.y : 0.f);
-    row[77] = to_bf16(active ? n.z : 0.f);
-    row[78] = 0;
-    row[79] = 0;
-}
-
 typedef __attribute__((ext_vector_type(8))) __bf16 g_bf8;
 
 // K = 32 tiles with gfx950's mfma_f32_16x16x32_bf16: A lane holds row
@@ -202,124 +168,237 @@ __device__ __forceinline__ g_s4 frag16(const uint16_t* W, int mt, uint32_t l) {
     return *reinterpret_cast<const g_s4*>(reinterpret_cast<const char*>(W) +
                                           (8u * l + 1024u * OUT_TILES * KT32 + 512u * (uint32_t)mt));
 }
-template <int KT32, bool TAIL, int OUT_TILES>
-struct Frags32 {
-    g_bf8 a[OUT_TILES][KT32];
-    g_s4 t[OUT_TILES][TAIL ? 1 : 1];
+__device__ __forceinline__ g_bf8 as_bf8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    const uint4 v = make_uint4(a, b, c, d);
+    g_bf8 r;
+    __builtin_memcpy(&r, &v, 16);
+    return r;
+}
+
+// The network runs on 16 samples per matrix tile without LDS.  A lane (sample s =
+// l % 16, group g = l / 16) computes the features of its sample that its B
+// operands hold, and a layer's outputs (accumulator: outputs 16 mt + 4 g .. +3 of
+// sample s) become the next layer's B operands (features 32 kt + 8 g .. +7) by two
+// lane swaps.  Through LDS rows a wave wrote 78 two-byte features per lane and
+// met four round trips per layer; its 20 KB also kept all but two waves off a SIMD.
+
+// First layer operands of a tile: features 32 kt + 8 g .. +7 and 64 + 4 g .. +3.
+struct GuideIn {
+    g_bf8 b[2];
+    g_s4 t;
 };
 
-template <int KT32, bool TAIL, int OUT_TILES>
-__device__ __forceinline__ void load_frags32(const uint16_t* __restrict__ W, Frags32<KT32, TAIL, OUT_TILES>& F) {
-    const uint32_t l = threadIdx.x & 63;
+// The lane's feature frequencies: sin / cos of 2^q pi u are those of 2 pi
+// (2^(q-1) u).  A run of eight starts with the cosine at q, then sine and cosine
+// at q + 1 (scale x = 2^(q-1)), then sine, cosine, sine, cosine, sine from the
+// next octave (scale z), perhaps of the next axis; the last four features
+// likewise.
+struct GuideLane {
+    int g;
+    float x[2], z[2], t;
+};
+__device__ __forceinline__ GuideLane guide_lane() {
+    const int g = (int)(threadIdx.x & 63u) >> 4;
+    auto scale = [](int q) { return __uint_as_float((uint32_t)(126 + q) << 23); };
+    GuideLane L;
+    L.g = g;
+    L.x[0] = scale(4 * g - 2);                // -, 2, 6, 10
+    L.z[0] = scale(g == 3 ? 0 : 4 * g);       // 0, 4, 8, 0
+    L.x[1] = scale(g == 3 ? 2 : 4 * g + 2);   // 2, 6, 10, 2
+    L.z[1] = scale(g == 0 || g == 3 ? 4 : (g == 1 ? 8 : 0));
+    L.t = scale(6 + 2 * g);                   // 6, 8, 10, -
+    return L;
+}
+
+// The hardware sine and cosine take revolutions; the argument's fraction (exact,
+// as is the power-of-two scaling) keeps them in range.  Absolute error about
+// 1.3e-7 (sincospif: 5e-8), far below the BF16 step.
+__device__ __forceinline__ GuideIn guide_features(const GuideView& G, const GuideLane& L, float3 p, float3 n) {
+    const float ux = (p.x - G.bmin[0]) * G.inv_ext[0], uy = (p.y - G.bmin[1]) * G.inv_ext[1],
+                uz = (p.z - G.bmin[2]) * G.inv_ext[2];
+    auto turns = [](float a) { return __builtin_amdgcn_fractf(a); };
+    auto run = [&](float x, float z, bool first) {
+        const float x0 = turns(x), x1 = turns(2.0f * x), z0 = turns(z), z1 = turns(2.0f * z), z2 = turns(4.0f * z);
+        float f0 = __builtin_amdgcn_cosf(x0), f1 = __builtin_amdgcn_sinf(x1), f2 = __builtin_amdgcn_cosf(x1);
+        if (first) {  // features 0 .. 2
+            f0 = L.g == 0 ? ux : f0;
+            f1 = L.g == 0 ? uy : f1;
+            f2 = L.g == 0 ? uz : f2;
+        }
+        return as_bf8(pack_bf16x2(f0, f1), pack_bf16x2(f2, __builtin_amdgcn_sinf(z0)),
+                      pack_bf16x2(__builtin_amdgcn_cosf(z0), __builtin_amdgcn_sinf(z1)),
+                      pack_bf16x2(__builtin_amdgcn_cosf(z1), __builtin_amdgcn_sinf(z2)));
+    };
+    GuideIn I;
+    I.b[0] = run(L.x[0] * ux, L.z[0] * (L.g == 3 ? uy : ux), true);
+    I.b[1] = run(L.x[1] * (L.g == 3 ? uz : uy), L.z[1] * (L.g < 2 ? uy : uz), false);
+    const float x = L.t * uz, x0 = turns(x), x1 = turns(2.0f * x), x2 = turns(4.0f * x);
+    float f[4] = {__builtin_amdgcn_cosf(x0), __builtin_amdgcn_sinf(x1), __builtin_amdgcn_cosf(x1),
+                  __builtin_amdgcn_sinf(x2)};
+    f[3] = L.g == 2 ? n.x : f[3];  // features 75 .. 77, then the padding
+    f[0] = L.g == 3 ? n.y : f[0];
+    f[1] = L.g == 3 ? n.z : f[1];
+    f[2] = L.g == 3 ? 0.f : f[2];
+    f[3] = L.g == 3 ? 0.f : f[3];
+    const uint2 t = make_uint2(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]));
+    __builtin_memcpy(&I.t, &t, 8);
+    return I;
+}
+
+// Y^T = W X^T for NT tiles of 16 samples: epi(mt, nt, acc).  w(mt, kt) and wt(mt)
+// give the A fragments.
+template <int KT32, bool TAIL, int OUT_TILES, int NT, class W, class WT, class Epi>
+__device__ __forceinline__ void guide_layer(W w, WT wt, const g_bf8 (&b)[NT][2], const g_s4* bt, Epi epi) {
 #pragma unroll
     for (int mt = 0; mt < OUT_TILES; ++mt) {
+        g_bf8 a[KT32];
 #pragma unroll
-        for (int kt = 0; kt < KT32; ++kt) F.a[mt][kt] = frag32<KT32, OUT_TILES>(W, mt, kt, l);
-        if (TAIL) F.t[mt][0] = frag16<KT32, OUT_TILES>(W, mt, l);
-    }
-}
-
-template <int KT32, bool TAIL, int OUT_TILES, class Epi>
-__device__ __forceinline__ void mfma_wx32(const Frags32<KT32, TAIL, OUT_TILES>& F, const uint16_t* in,
-                                          int in_stride, Epi epi) {
-    const int l = threadIdx.x & 63;
-    const int row = l & 15, grp = l >> 4;
+        for (int kt = 0; kt < KT32; ++kt) a[kt] = w(mt, kt);
+        g_s4 at = {0, 0, 0, 0};
+        if (TAIL) at = wt(mt);
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        const uint16_t* x = in + (16 * nt + row) * in_stride;
-        g_bf8 b[KT32];
-#pragma unroll
-        for (int kt = 0; kt < KT32; ++kt) b[kt] = *reinterpret_cast<const g_bf8*>(x + 32 * kt + 8 * grp);
-        g_s4 bt = {0, 0, 0, 0};
-        if (TAIL) bt = *reinterpret_cast<const g_s4*>(x + 32 * KT32 + 4 * grp);
-#pragma unroll
-        for (int mt = 0; mt < OUT_TILES; ++mt) {
+        for (int nt = 0; nt < NT; ++nt) {
             g_f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kt = 0; kt < KT32; ++kt) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(F.a[mt][kt], b[kt], acc, 0, 0, 0);
+            for (int kt = 0; kt < KT32; ++kt) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kt], b[nt][kt], acc, 0, 0, 0);
             if (TAIL) {  // the K = 16 tail accumulates separately: no mixed-shape accumulation chain
                 g_f4 t = {0.f, 0.f, 0.f, 0.f};
-                t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(F.t[mt][0], bt, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(at, bt[nt], t, 0, 0, 0);
                 acc += t;
             }
-            epi(16 * mt + 4 * grp, 16 * nt + row, acc);
+            epi(mt, nt, acc);
         }
     }
 }
 
-// mfma_wx32 with the A fragments read from W (global, L2-resident) inside
-// the loop instead of held in registers: the same MFMA sequence, so the
-// same sums, for kernels that cannot spare 128 VGPRs for the weights.
-template <int KT32, bool TAIL, int OUT_TILES, class Epi>
-__device__ __forceinline__ void mfma_wx32_mem(const uint16_t* __restrict__ W, const uint16_t* in, int in_stride,
-                                              Epi epi) {
-    const int l = threadIdx.x & 63;
-    const int row = l & 15, grp = l >> 4;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        const uint16_t* x = in + (16 * nt + row) * in_stride;
-        g_bf8 b[KT32];
-#pragma unroll
-        for (int kt = 0; kt < KT32; ++kt) b[kt] = *reinterpret_cast<const g_bf8*>(x + 32 * kt + 8 * grp);
-        g_s4 bt = {0, 0, 0, 0};
-        if (TAIL) bt = *reinterpret_cast<const g_s4*>(x + 32 * KT32 + 4 * grp);
-#pragma unroll
-        for (int mt = 0; mt < OUT_TILES; ++mt) {
-            g_f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < KT32; ++kt)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag32<KT32, OUT_TILES>(W, mt, kt, l), b[kt], acc, 0, 0, 0);
-            if (TAIL) {
-                g_f4 t = {0.f, 0.f, 0.f, 0.f};
-                t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(frag16<KT32, OUT_TILES>(W, mt, l), bt, t, 0, 0, 0);
-                acc += t;
-            }
-            epi(16 * mt + 4 * grp, 16 * nt + row, acc);
-        }
-    }
+// Bias, ReLU and BF16 of four outputs.
+__device__ __forceinline__ uint2 guide_relu(float4 b, g_f4 v) {
+    return make_uint2(pack_bf16x2(fmaxf(v[0] + b.x, 0.f), fmaxf(v[1] + b.y, 0.f)),
+                      pack_bf16x2(fmaxf(v[2] + b.z, 0.f), fmaxf(v[3] + b.w, 0.f)));
 }
 
+// B operands of the next layer's K tile from the output tiles h0 (its first 16
+// features) and h1: group g holds features 4 g .. +3 of both, and gets 8 g .. +7
+// of the 32.  Groups 2, 3 of h0 against 0, 1 of h1, then odd groups of the one
+// against even groups of the other.
+__device__ __forceinline__ g_bf8 guide_operand(uint2 h0, uint2 h1) {
+    const auto x = __builtin_amdgcn_permlane32_swap(h0.x, h1.x, false, false);
+    const auto y = __builtin_amdgcn_permlane32_swap(h0.y, h1.y, false, false);
+    const auto u = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+    const auto v = __builtin_amdgcn_permlane16_swap(y[0], y[1], false, false);
+    return as_bf8(u[0], v[0], u[1], v[1]);
+}
 
-// Epilogue of a hidden layer: bias, ReLU, BF16, one 8-byte LDS store of the
-// four consecutive features.
-struct HiddenEpi {
-    const float* bias;
-    uint16_t* out;
-    int stride;
-    __device__ __forceinline__ void operator()(int o, int smp, g_f4 v) const {
-        const float4 b = *reinterpret_cast<const float4*>(bias + o);
-        uint2 w;
-        w.x = pack_bf16x2(fmaxf(v[0] + b.x, 0.f), fmaxf(v[1] + b.y, 0.f));
-        w.y = pack_bf16x2(fmaxf(v[2] + b.z, 0.f), fmaxf(v[3] + b.w, 0.f));
-        *reinterpret_cast<uint2*>(out + smp * stride + o) = w;
+// Weight fragments and biases of layer L (0 .. 3) from memory.
+template <int L>
+struct GuideMem {
+    static constexpr int kW = L == 0 ? kGW1 : L == 1 ? kGW2 : L == 2 ? kGW3 : kGW4;
+    static constexpr int kB = L == 0 ? kGOffB1 : L == 1 ? kGOffB2 : L == 2 ? kGOffB3 : kGOffB4;
+    static constexpr int kTiles = L == 3 ? 3 : 4;
+    static __device__ __forceinline__ g_bf8 w(const GuideView& G, int mt, int kt, uint32_t l) {
+        return frag32<2, kTiles>(G.wbf + kW, mt, kt, l);
+    }
+    // padded outputs 40 .. 47 have no bias
+    static __device__ __forceinline__ float4 bias(const GuideView& G, int o) {
+        return *reinterpret_cast<const float4*>(G.theta + kB + (L == 3 && o >= kGOut ? 0 : o));
     }
 };
 
-// Epilogue of the output layer: 40 FP32 outputs per sample at out[smp * 40].
-struct OutputEpi {
-    const float* bias;
-    float* out;
-    __device__ __forceinline__ void operator()(int o, int smp, g_f4 v) const {
-        if (o >= kGOut) return;  // padded rows 40..47
-        const float4 b = *reinterpret_cast<const float4*>(bias + o);
-        *reinterpret_cast<float4*>(out + smp * kGOut + o) =
-            make_float4(v[0] + b.x, v[1] + b.y, v[2] + b.z, v[3] + b.w);
+// All weight fragments and biases in registers: 128 and 60 VGPRs, loaded once per
+// wave and used for every tile it takes.
+struct GuideRegs {
+    g_bf8 a[4][4][2];
+    g_s4 t[4];
+    float4 b[4][4];
+    template <int L>
+    __device__ __forceinline__ void load(const GuideView& G, uint32_t l) {
+#pragma unroll
+        for (int mt = 0; mt < GuideMem<L>::kTiles; ++mt) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) a[L][mt][kt] = GuideMem<L>::w(G, mt, kt, l);
+            b[L][mt] = GuideMem<L>::bias(G, 16 * mt + 4 * (int)(l >> 4));
+        }
+    }
+    __device__ __forceinline__ explicit GuideRegs(const GuideView& G) {
+        const uint32_t l = threadIdx.x & 63u;
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) t[mt] = frag16<2, 4>(G.wbf + kGW1, mt, l);
+        load<0>(G, l);
+        load<1>(G, l);
+        load<2>(G, l);
+        load<3>(G, l);
+    }
+    template <int L>
+    __device__ __forceinline__ g_bf8 w(int mt, int kt) const {
+        return a[L][mt][kt];
+    }
+    __device__ __forceinline__ g_s4 wt(int mt) const { return t[mt]; }
+    template <int L>
+    __device__ __forceinline__ float4 bias(int mt) const {
+        return b[L][mt];
     }
 };
 
-// The A fragments of all four layers (K = 80 as 2 x 32 + 16, then 2 x 32):
-// 128 VGPRs, loaded once per wave and reused for every 64 samples.
-struct GuideFrags {
-    Frags32<2, true, 4> w1;
-    Frags32<2, false, 4> w2, w3;
-    Frags32<2, false, 3> w4;
+// The same, read layer by layer from memory (L2): for kernels that cannot spare
+// the registers.
+struct GuideLoads {
+    const GuideView& G;
+    uint32_t l;
+    // The lane is opaque to the compiler, which otherwise keeps the addresses of all
+    // fragments in registers across the shade kernel's loop.
+    __device__ __forceinline__ explicit GuideLoads(const GuideView& g) : G(g), l(threadIdx.x & 63u) {
+        asm volatile("" : "+v"(l));
+    }
+    template <int L>
+    __device__ __forceinline__ g_bf8 w(int mt, int kt) const {
+        return GuideMem<L>::w(G, mt, kt, l);
+    }
+    __device__ __forceinline__ g_s4 wt(int mt) const { return frag16<2, 4>(G.wbf + kGW1, mt, l); }
+    template <int L>
+    __device__ __forceinline__ float4 bias(int mt) const {
+        return GuideMem<L>::bias(G, 16 * mt + 4 * (int)(l >> 4));
+    }
 };
 
-__device__ __forceinline__ void load_guide_frags(const GuideView& G, GuideFrags& F) {
-    load_frags32(G.wbf + kGW1, F.w1);
-    load_frags32(G.wbf + kGW2, F.w2);
-    load_frags32(G.wbf + kGW3, F.w3);
-    load_frags32(G.wbf + kGW4, F.w4);
+// The network for NT tiles: out(nt, first output, four outputs) for outputs
+// 0 .. 39 of the lane's sample.  Every forward evaluation of the guide (render,
+// pdf, sampling, tn_guide_forward) runs this arithmetic, so a density the
+// renderer sampled with is the density tn_guide_pdf reports.
+template <int NT, class Net, class Out>
+__device__ __forceinline__ void guide_network(const Net& N, const GuideIn (&in)[NT], Out out) {
+    const int g = (int)(threadIdx.x & 63u) >> 4;
+    g_bf8 b[NT][2];
+    g_s4 bt[NT];
+    uint2 h[NT][4];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        b[nt][0] = in[nt].b[0];
+        b[nt][1] = in[nt].b[1];
+        bt[nt] = in[nt].t;
+    }
+    auto operands = [&] {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            b[nt][0] = guide_operand(h[nt][0], h[nt][1]);
+            b[nt][1] = guide_operand(h[nt][2], h[nt][3]);
+        }
+    };
+    guide_layer<2, true, 4, NT>([&](int mt, int kt) { return N.template w<0>(mt, kt); }, [&](int mt) { return N.wt(mt); }, b,
+                                bt, [&](int mt, int nt, g_f4 v) { h[nt][mt] = guide_relu(N.template bias<0>(mt), v); });
+    operands();
+    guide_layer<2, false, 4, NT>([&](int mt, int kt) { return N.template w<1>(mt, kt); }, [](int) { return g_s4{}; }, b, bt,
+                                 [&](int mt, int nt, g_f4 v) { h[nt][mt] = guide_relu(N.template bias<1>(mt), v); });
+    operands();
+    guide_layer<2, false, 4, NT>([&](int mt, int kt) { return N.template w<2>(mt, kt); }, [](int) { return g_s4{}; }, b, bt,
+                                 [&](int mt, int nt, g_f4 v) { h[nt][mt] = guide_relu(N.template bias<2>(mt), v); });
+    operands();
+    guide_layer<2, false, 3, NT>([&](int mt, int kt) { return N.template w<3>(mt, kt); }, [](int) { return g_s4{}; }, b, bt,
+                                 [&](int mt, int nt, g_f4 v) {
+                                     const int o = 16 * mt + 4 * g;
+                                     if (o >= kGOut) return;  // padded rows 40 .. 47
+                                     const float4 c = N.template bias<3>(mt);
+                                     out(nt, o, make_float4(v[0] + c.x, v[1] + c.y, v[2] + c.z, v[3] + c.w));
+                                 });
 }
 
 // Separates a wave's writes of its LDS rows from its reads of other lanes' rows:
@@ -329,45 +408,28 @@ __device__ __forceinline__ void guide_wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// Runs the MLP for the 64 lanes' samples of one wave.  Leaves the 40
-// outputs of lane l's sample at out[l * 40 ..] (out may alias the first
-// 64 * kGStrideIn uint16 of lds).  `lds` holds 64 * (kGStrideIn +
-// kGStrideHid) uint16 values.  Every forward evaluation of the guide (render,
-// pdf, sampling, tn_guide_forward) runs this arithmetic, so a density the
-// renderer sampled with is the density tn_guide_pdf reports.
-__device__ __forceinline__ void guide_forward_wave32(const GuideView& G, const GuideFrags& F, float3 p,
-                                                     float3 n, bool active, float* out, uint16_t* lds) {
-    const int l = threadIdx.x & 63;
-    uint16_t* a = lds;                    // [64][kGStrideIn]
-    uint16_t* b = lds + 64 * kGStrideIn;  // [64][kGStrideHid]
-    guide_features(G, p, n, active, a + l * kGStrideIn);
-    guide_wave_sync();
-    mfma_wx32(F.w1, a, kGStrideIn, HiddenEpi{G.theta + kGOffB1, b, kGStrideHid});
-    guide_wave_sync();
-    mfma_wx32(F.w2, b, kGStrideHid, HiddenEpi{G.theta + kGOffB2, a, kGStrideIn});
-    guide_wave_sync();
-    mfma_wx32(F.w3, a, kGStrideIn, HiddenEpi{G.theta + kGOffB3, b, kGStrideHid});
-    guide_wave_sync();
-    mfma_wx32(F.w4, b, kGStrideHid, OutputEpi{G.theta + kGOffB4, out});
-    guide_wave_sync();
-}
-
-// As guide_forward_wave32 with the weights read from memory layer by layer
-// (same sums, far fewer registers: for the shade and evaluation kernels).
-__device__ __forceinline__ void guide_forward_wave(const GuideView& G, float3 p, float3 n, bool active,
-                                                   float* out, uint16_t* lds) {
-    const int l = threadIdx.x & 63;
-    uint16_t* a = lds;                    // [64][kGStrideIn]
-    uint16_t* b = lds + 64 * kGStrideIn;  // [64][kGStrideHid]
-    guide_features(G, p, n, active, a + l * kGStrideIn);
-    guide_wave_sync();
-    mfma_wx32_mem<2, true, 4>(G.wbf + kGW1, a, kGStrideIn, HiddenEpi{G.theta + kGOffB1, b, kGStrideHid});
-    guide_wave_sync();
-    mfma_wx32_mem<2, false, 4>(G.wbf + kGW2, b, kGStrideHid, HiddenEpi{G.theta + kGOffB2, a, kGStrideIn});
-    guide_wave_sync();
-    mfma_wx32_mem<2, false, 4>(G.wbf + kGW3, a, kGStrideIn, HiddenEpi{G.theta + kGOffB3, b, kGStrideHid});
-    guide_wave_sync();
-    mfma_wx32_mem<2, false, 3>(G.wbf + kGW4, b, kGStrideHid, OutputEpi{G.theta + kGOffB4, out});
+// The network for a wave's 16 NT samples, lane l holding sample l % (16 NT): the 40
+// outputs of sample k at out[k * 40 ..] (LDS).
+template <int NT>
+__device__ __forceinline__ void guide_forward_wave(const GuideView& G, float3 p, float3 n, bool active, float* out) {
+    const int s = (int)(threadIdx.x & 15u);
+    if (!active) p = n = make_float3(0.f, 0.f, 0.f);
+    const GuideLoads net(G);
+    const GuideLane L = guide_lane();
+    GuideIn in[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int src = 16 * nt + s;
+        float3 tp = p, tn = n;
+        if (NT > 1) {
+            tp = make_float3(__shfl(p.x, src, 64), __shfl(p.y, src, 64), __shfl(p.z, src, 64));
+            tn = make_float3(__shfl(n.x, src, 64), __shfl(n.y, src, 64), __shfl(n.z, src, 64));
+        }
+        in[nt] = guide_features(G, L, tp, tn);
+    }
+    guide_network<NT>(net, in, [&](int nt, int o, float4 v) {
+        *reinterpret_cast<float4*>(out + (16 * nt + s) * kGOut + o) = v;
+    });
     guide_wave_sync();
 }
 
