@@ -1738,19 +1738,28 @@ struct ChunkPlan {
 // Two pipelines, each with its own queues and streams, render alternate chunks
 // concurrently, so that one's launch tails (the slowest rays of a level) overlap
 // the other's work.  A render of one chunk is split evenly between them when the
-// halves are large enough to fill the chip: 2^19 paths each (m 1, depth 6: 2^18
-// samples 2.00 ms whole, 2.16 split; 2^20 3.69, 3.70), or 2^22 entries at the
-// deepest level (m 4, depth 3: 65,536 samples 2.47 ms whole, 2.63 split; 259,200
-// 7.16, 6.62).  Several chunks are made equal, with `even`, so that both
-// pipelines end together.
+// halves still fill the chip.  With the path tracer that is from 2^19 samples or
+// 2^23 segments at the deepest level (Cornell box 819,200 samples 0.87 ms whole,
+// 0.81 split; m 1, depth 6: 524,176 samples 2.43 and 2.34, 262,144 2.02 and 1.98,
+// but a batch of six small scenes of about as many 0.85 and 0.88; m 4, depth 3:
+// 65,536 samples 2.48 and 2.56, 259,200 7.2 and 6.6), with the raytracer, whose
+// levels thin out, from 2^20 (262,144 samples 0.68 and 0.73 ms, 524,176 0.78 and
+// 0.82, 2,079,604 1.33 with two).  Several chunks are made equal so that both
+// pipelines end together.  Neither holds for chunks that the caller sizes, nor
+// (`plain` false) for training renders: which records those keep depends on their
+// chunks.
+constexpr uint64_t kSplitPaths = 1u << 19, kSplitOther = 1u << 20;
+constexpr double kSplitEntries = 8388608.0;
 int plan_chunks(const tn_render_params* P, uint32_t requested, uint32_t entries, uint64_t total, int npipes,
-                bool even, ChunkPlan& plan) {
+                bool plain, ChunkPlan& plan) {
     int rc = chunk_size(P, requested, entries, plan.chunk, plan.cap);
     if (rc) return rc;
-    even = even && !requested && P->chunk_paths == 0;
+    const bool even = plain && !requested && P->chunk_paths == 0;
+    const bool paths = even && P->renderer == TN_RENDERER_PATHTRACER;
     uint64_t parts = 0;
     if (npipes > 1 && total <= plan.chunk) {
-        if (total >= (uint64_t)npipes << 19 || (even && path_fan(P) * (double)total >= 8388608.0)) parts = npipes;
+        if (total >= (paths ? kSplitPaths : kSplitOther) || (paths && path_fan(P) * (double)total >= kSplitEntries))
+            parts = npipes;
         else npipes = 1;
     } else if (npipes > 1 && even) {
         const uint64_t round = (uint64_t)npipes * plan.chunk;
@@ -1803,8 +1812,8 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
     // pipeline's stream, which itself forks its shadow stream, crashed the host
     // process, so that combination stays off.
     const int most_pipes = (shape.graph || persistent) ? 1 : kPipes;
-    // Which records a training render keeps depends on its chunks: they stay as
-    // small as their five records per bounce make advisable.
+    // a training render's chunks stay as small as their five records per bounce
+    // make advisable
     uint32_t entries = training ? kLeastQueueEntries : kQueueEntries;
     ChunkPlan plan;
     if ((rc = plan_chunks(&q, shape.chunk, entries, total, most_pipes, !training, plan))) return rc;
@@ -1974,7 +1983,15 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
     // for the shadow test of level k - 2; the raytracer's shade also reads
     // the child weights the shadow test of level k - 1 darkens, so it waits
     // for that one.
-    auto chunk_sequence = [&](int p, hipStream_t s) -> hipError_t {
+    const bool shadows = renderer != TN_RENDERER_RAYCASTER;
+    auto chunk_start = [&](int p, hipStream_t s) {
+        const RenderArgs& Ap = A[p];
+        const Queues& Qp = Q[p];
+        if (training) k_rec_clear<<<(uint32_t)(((size_t)chunk * Ap.rstride + 255) / 256), 256, 0, s>>>(Ap);
+        if (rays) k_raygen_rays<<<rgrid, kRBlock, 0, s>>>(Ap, Qp, ray_o, ray_d);
+        else k_raygen<<<rgrid, kRBlock, 0, s>>>(Ap, Qp);
+    };
+    auto chunk_level = [&](int p, hipStream_t s, int lv) -> hipError_t {
         hipError_t e = hipSuccess;
         auto chk = [&](hipError_t x) {
             if (e == hipSuccess) e = x;
@@ -1983,53 +2000,52 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         const RenderArgs& Ap = A[p];
         const Queues& Qp = Q[p];
         const hipStream_t side = rb.side;
-        if (training) k_rec_clear<<<(uint32_t)(((size_t)chunk * Ap.rstride + 255) / 256), 256, 0, s>>>(Ap);
-        if (rays) k_raygen_rays<<<rgrid, kRBlock, 0, s>>>(Ap, Qp, ray_o, ray_d);
-        else k_raygen<<<rgrid, kRBlock, 0, s>>>(Ap, Qp);
-        const bool shadows = renderer != TN_RENDERER_RAYCASTER;
-        int buf = 0;
+        const int buf = lv & 1;
         const bool refd = G.refined;
         const dim3 fgrid(32u);  // fix lists are short (a scan after an overflow is rare)
-        for (int lv = 0; lv < levels; ++lv) {
-            if (refd) {
-                if (exh) k_trace<true, true><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-                else k_trace<false, true><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-                if (exh) k_fix_hits<true><<<fgrid, kRBlock, 0, s>>>(Ap, Qp, lv, buf);
-                else k_fix_hits<false><<<fgrid, kRBlock, 0, s>>>(Ap, Qp, lv, buf);
-            } else {
-                if (exh) k_trace<true, false><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-                else k_trace<false, false><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-            }
-            if (renderer == TN_RENDERER_RAYCASTER) {
-                k_cast<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-                buf ^= 1;
-                continue;
-            }
-            const int dep = renderer == TN_RENDERER_RAYTRACER ? lv - 1 : lv - 2;
-            if (dep >= 0) chk(hipStreamWaitEvent(s, rb.ev_shadow[dep], 0));
-            if (renderer == TN_RENDERER_RAYTRACER) k_rt_shade<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-            else if (guided) k_shade_guided<<<tgrid.x * (kRBlock / kGuidedBlock), kGuidedBlock, 0, s>>>(Ap, Qp, lv, buf);
-            else k_shade_plain<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
-            chk(hipEventRecord(rb.ev_shade[lv], s));
-            chk(hipStreamWaitEvent(side, rb.ev_shade[lv], 0));
-            if (renderer == TN_RENDERER_RAYTRACER) {
-                if (exh) k_rt_shadow<true><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv, buf);
-                else k_rt_shadow<false><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv, buf);
-            } else if (refd) {
-                if (exh) k_shadow<true, true><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
-                else k_shadow<false, true><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
-                if (exh) k_fix_shadows<true><<<fgrid, kRBlock, 0, side>>>(Ap, Qp, lv);
-                else k_fix_shadows<false><<<fgrid, kRBlock, 0, side>>>(Ap, Qp, lv);
-            } else {
-                if (exh) k_shadow<true, false><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
-                else k_shadow<false, false><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
-            }
-            chk(hipEventRecord(rb.ev_shadow[lv], side));
-            buf ^= 1;
+        if (refd) {
+            if (exh) k_trace<true, true><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
+            else k_trace<false, true><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
+            if (exh) k_fix_hits<true><<<fgrid, kRBlock, 0, s>>>(Ap, Qp, lv, buf);
+            else k_fix_hits<false><<<fgrid, kRBlock, 0, s>>>(Ap, Qp, lv, buf);
+        } else {
+            if (exh) k_trace<true, false><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
+            else k_trace<false, false><<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
         }
+        if (renderer == TN_RENDERER_RAYCASTER) {
+            k_cast<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
+            return e;
+        }
+        const int dep = renderer == TN_RENDERER_RAYTRACER ? lv - 1 : lv - 2;
+        if (dep >= 0) chk(hipStreamWaitEvent(s, rb.ev_shadow[dep], 0));
+        if (renderer == TN_RENDERER_RAYTRACER) k_rt_shade<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
+        else if (guided) k_shade_guided<<<tgrid.x * (kRBlock / kGuidedBlock), kGuidedBlock, 0, s>>>(Ap, Qp, lv, buf);
+        else k_shade_plain<<<tgrid, tblock, 0, s>>>(Ap, Qp, lv, buf);
+        chk(hipEventRecord(rb.ev_shade[lv], s));
+        chk(hipStreamWaitEvent(side, rb.ev_shade[lv], 0));
+        if (renderer == TN_RENDERER_RAYTRACER) {
+            if (exh) k_rt_shadow<true><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv, buf);
+            else k_rt_shadow<false><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv, buf);
+        } else if (refd) {
+            if (exh) k_shadow<true, true><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
+            else k_shadow<false, true><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
+            if (exh) k_fix_shadows<true><<<fgrid, kRBlock, 0, side>>>(Ap, Qp, lv);
+            else k_fix_shadows<false><<<fgrid, kRBlock, 0, side>>>(Ap, Qp, lv);
+        } else {
+            if (exh) k_shadow<true, false><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
+            else k_shadow<false, false><<<tgrid, tblock, 0, side>>>(Ap, Qp, lv);
+        }
+        chk(hipEventRecord(rb.ev_shadow[lv], side));
+        return e;
+    };
+    auto chunk_finish = [&](int p, hipStream_t s) -> hipError_t {
+        RenderBuffers& rb = rbs[p];
+        const RenderArgs& Ap = A[p];
+        const Queues& Qp = Q[p];
         // every shadow test is done before the counts are read (the side
         // stream runs in order, so its last event covers all of them)
-        if (shadows) chk(hipStreamWaitEvent(s, rb.ev_shadow[levels - 1], 0));
+        hipError_t e = hipSuccess;
+        if (shadows) e = hipStreamWaitEvent(s, rb.ev_shadow[levels - 1], 0);
         // the raytracer also counts the mirror rays of its last level
         // (trace() is entered and returns {} beyond max_depth)
         if (training) k_collect<<<rgrid, kRBlock, 0, s>>>(Ap, P->max_depth);
@@ -2040,18 +2056,33 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
                                       report + p);
         return e;
     };
-    // One round: pipeline 0 on s0, pipeline 1 forked onto its own stream and
-    // joined back (the fork and join are events, so a captured round is a
-    // graph with the same concurrency).
-    auto round = [&](hipStream_t s0) -> hipError_t {
-        if (npipes == 1) return chunk_sequence(0, s0);
-        hipError_t e = hipEventRecord(C.ev_fork, s0);
-        for (int p = 1; p < npipes && e == hipSuccess; ++p) e = hipStreamWaitEvent(pipe_stream[p], C.ev_fork, 0);
-        if (e == hipSuccess) e = chunk_sequence(0, s0);
-        for (int p = 1; p < npipes && e == hipSuccess; ++p) e = chunk_sequence(p, pipe_stream[p]);
+    // One chunk of each of n pipelines on its stream, enqueued level by level, so
+    // that the second starts when the first does and not when the host has
+    // launched all of the first's kernels.
+    auto round = [&](const hipStream_t* s, int n) -> hipError_t {
+        hipError_t e = hipSuccess;
+        for (int p = 0; p < n; ++p) chunk_start(p, s[p]);
+        for (int lv = 0; lv < levels; ++lv)
+            for (int p = 0; p < n && e == hipSuccess; ++p) e = chunk_level(p, s[p], lv);
+        for (int p = 0; p < n && e == hipSuccess; ++p) e = chunk_finish(p, s[p]);
+        return e;
+    };
+    // All rounds: pipeline 0 on `stream`, pipeline 1 forked onto its own stream and
+    // joined back after its last chunk.  The pipelines share nothing but the
+    // accumulator's atomics, and joined after every round the one waited for the
+    // other's last shadow test.
+    auto all_rounds = [&](uint64_t rounds) -> hipError_t {
+        hipError_t e = hipSuccess;
+        hipStream_t s[kPipes] = {stream};
+        if (npipes > 1) e = hipEventRecord(C.ev_fork, stream);
         for (int p = 1; p < npipes && e == hipSuccess; ++p) {
-            e = hipEventRecord(C.ev_join[p], pipe_stream[p]);
-            if (e == hipSuccess) e = hipStreamWaitEvent(s0, C.ev_join[p], 0);
+            s[p] = pipe_stream[p];
+            e = hipStreamWaitEvent(s[p], C.ev_fork, 0);
+        }
+        for (uint64_t c = 0; c < rounds && e == hipSuccess; ++c) e = round(s, npipes);
+        for (int p = 1; p < npipes && e == hipSuccess; ++p) {
+            e = hipEventRecord(C.ev_join[p], s[p]);
+            if (e == hipSuccess) e = hipStreamWaitEvent(stream, C.ev_join[p], 0);
         }
         return e;
     };
@@ -2083,7 +2114,7 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         hipGraph_t graph = nullptr;
         hipError_t e = hipStreamBeginCapture(C.cap_stream, hipStreamCaptureModeThreadLocal);
         if (e == hipSuccess) {
-            const hipError_t es = round(C.cap_stream);  // the other streams join and leave the capture
+            const hipError_t es = round(&C.cap_stream, 1);  // its shadow stream joins and leaves the capture
             e = hipStreamEndCapture(C.cap_stream, &graph);
             if (e == hipSuccess) e = es;
         }
@@ -2108,10 +2139,8 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         if (graph) (void)hipGraphDestroy(graph);
         if (e != hipSuccess) return fail(hip_error(e, "captured chunk sequence"));
     } else {
-        for (uint64_t c = 0; c < rounds; ++c) {
-            const hipError_t e = round(stream);
-            if (e != hipSuccess) return fail(hip_error(e, "chunk sequence"));
-        }
+        const hipError_t e = all_rounds(rounds);
+        if (e != hipSuccess) return fail(hip_error(e, "chunk sequence"));
     }
     TN_RHIP(hipGetLastError());
     if (training) {
