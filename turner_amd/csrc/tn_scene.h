@@ -49,9 +49,9 @@ struct tn_scene {
     unsigned long long* d_counters = nullptr;  // 8 counters
     uint32_t* d_status = nullptr;              // [0] incomplete traversals, [1] queue overflow
     // Work counters of large tn_intersect / tn_occluded launches: a ring of
-    // slots, each 8 per-XCD chunk counters and a finished-wave counter (16
-    // words apart), zero between launches (the last wave of a launch clears
-    // its slot).  A slot is reused only after the event recorded behind its
+    // slots, each a line of a chunk and a finished-wave counter per XCD, then
+    // one of finished XCDs (16 words apart), zero between launches (the last
+    // wave of a launch clears its slot).  A slot is reused only after the event recorded behind its
     // previous launch, so launches on different streams never share one.
     static constexpr int kWorkSlots = 16;
     static constexpr int kWorkWords = 16 * 9;
