@@ -159,9 +159,10 @@ __host__ __device__ inline uint32_t small_share(uint32_t n, uint32_t waves, uint
 // occ != NULL visibility against tmax into occ.
 // fixed_work: zeroed work counters (16 x 9 words) the launch may use instead
 // of a work slot of the scene, also under stream capture (null: a slot).
+// report: where the last kernel leaves the scene's count of abandoned traversals.
 int launch_rays(tn_scene* sc, const float* o3, const float* d3, const float* tmax, uint32_t n,
                 uint32_t* id, float* r, float* s, float* t, uint8_t* occ, uint32_t flags,
-                hipStream_t stream, uint32_t* fixed_work = nullptr);
+                hipStream_t stream, uint32_t* fixed_work = nullptr, uint32_t* report = nullptr);
 // Launches closest-hit traversal over n rays (device arrays) into id/r/s/t.
 int launch_intersect(tn_scene* sc, const float* o3, const float* d3, uint32_t n, uint32_t* id,
                      float* r, float* s, float* t, uint32_t flags, hipStream_t stream);
