@@ -198,7 +198,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     uint32_t nrays = 0;
     TraversalCounters cnt;
     coop_loop<kStack, EXH, MT, ANY, COUNT, TIE>(
-        sc, stk + threadIdx.x, kBlock, wl + threadIdx.x / 64,
+        sc, stk + threadIdx.x, kBlock, wl + threadIdx.x / 64, !REF && !work && chunk <= 64u,
         RayChunks{work, n, chunk, gridDim.x * (kBlock / 64), wave * chunk, blockIdx.x % kXcds, false},
         // rays and results stream through once: non-temporal loads and
         // stores keep them from evicting tree nodes and records from L2

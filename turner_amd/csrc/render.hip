@@ -444,6 +444,9 @@ __global__ __launch_bounds__(kRBlock) void k_raygen_rays(RenderArgs A, Queues Q,
     Q.rng[0][i] = rng_seed(A.seed_pass, j);
 }
 
+// coop_loop's `whole`.
+__device__ __forceinline__ bool a_ray_per_lane(uint32_t n) { return n <= gridDim.x * blockDim.x; }
+
 // Per-wave chunks of a device-counted queue.  The chunk shrinks with the
 // queue (a sixteenth of a wave's share, at least 64; queues of less than 64
 // paths for every fourth wave by small_share: a shadow launch and the other
@@ -562,7 +565,7 @@ __device__ __forceinline__ void trace_body(const RenderArgs& A, const Queues& Q,
     uint4* hit = Q.hit;
     TraversalCounters cnt;
     coop_loop<kRStack, EXH, false, false, false, REF>(
-        A.sv, stk + threadIdx.x, kRBlock, wl + threadIdx.x / 64,
+        A.sv, stk + threadIdx.x, kRBlock, wl + threadIdx.x / 64, !REF && a_ray_per_lane(n),
         DynamicChunks{n, Q.xwork + 16 * kXcds * level},
         [&](uint32_t k, float3& o, float3& d, float&, uint32_t& scene) {
             const float4 a = qo[k], b = qd[k];
@@ -628,7 +631,7 @@ __device__ __forceinline__ void shadow_body(const RenderArgs& A, const Queues& Q
     TraversalCounters cnt;
     SettledChunks chunks(n, Q.xwork + 16 * kXcds * (kMaxLevels + level));
     coop_loop<kRStack, EXH, false, true, false>(
-        A.sv, stk + threadIdx.x, kRBlock, wl + threadIdx.x / 64,
+        A.sv, stk + threadIdx.x, kRBlock, wl + threadIdx.x / 64, !REF && a_ray_per_lane(n),
         [&](uint32_t& b, uint32_t& e) { return chunks(b, e); },
         [&](uint32_t k, float3& o, float3& d, float& tmax, uint32_t& scene) {
             const float4 a = Q.so[sb][k], b = Q.sd[sb][k];
@@ -874,7 +877,7 @@ __global__ __launch_bounds__(kRBlock) __attribute__((amdgpu_waves_per_eu(7))) vo
     auto darken = [&](float4 c) { return make_float4(c.x - c.x * si, c.y - c.y * si, c.z - c.z * si, c.w - c.w * si); };
     SettledChunks chunks(n, Q.xwork + 16 * kXcds * (kMaxLevels + level));
     coop_loop<kRStack, EXH, false, true, false>(
-        sv, stk + threadIdx.x, kRBlock, wl + threadIdx.x / 64,
+        sv, stk + threadIdx.x, kRBlock, wl + threadIdx.x / 64, a_ray_per_lane(n),
         [&](uint32_t& b, uint32_t& e) { return chunks(b, e); },
         [&](uint32_t k, float3& o, float3& d, float& tmax, uint32_t& scene) {
             const float4 a = Q.so[sb][k], b = Q.sd[sb][k];

@@ -172,10 +172,18 @@ __device__ __forceinline__ int leaf_test_ref(const float4* __restrict__ pa, cons
 // 3 for a hit at exactly r == bound, which does not replace the best.
 template <bool ANY, bool TIE>
 __device__ __forceinline__ int pair_test_ref(const float4* __restrict__ pa, const float4* __restrict__ pc,
-                                             float3 o, float3 d, float bound, float& r, float& snum,
+                                             float3 o, float3 d, float bound, bool whole, float& r, float& snum,
                                              float& tnum) {
     const float4 a = pa[0];  // v0, uv
     const float4 b = pa[1];  // n, vv
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    const v4* second = reinterpret_cast<const v4*>(pc);
+    v4 c = {}, e = {};
+    if (whole) {
+        c = second[0];
+        e = second[1];
+        asm volatile("" : "+v"(c), "+v"(e));  // read here, not where they are used
+    }
     const float den = b.x * d.x + b.y * d.y + b.z * d.z;
     const float nom = b.x * (a.x - o.x) + b.y * (a.y - o.y) + b.z * (a.z - o.z);
     const float rr = nom / den;
@@ -183,8 +191,10 @@ __device__ __forceinline__ int pair_test_ref(const float4* __restrict__ pa, cons
     asm volatile("" : "+v"(uv), "+v"(vv));  // read with the rest of their 16 bytes, not again below
     // a ray along the plane (den 0) has no hit: the quotient is infinite or NaN
     if (!(rr >= 0.f) || ((ANY || TIE) ? !(rr <= bound) : !(rr < bound)) || (ANY && den == 0.f)) return 0;
-    const float4 c = pc[0];  // u, uu
-    const float4 e = pc[1];  // v, denom
+    if (!whole) {
+        c = second[0];  // u, uu
+        e = second[1];  // v, denom
+    }
     const float px = o.x + rr * d.x, py = o.y + rr * d.y, pz = o.z + rr * d.z;
     const float wx = px - a.x, wy = py - a.y, wz = pz - a.z;
     const float wv = wx * e.x + wy * e.y + wz * e.z;
@@ -650,6 +660,14 @@ __device__ __forceinline__ NodeStep node_step(const CoopRay& R, uint32_t split, 
 //     a verdict (pair_test_ref): a two-level step takes 60 VALU instructions
 //     (was 90), a round of 64 pairs 95 (was 146); 298 -> 257 us, 2.63 -> 2.26
 //     ms, 4099 rays 195 -> 153 us, the 2^24 batch 5.50 -> 5.36 ms.
+//   whole: read a record's second half with the first instead of when the first
+//                      half asks for it: a latency less per leaf, and twice the
+//                      bytes per test.  For launches of at most a ray per lane,
+//                      which wait for their slowest ray (512^2 one-sample pass
+//                      2.035 -> 1.975 ms, guided 512^2 x 8 3.98 -> 3.94); always, the
+//                      2^24 batch went 4.95 -> 6.17 ms, 1080p m 4 85.1 -> 93.3.  Not
+//                      with TIE or on a refined tree, whose kernels spill with it
+//                      (1080p 87.1 ms, 4099 rays 92 -> 93.5 us);
 //   chunk(begin, end): called by all lanes of the wave; returns false when no
 //                      work is left (may update begin/end);
 //   load(k, o, d, tmax, scene), store(k, hit): per-ray I/O (scene: the ray's
@@ -661,7 +679,7 @@ __device__ __forceinline__ NodeStep node_step(const CoopRay& R, uint32_t split, 
 constexpr uint32_t kRefill = 16, kDescendTail = 3;
 
 template <int S, bool EXH, bool MT, bool ANY, bool COUNT, bool TIE = false, class Chunk, class Load, class Store>
-__device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int stride, CoopLds* wl, Chunk chunk,
+__device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int stride, CoopLds* wl, bool whole, Chunk chunk,
                                           Load load, Store store, TraversalCounters& cnt) {
     static_assert(!TIE || (!ANY && !MT), "tie detection is for the reference leaf test's closest hit");
     static_assert(S > 0 && (S & (S - 1)) == 0, "the circular stack index wraps with & (S - 1)");
@@ -810,7 +828,7 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                     const size_t r = rb + item;  // reference slot of the pair
                     float rr, ss, tt;  // barycentrics, or their numerators (pair_test_ref)
                     const int code = MT ? leaf_test_mt<ANY>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt)
-                                        : pair_test_ref<ANY, TIE>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, rr, ss, tt);
+                                        : pair_test_ref<ANY, TIE>(sc.lra + 2 * r, sc.lrb + 2 * r, ro, rd, bnd, whole, rr, ss, tt);
                     if (COUNT) {
                         cnt.refs++;
                         cnt.tests++;
@@ -861,7 +879,7 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                             float ss, tt;
                             const float4 *pa = sc.lra + 2 * (size_t)r, *pc = sc.lrb + 2 * (size_t)r;
                             if (MT) leaf_test_mt<ANY>(pa, pc, R.o, R.d, bound_own, R.best_r, ss, tt);
-                            else pair_test_ref<ANY, TIE>(pa, pc, R.o, R.d, bound_own, R.best_r, ss, tt);
+                            else pair_test_ref<ANY, TIE>(pa, pc, R.o, R.d, bound_own, false, R.best_r, ss, tt);
                         }
                     }
                 }
