@@ -88,10 +88,11 @@ typedef struct {
  * precomputes the triangles (lib/triangle.h:22-39), builds the SAH kd-tree on
  * the host with the reference's algorithm and constants (lib/kdtree.cpp:124-467)
  * and uploads nodes, triangle references, triangle records and shading data
- * to the device.  Device memory: 8 B per node, 4 B per triangle reference,
- * 64 B per triangle record plus a 64-byte copy of the record per triangle
- * reference (reference order, read by the traversal), 68 B of shading data per
- * triangle.  verts9: 9 floats per triangle (v0 v1 v2).  normals9: vertex
+ * to the device.  Device memory: 8 B per node plus about 16 B for the same
+ * tree two levels at a time (read by the traversal), 4 B per triangle
+ * reference, 64 B per triangle record plus a 64-byte copy of the record per
+ * triangle reference (reference order, read by the traversal), 68 B of shading
+ * data per triangle.  verts9: 9 floats per triangle (v0 v1 v2).  normals9: vertex
  * normals (NULL: face normals).  albedo4: RGBA diffuse per triangle (NULL:
  * 0.8 grey, alpha 1).  emission4: RGBA emission per triangle (NULL: none).
  */
@@ -202,7 +203,8 @@ int tn_intersect(tn_scene* scene, const float* o3, const float* d3, uint32_t n,
  * (TN_ERR_LIMIT). */
 int tn_intersect_noalloc(tn_scene* scene, const float* o3, const float* d3, uint32_t n,
                          uint32_t* id, float* r, float* s, float* t, uint32_t flags, void* stream);
-/* Host-pointer variant (copies in and out, synchronous). */
+/* Host-pointer variant (synchronous; up to 65,536 rays pass through pinned
+ * memory that the kernels access, larger calls are copied in and out). */
 int tn_intersect_host(tn_scene* scene, const float* o3, const float* d3, uint32_t n,
                       uint32_t* id, float* r, float* s, float* t, uint32_t flags);
 /* Shadow / visibility query with the reference's predicate
