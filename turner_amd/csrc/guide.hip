@@ -42,18 +42,22 @@ __device__ __forceinline__ void store_operands(uint16_t* __restrict__ wbf, int p
     const uint16_t h = to_bf16(value);
     if (p < kGOffB1) {
         wbf[kGW1 + frag_at(p / kGIn, p % kGIn, 2, 4)] = h;
+        wbf[kGTW1 + frag16_at(p / kGIn, p % kGIn, 5)] = h;
     } else if (p >= kGOffW2 && p < kGOffB2) {
         const int k = p - kGOffW2;
         wbf[kGW2 + frag_at(k / kGHid, k % kGHid, 2, 4)] = h;
-        wbf[kGWT2 + frag_at(k % kGHid, k / kGHid, 2, 4)] = h;
+        wbf[kGTW2 + frag16_at(k / kGHid, k % kGHid, 4)] = h;
+        wbf[kGWT2 + frag16_at(k % kGHid, k / kGHid, 4)] = h;
     } else if (p >= kGOffW3 && p < kGOffB3) {
         const int k = p - kGOffW3;
         wbf[kGW3 + frag_at(k / kGHid, k % kGHid, 2, 4)] = h;
-        wbf[kGWT3 + frag_at(k % kGHid, k / kGHid, 2, 4)] = h;
+        wbf[kGTW3 + frag16_at(k / kGHid, k % kGHid, 4)] = h;
+        wbf[kGWT3 + frag16_at(k % kGHid, k / kGHid, 4)] = h;
     } else if (p >= kGOffW4 && p < kGOffB4) {
         const int k = p - kGOffW4;
         wbf[kGW4 + frag_at(k / kGHid, k % kGHid, 2, 3)] = h;
-        wbf[kGWT4 + frag_at(k % kGHid, k / kGHid, 1, 4)] = h;
+        wbf[kGTW4 + frag16_at(k / kGHid, k % kGHid, 4)] = h;
+        wbf[kGWT4 + frag16_at(k % kGHid, k / kGHid, 3)] = h;
     }
 }
 
@@ -165,10 +169,12 @@ constexpr int kTStride = 64 + 8;  // row stride (u16) of the transposed [feature
 // outputs.  Returns -log q.
 __device__ __forceinline__ float guide_dout(const float* o, float3 w, float c, float* d) {
     const float kLog2Pi = 1.83787706640934548356f;
-    auto sum8 = [](float x) {
-        x += __shfl_xor(x, 8, 64);
-        x += __shfl_xor(x, 16, 64);
-        return x + __shfl_xor(x, 32, 64);
+    auto sum8 = [](float x) {  // in the lobes' order
+        const int first = (int)(threadIdx.x & 7u);
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < kGLobes; ++j) s += __shfl(x, first + 8 * j, 64);
+        return s;
     };
     auto max8 = [](float x) {
         x = fmaxf(x, __shfl_xor(x, 8, 64));
@@ -219,34 +225,28 @@ struct TrainSrc {
     uint64_t subset_seed;  // fixes which ones
 };
 
-// Two output tiles, mt0 and mt0 + 1, of Y^T = W X^T for 16 samples (guide_layer's
-// sequence): B fragments from their rows (stride in u16), epi(0 or 1, first
-// output, accumulator).
-template <int KT32, bool TAIL, int OUT_TILES, class Epi>
+// Two output tiles, mt0 and mt0 + 1, of Y^T = W X^T for 16 samples, K = 16 KT:
+// B fragments from their rows (stride in u16), epi(0 or 1, first output,
+// accumulator).  In K = 16 steps: a rounding that falls otherwise flips the sign of
+// a gradient near zero, and with it a whole Adam step, so the sums keep one order.
+template <int KT, class Epi>
 __device__ __forceinline__ void train_product(int l, const uint16_t* W, int mt0, const uint16_t* rows, int stride,
                                               Epi epi) {
     const int s = l & 15, grp = l >> 4;
-    g_bf8 a[2][KT32], b[KT32];
-    g_s4 at[2] = {}, bt = {};
+    g_s4 a[2][KT], b[KT];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
+    for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-        for (int kt = 0; kt < KT32; ++kt) a[mt][kt] = frag32<KT32, OUT_TILES>(W, mt0 + mt, kt, l);
-        if (TAIL) at[mt] = frag16<KT32, OUT_TILES>(W, mt0 + mt, l);
-    }
+        for (int kt = 0; kt < KT; ++kt)
+            a[mt][kt] = *reinterpret_cast<const g_s4*>(reinterpret_cast<const char*>(W) +
+                                                       (8u * (uint32_t)l + 512u * (uint32_t)((mt0 + mt) * KT + kt)));
 #pragma unroll
-    for (int kt = 0; kt < KT32; ++kt) b[kt] = *reinterpret_cast<const g_bf8*>(rows + s * stride + 32 * kt + 8 * grp);
-    if (TAIL) bt = *reinterpret_cast<const g_s4*>(rows + s * stride + 32 * KT32 + 4 * grp);
+    for (int kt = 0; kt < KT; ++kt) b[kt] = *reinterpret_cast<const g_s4*>(rows + s * stride + 16 * kt + 4 * grp);
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
         g_f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kt = 0; kt < KT32; ++kt) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][kt], b[kt], acc, 0, 0, 0);
-        if (TAIL) {
-            g_f4 t = {0.f, 0.f, 0.f, 0.f};
-            t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(at[mt], bt, t, 0, 0, 0);
-            acc += t;
-        }
+        for (int kt = 0; kt < KT; ++kt) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mt][kt], b[kt], acc, 0, 0, 0);
         epi(mt, 16 * (mt0 + mt) + 4 * grp, acc);
     }
 }
@@ -257,10 +257,10 @@ __device__ __forceinline__ void grad_tile(int l, g_f4& acc, const uint16_t* dt, 
                                           int hrow) {
     const int r = l & 15, grp = l >> 4;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-        const g_bf8 a = *reinterpret_cast<const g_bf8*>(dt + (drow + r) * kTStride + 32 * kt + 8 * grp);
-        const g_bf8 b = *reinterpret_cast<const g_bf8*>(ht + (hrow + r) * kTStride + 32 * kt + 8 * grp);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+    for (int kt = 0; kt < 4; ++kt) {
+        const g_s4 a = *reinterpret_cast<const g_s4*>(dt + (drow + r) * kTStride + 16 * kt + 4 * grp);
+        const g_s4 b = *reinterpret_cast<const g_s4*>(ht + (hrow + r) * kTStride + 16 * kt + 4 * grp);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
     }
 }
 
@@ -419,15 +419,15 @@ __global__ __launch_bounds__(kTrainBlock, 2 * kTrainBlocksPerCu) void k_guide_tr
                 t[3 * kTStride] = (uint16_t)(h.y >> 16);
             };
         };
-        train_product<2, true, 4>(lo, G.wbf + kGW1, 2 * half, ra, kGStrideIn, hidden(0, G.theta + kGOffB1, rb, kGStrideHid));
+        train_product<5>(lo, G.wbf + kGTW1, 2 * half, ra, kGStrideIn, hidden(0, G.theta + kGOffB1, rb, kGStrideHid));
         __syncthreads();
-        train_product<2, false, 4>(lo, G.wbf + kGW2, 2 * half, rb, kGStrideHid, hidden(1, G.theta + kGOffB2, ra, kGStrideIn));
+        train_product<4>(lo, G.wbf + kGTW2, 2 * half, rb, kGStrideHid, hidden(1, G.theta + kGOffB2, ra, kGStrideIn));
         __syncthreads();
-        train_product<2, false, 4>(lo, G.wbf + kGW3, 2 * half, ra, kGStrideIn, hidden(2, G.theta + kGOffB3, rb, kGStrideHid));
+        train_product<4>(lo, G.wbf + kGTW3, 2 * half, ra, kGStrideIn, hidden(2, G.theta + kGOffB3, rb, kGStrideHid));
         __syncthreads();
         float* out = reinterpret_cast<float*>(ra);
         // 48 padded outputs: the second half's tiles overlap the first's by one
-        train_product<2, false, 3>(lo, G.wbf + kGW4, half, rb, kGStrideHid, [&](int mt, int o, g_f4 v) {
+        train_product<4>(lo, G.wbf + kGTW4, half, rb, kGStrideHid, [&](int mt, int o, g_f4 v) {
             if (o >= kGOut || (half && mt == 0)) return;  // padded rows 40..47
             const float4 b = *reinterpret_cast<const float4*>(G.theta + kGOffB4 + o);
             *reinterpret_cast<float4*>(out + smp * kGOut + o) =
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(kTrainBlock, 2 * kTrainBlocksPerCu) void k_guide_tr
             };
         };
         // layer 4 (64 -> 40)
-        train_product<1, true, 4>(lo, G.wbf + kGWT4, 2 * half, rb, kGStrideHid, back(2, ra, kGStrideIn, dt[1]));
+        train_product<3>(lo, G.wbf + kGWT4, 2 * half, rb, kGStrideHid, back(2, ra, kGStrideIn, dt[1]));
         if (half) {
             grad_tile(lo, a4[0], dt[0], 32, ht[2], 16 * q);
             if (q < 3) bias_tile(lo, b4, dt[0], 16 * q);
@@ -480,13 +480,13 @@ __global__ __launch_bounds__(kTrainBlock, 2 * kTrainBlocksPerCu) void k_guide_tr
         }
         __syncthreads();
         // layer 3
-        train_product<2, false, 4>(lo, G.wbf + kGWT3, 2 * half, ra, kGStrideIn, back(1, rb, kGStrideHid, dt[0]));
+        train_product<4>(lo, G.wbf + kGWT3, 2 * half, ra, kGStrideIn, back(1, rb, kGStrideHid, dt[0]));
 #pragma unroll
         for (int k = 0; k < 2; ++k) grad_tile(lo, a3[k], dt[1], 16 * q, ht[1], 32 * half + 16 * k);
         if (half) bias_tile(lo, b3, dt[1], 16 * q);
         __syncthreads();
         // layer 2
-        train_product<2, false, 4>(lo, G.wbf + kGWT2, 2 * half, rb, kGStrideHid, back(0, ra, kGStrideIn, dt[1]));
+        train_product<4>(lo, G.wbf + kGWT2, 2 * half, rb, kGStrideHid, back(0, ra, kGStrideIn, dt[1]));
 #pragma unroll
         for (int k = 0; k < 2; ++k) grad_tile(lo, a2[k], dt[0], 16 * q, ht[0], 32 * half + 16 * k);
         if (!half) bias_tile(lo, b2, dt[0], 16 * q);

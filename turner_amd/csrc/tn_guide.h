@@ -30,7 +30,11 @@ constexpr int kGParams = kGOffB4 + 40;  // 15976
 // (backward A operand, [in_pad][out_pad]) in fragment order (frag_at)
 constexpr int kGW1 = 0, kGW2 = kGW1 + 64 * kGInPad, kGW3 = kGW2 + 64 * 64, kGW4 = kGW3 + 64 * 64;
 constexpr int kGWT2 = kGW4 + kGOutPad * 64, kGWT3 = kGWT2 + 64 * 64, kGWT4 = kGWT3 + 64 * 64;
-constexpr int kGBf16 = kGWT4 + 64 * kGOutPad;
+// the training kernel's copies of W_l; these and W_l^T in fragments of K = 16
+// (frag16_at)
+constexpr int kGTW1 = kGWT4 + 64 * kGOutPad, kGTW2 = kGTW1 + 64 * kGInPad, kGTW3 = kGTW2 + 64 * 64,
+              kGTW4 = kGTW3 + 64 * 64;
+constexpr int kGBf16 = kGTW4 + kGOutPad * 64;
 
 // Position of element (row, col) of a padded [16 out_tiles][cols] matrix in
 // fragment order: for every 16-row tile the K = 32 fragments of its columns,
@@ -44,6 +48,11 @@ __host__ __device__ constexpr int frag_at(int row, int col, int kt32, int out_ti
     if (col < 32 * kt32) return ((mt * kt32 + col / 32) * 64 + col % 32 / 8 * 16 + r) * 8 + col % 8;
     const int c = col - 32 * kt32;
     return out_tiles * kt32 * 512 + (mt * 64 + c / 4 * 16 + r) * 4 + c % 4;
+}
+
+// The same in K = 16 fragments alone (64 lanes of 4 columns each), kt16 per row tile.
+__host__ __device__ constexpr int frag16_at(int row, int col, int kt16) {
+    return ((row / 16 * kt16 + col / 16) * 64 + col % 16 / 4 * 16 + row % 16) * 4 + col % 4;
 }
 
 struct GuideView {
