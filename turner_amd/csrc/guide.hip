@@ -307,10 +307,10 @@ __device__ __forceinline__ void store_bias(const g_f4& acc, float* __restrict__ 
 // gradients stay in registers over all groups of the block: one 64 KB slice per
 // block, at most two blocks per compute unit.
 // Measured against blocks of four waves that each took 64 samples by themselves,
-// with row-major weights: 16,384 samples 37.4 -> 20.7 us (33.9 with eight waves
-// but row-major weights, 31.2 with four); whole step with its update at 64
-// samples 39.5 -> 16.9, 16,384 47.8 -> 26.2, 131,072 104.5 -> 65.7, 1,048,576
-// 897 -> 375 us.
+// with row-major weights: 16,384 samples 37.4 -> 23.8 us (20.7 with K = 32 steps
+// and tree sums, which round otherwise; then 33.9 with row-major weights, 31.2
+// with four waves); whole step with its update at 64 samples 39.5 -> 20.0, 16,384
+// 47.8 -> 29.2, 131,072 104.5 -> 82.9, 1,048,576 897 -> 509 us.
 __global__ __launch_bounds__(kTrainBlock, 2 * kTrainBlocksPerCu) void k_guide_train(GuideView G, TrainSrc S,
                                                                                    float* __restrict__ partial,
                                                                                    float* __restrict__ sums) {
