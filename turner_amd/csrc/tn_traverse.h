@@ -582,7 +582,7 @@ struct CoopHit {
     uint32_t id;
     float r, s, t;
     bool tie;         // another triangle was hit at exactly r (TIE)
-    uint32_t visits;  // leaves visited
+    uint32_t visits;  // leaves visited (COUNT)
 };
 
 // One ray of the cooperative loop.  Its stack holds the entries base .. head-1
@@ -597,7 +597,7 @@ struct CoopRay {
     float tenter, texit, root_exit;
     uint32_t node, root;
     int head, base, restarts;
-    uint32_t visits;  // leaves visited, kTied: another triangle was hit at exactly best_r
+    uint32_t visits;  // leaves left behind, kTied: another triangle was hit at exactly best_r
     float best_r;
     uint32_t best_ref;  // reference slot of the best hit
 };
@@ -913,7 +913,11 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                 }
             }
             if (done) {
-                if (COUNT) cnt.restarts += R.restarts;
+                if (COUNT) {
+                    cnt.restarts += R.restarts;
+                    // its last leaf, unless that is the one it was abandoned at
+                    R.visits += (R.visits & ~kTied) <= kMaxLeafVisits ? 1u : 0u;
+                }
                 R.node = kDone;
             }
         }
