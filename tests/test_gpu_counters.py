@@ -1,6 +1,8 @@
 """Work counters of TN_ISECT_COUNT launches.  The cooperative traversal visits the
 nodes, leaves and triangles that the schedule of a leaf per lane does, so all counts
-but [6] are equal: whole numbers, no tolerance."""
+but [6] are equal: whole numbers, no tolerance.  [6] counts the records read whole:
+every one in launches of at most a ray per lane on the reference tree (which read
+both halves at once), else those whose first half did not decide."""
 import numpy as np
 import pytest
 
@@ -41,3 +43,16 @@ def test_longest_traversal_of_a_refined_tree(gpu):
     tree = T.KDTree(SCENES["one"](), refined=True)
     c = _counts(tree, 64, TN_ISECT_REFINED)
     assert c[1] > 0 and c[7] == 1  # the only leaf
+
+
+def test_whole_records(gpu):
+    tree = T.KDTree(SCENES["sphere"](), refined=True)
+    _, cus = T.device_info()
+    lanes = cus * 28 * 64  # resident lanes
+    for n in (1, 1000, lanes):
+        c = _counts(tree, n, 0)
+        assert c[6] == c[3] > 0, f"{n} rays"
+    c = _counts(tree, lanes + 1, 0)
+    assert 0 < c[6] < c[3]
+    c = _counts(tree, 1000, TN_ISECT_REFINED)
+    assert 0 < c[6] < c[3]

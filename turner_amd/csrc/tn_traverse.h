@@ -832,7 +832,7 @@ __device__ __forceinline__ void coop_loop(const SceneView& sc, uint2* stk, int s
                     if (COUNT) {
                         cnt.refs++;
                         cnt.tests++;
-                        cnt.full += code >= 1 ? 1u : 0u;
+                        cnt.full += whole || code >= 1 ? 1u : 0u;
                     }
                     if (code >= 2) {
                         if (ANY) {
