@@ -204,7 +204,8 @@ int tn_intersect(tn_scene* scene, const float* o3, const float* d3, uint32_t n,
 int tn_intersect_noalloc(tn_scene* scene, const float* o3, const float* d3, uint32_t n,
                          uint32_t* id, float* r, float* s, float* t, uint32_t flags, void* stream);
 /* Host-pointer variant (synchronous; up to 65,536 rays pass through pinned
- * memory that the kernels access, larger calls are copied in and out). */
+ * memory that the kernels access; larger calls, and all where no pinned memory
+ * is to be had, are copied in and out). */
 int tn_intersect_host(tn_scene* scene, const float* o3, const float* d3, uint32_t n,
                       uint32_t* id, float* r, float* s, float* t, uint32_t flags);
 /* Shadow / visibility query with the reference's predicate

@@ -1,0 +1,45 @@
+"""Calls that use pinned host memory when they can get it, in a process where it is
+refused: they work as they do with it."""
+import os
+import subprocess
+
+import pytest
+
+from tests import child
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def refuse(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("refuse") / "librefuse.so")
+    src = os.path.join(child.ROOT, "tests", "cpp", "refuse_alloc.cpp")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-o", so, src, "-ldl"], check=True)
+    return so
+
+
+SETUP = """
+import ctypes, json, sys
+shim = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+shim.refuse_host_blocks.argtypes = [ctypes.c_size_t]
+import numpy as np, torch
+import turner_amd as T
+from turner_amd import scenes
+"""
+
+
+@pytest.mark.parametrize("refined", [0, 1])
+def test_host_rays(gpu, refuse, refined):
+    got = child.run(SETUP + """
+tree = T.KDTree(scenes.intersect_scene(level=3)["verts"], refined=bool(int(sys.argv[2])))
+q = T.KDTreeIntersection(tree)
+res = {}
+shim.refuse_pinned_memory(1)
+o, d = scenes.random_rays(65536, seed=5)
+for n in (1, 1000, 65536):
+    res[n] = q.intersect_batch(o[:n], d[:n])
+shim.refuse_pinned_memory(0)
+print(json.dumps([all(np.array_equal(a.view(np.uint32), b.view(np.uint32))
+                      for a, b in zip(res[n], q.intersect_batch(o[:n], d[:n]))) for n in res]))
+""", refuse, refined)
+    assert got == [True, True, True]

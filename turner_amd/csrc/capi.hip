@@ -352,15 +352,19 @@ int tn_scene::reserve_stage(size_t bytes) {
     return TN_OK;
 }
 
-int tn_scene::reserve_pinned(size_t bytes) {
-    if (h_stage && h_cap >= bytes) return TN_OK;
+bool tn_scene::reserve_pinned(size_t bytes) {
+    if (h_stage && h_cap >= bytes) return true;
     if (h_stage) (void)hipHostFree(h_stage);
     h_stage = nullptr;
     h_cap = 0;
     bytes = std::max<size_t>(bytes, 4096);
-    TN_HIP(hipHostMalloc((void**)&h_stage, bytes, hipHostMallocDefault));
+    if (hipHostMalloc((void**)&h_stage, bytes, hipHostMallocDefault) != hipSuccess) {
+        h_stage = nullptr;
+        (void)hipGetLastError();  // the caller does without
+        return false;
+    }
     h_cap = bytes;
-    return TN_OK;
+    return true;
 }
 
 namespace tn {
@@ -861,12 +865,12 @@ int tn_intersect_host(tn_scene* sc, const float* o3, const float* d3, uint32_t n
     TN_HIP(hipSetDevice(sc->device));
     std::lock_guard<std::mutex> lock(sc->stage_mu);
     const size_t ray_bytes = (size_t)n * 12;
-    if (n <= tn_scene::kPinnedRays) {
+    if (n <= tn_scene::kPinnedRays && sc->reserve_pinned(64 + 2 * ray_bytes + (size_t)n * 16)) {
         // The kernels read the rays from pinned memory and write the hits there:
         // one wait instead of seven copies that each block.  One ray 98 -> 26 us
         // (refined tree 101 -> 30), 65,536 rays 330 -> 239 us; the line bounds the
-        // pinned memory, beyond it the traversal outweighs the copies.
-        if (int rc = sc->reserve_pinned(64 + 2 * ray_bytes + (size_t)n * 16)) return rc;
+        // pinned memory, beyond it the traversal outweighs the copies.  Where no
+        // pinned memory is to be had, small calls are copied as well.
         uint32_t* h_st = (uint32_t*)sc->h_stage;
         float* h_o = (float*)(sc->h_stage + 64);
         float* h_d = h_o + 3 * (size_t)n;

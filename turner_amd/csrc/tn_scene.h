@@ -74,9 +74,9 @@ struct tn_scene {
     size_t h_cap = 0;
 
     // Device memory of at least `bytes` in d_stage, pinned memory in h_stage
-    // (caller holds stage_mu).
+    // (false: there is none; caller holds stage_mu).
     int reserve_stage(size_t bytes);
-    int reserve_pinned(size_t bytes);
+    bool reserve_pinned(size_t bytes);
 
     // the refined tree (TN_SCENE_REFINED scenes only)
     tn::SceneView fview() const {
