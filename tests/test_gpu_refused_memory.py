@@ -43,3 +43,27 @@ print(json.dumps([all(np.array_equal(a.view(np.uint32), b.view(np.uint32))
                       for a, b in zip(res[n], q.intersect_batch(o[:n], d[:n]))) for n in res]))
 """, refuse, refined)
     assert got == [True, True, True]
+
+
+def test_renders(gpu, refuse):
+    got = child.run(SETUP + """
+from turner_amd import batch
+sc = scenes.cornell_box()
+tree = T.KDTree(sc["verts"], sc["normals"], sc["albedo"], sc["emission"])
+b = batch.Batch([tree, tree])
+jobs = [{"camera": sc["camera"], "lights": sc["lights"], "width": w, "height": 40, "spp": 2} for w in (30, 41)]
+conf = T.TracerConfig(width=64, max_recursion_depth=2, num_pixel_samples=4, num_monte_carlo_samples=2, flags=4)
+
+def all_of():
+    img, st = T.render(tree, sc["camera"], sc["lights"], conf)
+    images, bst, _ = b.render(jobs, max_depth=2, mc_samples=1, flags=3, seed=1)
+    return [img, *(np.asarray(x.cpu() if hasattr(x, "cpu") else x) for x in images)], [st["rays"], st["shadow_rays"], bst["rays"]]
+
+shim.refuse_pinned_memory(1)
+a, sa = all_of()
+shim.refuse_pinned_memory(0)
+c, sc_ = all_of()
+# FP32 sums of at most 4 x 7 contributions in another order
+print(json.dumps([sa == sc_, all(bool(np.allclose(x, y, rtol=1e-5, atol=1e-6)) for x, y in zip(a, c)), sa[0] > 0]))
+""", refuse)
+    assert got == [True, True, True]

@@ -343,7 +343,8 @@ __device__ __forceinline__ void chunk_begin_block(uint32_t* cnt, uint32_t* xwork
     }
 }
 
-// What a render reports, in pinned host memory: each pipeline writes its own
+// What a render reports, in pinned host memory (or, where there is none, in the
+// pipeline's own memory, copied back at the end): each pipeline writes its own
 // after every chunk, so that the call ends with a stream synchronisation alone.
 struct RenderReport {
     unsigned long long rays, shadow_rays;
@@ -1396,6 +1397,7 @@ struct RenderBuffers {
     size_t bytes = 0;
     char* base = nullptr;
     ChunkState* cs = nullptr;
+    RenderReport* rep = nullptr;  // where no memory is pinned
     SceneParams* sp = nullptr;
     uint32_t sp_cap = 0;
     // the shadow tests run on a second stream (default priority), ordered
@@ -1423,7 +1425,7 @@ constexpr int kMaxDevices = 64;
 
 // Carves the queue buffers out of one allocation; with base == nullptr it
 // only measures (every piece is rounded up to 256 bytes).
-size_t carve(Queues& q, ChunkState** cs, char* base, uint32_t cap) {
+size_t carve(Queues& q, ChunkState** cs, RenderReport** rep, char* base, uint32_t cap) {
     size_t off = 0;
     auto take = [&](size_t b) {
         char* r = base ? base + off : nullptr;
@@ -1451,6 +1453,7 @@ size_t carve(Queues& q, ChunkState** cs, char* base, uint32_t cap) {
     q.totals = (unsigned long long*)take(2 * sizeof(unsigned long long));
     q.bar = (uint32_t*)take(kBarWords * sizeof(uint32_t));
     *cs = (ChunkState*)take(sizeof(ChunkState));
+    *rep = (RenderReport*)take(sizeof(RenderReport));
     q.cap = cap;
     return off;
 }
@@ -1469,7 +1472,8 @@ int reserve_scenes(RenderBuffers& rb, uint32_t nscenes) {
 size_t queue_bytes(uint32_t cap) {
     Queues probe{};
     ChunkState* pcs = nullptr;
-    return carve(probe, &pcs, nullptr, cap);
+    RenderReport* prep = nullptr;
+    return carve(probe, &pcs, &prep, nullptr, cap);
 }
 
 // Queues of `cap` entries for the first npipes pipelines.  share > 0: refused with
@@ -1511,7 +1515,7 @@ int reserve_queues(RenderBuffers* rbs, int npipes, uint32_t cap, size_t share) {
             return hip_error(e, "hipMalloc(ray queues)");
         }
         rb.bytes = need;
-        carve(rb.q, &rb.cs, rb.base, take);
+        carve(rb.q, &rb.cs, &rb.rep, rb.base, take);
     }
     return TN_OK;
 }
@@ -1541,7 +1545,8 @@ struct RenderContext {
     float* jitter = nullptr;  // reference pixel jitter (TN_RENDER_REF_JITTER)
     size_t jitter_cap = 0;
     // pinned: the pipelines' reports, then scene table and jitter on their way to
-    // the device (free again when the call that wrote them returns)
+    // the device (free again when the call that wrote them returns; null where no
+    // pinned memory is to be had)
     char* host = nullptr;
     size_t host_cap = 0;
     // graph replay (TN_RENDER_GRAPH): the capture stream and the executable
@@ -1555,15 +1560,19 @@ struct RenderContext {
 // Pinned jitter is at most this; a longer table takes a copy of its own.
 constexpr size_t kPinnedJitter = 1u << 20;
 
-int reserve_host(RenderContext& C, size_t bytes) {
-    if (C.host && C.host_cap >= bytes) return TN_OK;
+bool reserve_host(RenderContext& C, size_t bytes) {
+    if (C.host && C.host_cap >= bytes) return true;
     if (C.host) (void)hipHostFree(C.host);
     C.host = nullptr;
     C.host_cap = 0;
     bytes = std::max<size_t>(bytes, 1u << 16);
-    TN_HIP(hipHostMalloc((void**)&C.host, bytes, hipHostMallocDefault));
+    if (hipHostMalloc((void**)&C.host, bytes, hipHostMallocDefault) != hipSuccess) {
+        C.host = nullptr;
+        (void)hipGetLastError();  // the caller does without
+        return false;
+    }
     C.host_cap = bytes;
-    return TN_OK;
+    return true;
 }
 
 RenderContext& render_context(int device) {
@@ -1878,14 +1887,18 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         if ((rc = alloc_records(C.recs[p], (size_t)chunk * ((uint32_t)P->max_depth + 1)))) return rc;
     const size_t table_bytes = table.size() * sizeof(SceneParams);
     const size_t jitter_bytes = jitter_host ? jitter_len * sizeof(float) : 0;
-    const bool pin_jitter = jitter_bytes <= kPinnedJitter;
+    bool pin_table = true, pin_jitter = jitter_bytes <= kPinnedJitter;
     static_assert(sizeof(RenderReport) * kPipes <= 256 && sizeof(SceneParams) % 4 == 0, "layout of the pinned memory");
-    if ((rc = reserve_host(C, 256 + table_bytes + (pin_jitter ? jitter_bytes : 0)))) return rc;
-    RenderReport* report = (RenderReport*)C.host;
-    std::memcpy(C.host + 256, table.data(), table_bytes);
-    if (pin_jitter && jitter_bytes) std::memcpy(C.host + 256 + table_bytes, jitter_host, jitter_bytes);
-    for (int p = 0; p < npipes; ++p) report[p] = RenderReport{};
+    const size_t jitter_at = 256 + (pin_table ? table_bytes : 0);
+    const bool pinned = reserve_host(C, jitter_at + (pin_jitter ? jitter_bytes : 0));
+    if (!pinned) pin_table = pin_jitter = false;
+    if (pin_table) std::memcpy(C.host + 256, table.data(), table_bytes);
+    if (pin_jitter && jitter_bytes) std::memcpy(C.host + jitter_at, jitter_host, jitter_bytes);
+    RenderReport* report[kPipes];
+    for (int p = 0; p < npipes; ++p) report[p] = pinned ? (RenderReport*)C.host + p : rbs[p].rep;
     enqueued = true;
+    if (!pin_table)
+        TN_RHIP(hipMemcpyAsync(rbs[0].sp, table.data(), table_bytes, hipMemcpyHostToDevice, stream));
 
     RenderArgs A0{};
     A0.sv = G.sv;
@@ -1966,10 +1979,10 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
     R.total = total;
     R.persistent = persistent;
     R.incomplete = G.status + 2;
-    R.src[0] = (const uint32_t*)(C.host + 256);
+    R.src[0] = pin_table ? (const uint32_t*)(C.host + 256) : nullptr;
     R.dst[0] = (uint32_t*)rbs[0].sp;
-    R.words[0] = (uint32_t)(table_bytes / 4);
-    R.src[1] = (const uint32_t*)(C.host + 256 + table_bytes);
+    R.words[0] = pin_table ? (uint32_t)(table_bytes / 4) : 0u;
+    R.src[1] = pin_jitter ? (const uint32_t*)(C.host + jitter_at) : nullptr;
     R.dst[1] = (uint32_t*)C.jitter;
     R.words[1] = pin_jitter ? (uint32_t)(jitter_bytes / 4) : 0u;
     const uint32_t start_blocks = std::min<uint32_t>(64u, 1u + (R.words[0] + R.words[1]) / 512u);
@@ -2056,7 +2069,7 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
                                       renderer == TN_RENDERER_RAYCASTER   ? -1
                                       : renderer == TN_RENDERER_RAYTRACER ? levels + 1
                                                                           : levels,
-                                      report + p);
+                                      report[p]);
         return e;
     };
     // One chunk of each of n pipelines on its stream, enqueued level by level, so
@@ -2106,7 +2119,7 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         int plevels = levels;
         void* args[] = {&pa, &pq, &plevels};
         TN_RHIP(hipLaunchCooperativeKernel(kfn, pgrid, dim3(kRBlock), args, 0, stream));
-        k_persist_end<<<1, 64, 0, stream>>>(Q[0], G.status + 2, report);
+        k_persist_end<<<1, 64, 0, stream>>>(Q[0], G.status + 2, report[0]);
     } else if (shape.graph && rounds > 1) {
         // The chunk sequence is captured on every call (host-side recording;
         // its kernel arguments change from call to call) and applied to the
@@ -2152,21 +2165,26 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
     }
     if (deferred) TN_RHIP(hipStreamWaitEvent(stream, guide->ev_join, 0));
     TN_RHIP(hipStreamSynchronize(stream));
+    RenderReport seen[kPipes];
+    for (int p = 0; p < npipes; ++p) {
+        if (pinned) seen[p] = *report[p];
+        else TN_RHIP(hipMemcpy(&seen[p], report[p], sizeof(RenderReport), hipMemcpyDeviceToHost));
+    }
 #undef TN_RHIP
     const double ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     for (int p = 0; p < npipes; ++p)
-        if (report[p].overflow) return set_error(TN_ERR_QUEUE, "a ray queue overflowed");
-    if (report[0].barrier_out) return set_error(TN_ERR_INCOMPLETE, "a grid barrier wait of the persistent kernel ran out");
+        if (seen[p].overflow) return set_error(TN_ERR_QUEUE, "a ray queue overflowed");
+    if (seen[0].barrier_out) return set_error(TN_ERR_INCOMPLETE, "a grid barrier wait of the persistent kernel ran out");
     // counted by both pipelines in one word: the later report has them all
     uint32_t incomplete = 0;
-    for (int p = 0; p < npipes; ++p) incomplete = std::max(incomplete, report[p].incomplete);
+    for (int p = 0; p < npipes; ++p) incomplete = std::max(incomplete, seen[p].incomplete);
     if (incomplete) return set_error(TN_ERR_INCOMPLETE, "%u render traversals hit the visit cap", incomplete);
     if (st) {
         st->rays = st->shadow_rays = 0;
         for (int p = 0; p < npipes; ++p) {
-            st->rays += report[p].rays;
-            st->shadow_rays += report[p].shadow_rays;
+            st->rays += seen[p].rays;
+            st->shadow_rays += seen[p].shadow_rays;
         }
         st->primary_rays = rays ? 0 : total;
         st->ms = ms;
