@@ -1557,8 +1557,8 @@ struct RenderContext {
     uint64_t graph_instantiations = 0, graph_updates = 0;
 };
 
-// Pinned jitter is at most this; a longer table takes a copy of its own.
-constexpr size_t kPinnedJitter = 1u << 20;
+// A pinned scene table or jitter is at most this; a longer one takes a copy of its own.
+constexpr size_t kPinnedTable = 1u << 20;
 
 bool reserve_host(RenderContext& C, size_t bytes) {
     if (C.host && C.host_cap >= bytes) return true;
@@ -1887,7 +1887,7 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         if ((rc = alloc_records(C.recs[p], (size_t)chunk * ((uint32_t)P->max_depth + 1)))) return rc;
     const size_t table_bytes = table.size() * sizeof(SceneParams);
     const size_t jitter_bytes = jitter_host ? jitter_len * sizeof(float) : 0;
-    bool pin_table = true, pin_jitter = jitter_bytes <= kPinnedJitter;
+    bool pin_table = table_bytes <= kPinnedTable, pin_jitter = jitter_bytes <= kPinnedTable;
     static_assert(sizeof(RenderReport) * kPipes <= 256 && sizeof(SceneParams) % 4 == 0, "layout of the pinned memory");
     const size_t jitter_at = 256 + (pin_table ? table_bytes : 0);
     const bool pinned = reserve_host(C, jitter_at + (pin_jitter ? jitter_bytes : 0));
