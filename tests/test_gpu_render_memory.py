@@ -1,0 +1,65 @@
+"""Device memory of the ray queues: what a first render takes, and what is left when
+little is free.  Each in a process of its own, in bytes that the driver reports free."""
+import pytest
+
+from tests import child
+
+pytestmark = pytest.mark.gpu
+
+SETUP = """
+import json, sys
+import numpy as np, torch
+import turner_amd as T
+from turner_amd import scenes
+
+def free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+def tree_of(sc):
+    t = T.KDTree(sc["verts"], sc["normals"], sc["albedo"], sc["emission"])
+    T.KDTreeIntersection(t).intersect([0, 0, 0], [0, 0, 1])
+    return t
+
+def render(t, sc, w, h, spp, m, depth, **kw):
+    conf = T.TracerConfig(width=w, aspect=w / h, max_recursion_depth=depth, num_pixel_samples=spp,
+                          num_monte_carlo_samples=m, seed=5, flags=3, **kw)
+    acc = torch.zeros((h, w, 4), device="cuda")
+    st = T.render_accumulate(t, sc["camera"], sc["lights"], conf, acc)
+    return acc.cpu().numpy(), st["rays"]
+
+def leave(n):  # a ballast that leaves n bytes free
+    global ballast
+    ballast = None
+    torch.cuda.empty_cache()
+    ballast = torch.empty(free() - n, dtype=torch.uint8, device="cuda")
+
+sc = scenes.furnace(level=1)
+sc["lights"] = [((0.0, 3.0, -3.0), (1.0, 1.0, 1.0, 1.0))]
+t = tree_of(sc)
+acc = torch.zeros((512, 1024, 4), device="cuda")
+"""
+
+MB = 1 << 20
+
+
+def test_chunks_sized_by_the_caller(gpu):
+    few, many = (child.run(SETUP + """
+f = free()
+render(t, sc, 1024, 1024, 1, 1, 2, chunk_paths=int(sys.argv[1]))
+print(json.dumps(f - free()))
+""", chunk) for chunk in (4096, 1 << 19))
+    # two pipelines with 404 B per entry: what the larger chunks take more (what streams
+    # take is in both); an allocation is a multiple of 2 MiB
+    assert abs(many - few - 2 * 404 * ((1 << 19) - 4096)) <= 8 * MB
+
+
+def test_small_render_with_little_memory_free(gpu):
+    got = child.run(SETUP + """
+leave(3 << 30)
+f = free()
+img, n = render(t, sc, 64, 64, 1, 2, 2)
+print(json.dumps([f - free(), n, int(np.isfinite(img).all())]))
+""")
+    # at most a quarter of 3 GiB goes to queues that this render does not need
+    assert got[0] <= 768 * MB and got[1] == 64 * 64 * 7 and got[2]

@@ -1390,7 +1390,9 @@ std::vector<float> reference_jitter(uint32_t width, uint32_t spp) {
     return j;
 }
 
-constexpr uint32_t kLeastQueueAlloc = 1u << 22;  // entries: small renders of growing sizes share one allocation
+// Entries of a first allocation (1.7 GB), so that small renders of growing sizes
+// share it; not when the caller sizes the chunks, nor from scarce memory.
+constexpr uint32_t kLeastQueueAlloc = 1u << 22;
 
 struct RenderBuffers {
     Queues q{};
@@ -1476,24 +1478,27 @@ size_t queue_bytes(uint32_t cap) {
     return carve(probe, &pcs, &prep, nullptr, cap);
 }
 
-// Queues of `cap` entries for the first npipes pipelines.  share > 0: refused with
-// TN_ERR_OOM, before anything is touched, if what has to be allocated exceeds
-// 1/share of the memory that is free or held by the queues it replaces.
-int reserve_queues(RenderBuffers* rbs, int npipes, uint32_t cap, size_t share) {
-    const uint32_t least = std::max(cap, kLeastQueueAlloc);
-    size_t grow = 0, held = 0;
+constexpr size_t kFreeShare = 4;  // new queues take at most a quarter of the free memory
+
+// Queues of `cap` entries for the first npipes pipelines, of kLeastQueueAlloc
+// unless `exact` or those exceed 1/kFreeShare of the memory that is free or held by
+// the queues they replace.  limited: TN_ERR_OOM, before anything is touched, if
+// `cap` entries exceed it.
+int reserve_queues(RenderBuffers* rbs, int npipes, uint32_t cap, bool exact, bool limited) {
+    size_t lacking = 0, held = 0;  // pipelines to allocate for, and what they hold
     for (int p = 0; p < npipes; ++p)
         if (!rbs[p].base || rbs[p].q.cap < cap) {
-            grow += queue_bytes(least);
+            ++lacking;
             held += rbs[p].bytes;
         }
-    if (!grow) return TN_OK;
-    if (share) {
-        size_t free_bytes = 0, all = 0;
-        TN_HIP(hipMemGetInfo(&free_bytes, &all));
-        if (grow > (free_bytes + held) / share)
-            return set_error(TN_ERR_OOM, "queues of %zu bytes, %zu are free", grow, free_bytes);
-    }
+    if (!lacking) return TN_OK;
+    size_t free_bytes = 0, all = 0;
+    TN_HIP(hipMemGetInfo(&free_bytes, &all));
+    const size_t share = (free_bytes + held) / kFreeShare;
+    uint32_t least = exact ? cap : std::max(cap, kLeastQueueAlloc);
+    if (least > cap && lacking * queue_bytes(least) > share) least = cap;
+    if (limited && lacking * queue_bytes(least) > share)
+        return set_error(TN_ERR_OOM, "queues of %zu bytes, %zu are free", lacking * queue_bytes(least), free_bytes);
     for (int p = 0; p < npipes; ++p) {
         RenderBuffers& rb = rbs[p];
         if (rb.base && rb.q.cap >= cap) continue;
@@ -1721,7 +1726,6 @@ int check_render_params(const tn_render_params* P) {
 // per chunk 19.0, 2^23 17.7, 2^24 17.6.  2^25 entries are 13.6 GB a pipeline;
 // where that is more than a share of the free memory, half, down to the least.
 constexpr uint32_t kQueueEntries = 1u << 25, kLeastQueueEntries = 1u << 23;
-constexpr size_t kFreeShare = 4;  // new queues take at most a quarter of the free memory
 
 double path_fan(const tn_render_params* P) {
     double fan = 1;
@@ -1858,7 +1862,8 @@ int render_core(const RenderGeom& G, const std::vector<SceneParams>& table, uint
         hipError_t e_ = (call);                                          \
         if (e_ != hipSuccess) return fail(::tn::hip_error(e_, #call));   \
     } while (0)
-    while ((rc = reserve_queues(rbs, plan.npipes, plan.cap, entries > kLeastQueueEntries ? kFreeShare : 0))) {
+    const bool sized = shape.chunk || q.chunk_paths;  // by the caller
+    while ((rc = reserve_queues(rbs, plan.npipes, plan.cap, sized, entries > kLeastQueueEntries))) {
         if (rc != TN_ERR_OOM || entries <= kLeastQueueEntries) return rc;
         entries /= 2;
         if ((rc = plan_chunks(&q, shape.chunk, entries, total, most_pipes, !training, plan))) return rc;
