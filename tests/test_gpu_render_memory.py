@@ -63,3 +63,19 @@ print(json.dumps([f - free(), n, int(np.isfinite(img).all())]))
 """)
     # at most a quarter of 3 GiB goes to queues that this render does not need
     assert got[0] <= 768 * MB and got[1] == 64 * 64 * 7 and got[2]
+
+
+# 524,288 samples of 64 segments at the deepest level: 2 x 2^24 entries by default.
+# With 40 GiB free they would be a third of it, with 60 a quarter of it at most.
+@pytest.mark.parametrize("gib,most", [(40, 2 * 2**23 * 404), (60, 2 * 2**24 * 404)])
+def test_queues_take_a_share_of_the_free_memory(gpu, gib, most):
+    got = child.run(SETUP + """
+want, rays = render(t, sc, 1024, 512, 1, 4, 3, chunk_paths=20000)
+leave(int(sys.argv[1]) << 30)
+f = free()
+img, n = render(t, sc, 1024, 512, 1, 4, 3)
+# sums of one sample: at most 85 contributions each, in another order
+ok = bool(np.allclose(img, want, rtol=1e-5, atol=1e-6)) and n == rays == 1024 * 512 * 85
+print(json.dumps([f - free(), ok]))
+""", gib)
+    assert got[0] <= most + 64 * MB and got[1]
