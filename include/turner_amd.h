@@ -110,6 +110,9 @@ int tn_scene_create_with_tree(const float* verts9, const float* normals9,
  * of Triangle (lib/triangle.h:23-33, main.cpp:40-47), read by the raytracer
  * (raytracer.cpp:37-46).  Without this call every reflectivity is 0. */
 int tn_scene_set_reflection(tn_scene* scene, const float* reflective4, const float* reflectivity);
+/* The last scene or batch of a device to be destroyed gives back the memory
+ * that renders on it shared (ray queues, records, pinned tables) if it is more
+ * than 6.8 GB. */
 int tn_scene_destroy(tn_scene* scene);
 int tn_scene_get_info(const tn_scene* scene, tn_scene_info* info);
 /* Copies the reference-format FlatNode array (cap = capacity in nodes). */

@@ -1,5 +1,6 @@
-"""Device memory of the ray queues: what a first render takes, and what is left when
-little is free.  Each in a process of its own, in bytes that the driver reports free."""
+"""Device memory of the ray queues: what a first render takes, what is left when
+little is free, and that large queues go back with the last scene and batch of the
+device.  Each in a process of its own, in bytes that the driver reports free."""
 import pytest
 
 from tests import child
@@ -79,3 +80,29 @@ ok = bool(np.allclose(img, want, rtol=1e-5, atol=1e-6)) and n == rays == 1024 * 
 print(json.dumps([f - free(), ok]))
 """, gib)
     assert got[0] <= most + 64 * MB and got[1]
+
+
+def test_queues_go_back_with_the_last_scene_and_batch(gpu):
+    got = child.run(SETUP + """
+from turner_amd import batch
+other = tree_of(scenes.cornell_box())
+b = batch.Batch([t])
+render(t, sc, 64, 64, 1, 1, 2, chunk_paths=1024)  # streams and events stay
+jobs = [{"camera": sc["camera"], "lights": sc["lights"], "width": 64, "height": 64, "spp": 1}]
+f = free()
+img, n = render(t, sc, 1024, 512, 1, 4, 3)
+taken = f - free()
+t.close()
+other.close()
+kept = f - free()
+b.render(jobs, max_depth=2, mc_samples=1, flags=3, seed=1)
+b.close()
+back = f - free()
+t = tree_of(sc)
+again, n2 = render(t, sc, 1024, 512, 1, 4, 3)
+print(json.dumps([taken, kept, back, n == n2, bool(np.allclose(img, again, rtol=1e-5, atol=1e-6))]))
+""")
+    taken, kept, back, same, close = got
+    # beyond what may stay (2 x 2^23 entries), kept while a batch lives, then all of it back
+    assert taken > 2 * 2**23 * 404 and kept > 2 * 2**23 * 404 and back <= 64 * MB
+    assert same and close

@@ -744,6 +744,7 @@ int tn_scene_create(const float* verts9, const float* normals9, const float* alb
         free_device(sc.get());
         return set_error(TN_ERR_OOM, "host allocation failed during build");
     }
+    add_owner(sc->device);
     *out = sc.release();
     return TN_OK;
 }
@@ -774,6 +775,7 @@ int tn_scene_create_with_tree(const float* verts9, const float* normals9, const 
         free_device(sc.get());
         return set_error(TN_ERR_OOM, "host allocation failed");
     }
+    add_owner(sc->device);
     *out = sc.release();
     return TN_OK;
 }
@@ -794,6 +796,7 @@ int tn_scene_set_reflection(tn_scene* sc, const float* reflective4, const float*
 int tn_scene_destroy(tn_scene* sc) {
     if (!sc) return set_error(TN_ERR_INVALID, "scene is NULL");
     free_device(sc);
+    release_owner(sc->device);
     delete sc;
     return TN_OK;
 }

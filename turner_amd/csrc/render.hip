@@ -42,6 +42,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -1390,6 +1391,14 @@ std::vector<float> reference_jitter(uint32_t width, uint32_t spp) {
     return j;
 }
 
+// Queue entries a pipeline's deepest level may take by default (404 bytes each):
+// larger chunks are fewer launches, and fewer levels that only part of the chip
+// works on.  1920 x 1080 x 2, depth 3, m 4 at 2^23 entries 100.3 ms, 2^24 90.8,
+// 2^25 85.8, 2^26 83.7; m 2 18.1, 16.6, 16.5, 16.5; m 1 (8 samples) at 2^22 paths
+// per chunk 19.0, 2^23 17.7, 2^24 17.6.  2^25 entries are 13.6 GB a pipeline;
+// where that is more than a share of the free memory, half, down to the least.
+constexpr uint32_t kQueueEntries = 1u << 25, kLeastQueueEntries = 1u << 23;
+
 // Entries of a first allocation (1.7 GB), so that small renders of growing sizes
 // share it; not when the caller sizes the chunks, nor from scarce memory.
 constexpr uint32_t kLeastQueueAlloc = 1u << 22;
@@ -1422,7 +1431,8 @@ int ensure_side_stream(RenderBuffers& rb) {
 // Queues, streams and events of the renders on one device.  A render call
 // holds the context's lock from its first enqueued operation until its
 // streams have drained, so concurrent calls on one device take turns; the
-// buffers only grow (no allocation once a call of the same size has run).
+// buffers grow (no allocation once a call of the same size has run); large ones go
+// back with the last scene and batch of the device (release_owner).
 constexpr int kMaxDevices = 64;
 
 // Carves the queue buffers out of one allocation; with base == nullptr it
@@ -1542,6 +1552,7 @@ int alloc_records(RecordBuffers& rb, size_t slots) {
 
 struct RenderContext {
     std::mutex mu;
+    std::atomic<int> owners{0};  // scenes and batches of the device
     RenderBuffers rbs[kPipes];
     RecordBuffers recs[kPipes];
     // main streams of pipelines 1.. (pipeline 0 runs on the caller's stream)
@@ -1583,6 +1594,36 @@ bool reserve_host(RenderContext& C, size_t bytes) {
 RenderContext& render_context(int device) {
     static RenderContext ctx[kMaxDevices];
     return ctx[device];
+}
+
+// Gives back the context's device memory and pinned tables (its lock held, no render
+// under way) if that is more than the least default queues of all pipelines (6.8 GB).
+// A program that makes a scene, renders it and destroys it, again and again, thus
+// keeps the memory of small renders: 64 x 64 Cornell box 0.34 ms a turn, 0.84 with all
+// memory given back each time.  Large renders outweigh that (0.4 ms to allocate 27 GB,
+// 0.7 to free them).
+void release_memory(RenderContext& C) {
+    size_t held = C.jitter_cap * sizeof(float);
+    for (int p = 0; p < kPipes; ++p) held += C.rbs[p].bytes + C.recs[p].slots * 5 * sizeof(float4);
+    if (held <= kPipes * queue_bytes(kLeastQueueEntries)) return;
+    for (RenderBuffers& rb : C.rbs) {
+        (void)hipFree(rb.base);
+        (void)hipFree(rb.sp);
+        rb.base = nullptr;
+        rb.bytes = 0;
+        rb.sp = nullptr;
+        rb.sp_cap = 0;
+    }
+    for (RecordBuffers& r : C.recs) {
+        (void)hipFree(r.base);
+        r = RecordBuffers{};
+    }
+    (void)hipFree(C.jitter);
+    C.jitter = nullptr;
+    C.jitter_cap = 0;
+    if (C.host) (void)hipHostFree(C.host);
+    C.host = nullptr;
+    C.host_cap = 0;
 }
 
 __global__ void k_scale(const float4* __restrict__ a, float4* __restrict__ out, uint32_t n, float f) {
@@ -1718,14 +1759,6 @@ int check_render_params(const tn_render_params* P) {
     if ((uint32_t)P->max_depth + 2 > kMaxLevels) return set_error(TN_ERR_LIMIT, "max_depth too large");
     return TN_OK;
 }
-
-// Queue entries a pipeline's deepest level may take by default (404 bytes each):
-// larger chunks are fewer launches, and fewer levels that only part of the chip
-// works on.  1920 x 1080 x 2, depth 3, m 4 at 2^23 entries 100.3 ms, 2^24 90.8,
-// 2^25 85.8, 2^26 83.7; m 2 18.1, 16.6, 16.5, 16.5; m 1 (8 samples) at 2^22 paths
-// per chunk 19.0, 2^23 17.7, 2^24 17.6.  2^25 entries are 13.6 GB a pipeline;
-// where that is more than a share of the free memory, half, down to the least.
-constexpr uint32_t kQueueEntries = 1u << 25, kLeastQueueEntries = 1u << 23;
 
 double path_fan(const tn_render_params* P) {
     double fan = 1;
@@ -2383,6 +2416,22 @@ int autotune(tn_batch* b, const std::vector<SceneParams>& table, uint64_t total,
 }  // namespace
 }  // namespace tn
 
+namespace tn {
+
+void add_owner(int device) {
+    if (device >= 0 && device < kMaxDevices) ++render_context(device).owners;
+}
+
+void release_owner(int device) {
+    if (device < 0 || device >= kMaxDevices) return;
+    RenderContext& C = render_context(device);
+    if (--C.owners != 0) return;  // without the lock: renders of the others may be under way
+    std::lock_guard<std::mutex> lock(C.mu);
+    if (C.owners == 0) release_memory(C);
+}
+
+}  // namespace tn
+
 using namespace tn;
 
 extern "C" {
@@ -2574,6 +2623,7 @@ int tn_batch_create(tn_scene* const* scenes, uint32_t n, tn_batch** out) {
         delete b;
         return rc;
     }
+    add_owner(b->device);
     *out = b;
     return TN_OK;
 }
@@ -2583,6 +2633,7 @@ int tn_batch_destroy(tn_batch* b) {
     (void)hipSetDevice(b->device);
     (void)hipDeviceSynchronize();
     free_batch(b);
+    release_owner(b->device);
     delete b;
     return TN_OK;
 }

@@ -121,6 +121,11 @@ int hip_error(hipError_t e, const char* what);
 // for r < nrefs (every refs[r] indexes tris), on the null stream, and waits.
 int gather_leaf_records(const float4* tris, const uint32_t* refs, size_t nrefs, float4* out);
 
+// Scenes and batches of a device are counted: renders on it share memory that the
+// last one to be destroyed gives back.
+void add_owner(int device);
+void release_owner(int device);
+
 // Fixed launch shape of the traversal kernels: 256 lanes = 4 wave64.
 constexpr int kBlock = 256;
 constexpr int kStack = 8;
