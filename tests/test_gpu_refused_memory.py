@@ -1,5 +1,6 @@
 """Calls that use pinned host memory when they can get it, in a process where it is
-refused: they work as they do with it."""
+refused: they work as they do with it.  And a batch whose host memory is refused is an
+error, not an exception through the C interface."""
 import os
 import subprocess
 
@@ -67,3 +68,25 @@ c, sc_ = all_of()
 print(json.dumps([sa == sc_, all(bool(np.allclose(x, y, rtol=1e-5, atol=1e-6)) for x, y in zip(a, c)), sa[0] > 0]))
 """, refuse)
     assert got == [True, True, True]
+
+
+def test_batch_without_host_memory(gpu, refuse):
+    got = child.run(SETUP + """
+from turner_amd import _lib, batch
+tree = T.KDTree(scenes.intersect_scene(level=5)["verts"])
+before = torch.cuda.mem_get_info()[0]
+codes = []
+for size in (1 << 16, 1 << 18, 1 << 20):
+    shim.refuse_host_blocks(size)
+    try:
+        batch.Batch([tree])
+        codes.append(0)
+    except T.TurnerError as e:
+        codes.append(e.code)
+    shim.refuse_host_blocks(0)
+b = batch.Batch([tree])
+b.close()
+print(json.dumps([codes, before - torch.cuda.mem_get_info()[0], _lib.TN_ERR_OOM]))
+""", refuse)
+    codes, lost, oom = got
+    assert codes[0] == oom and set(codes) <= {0, oom} and lost <= 4 << 20

@@ -46,7 +46,9 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <type_traits>
 #include <vector>
 
@@ -2339,6 +2341,84 @@ void free_batch(tn_batch* b) {
         if (p) (void)hipFree(p);
 }
 
+// Packs n scenes (of one device, current) into b; what it allocated is freed by the
+// caller, also after an error.
+int fill_batch(tn_scene* const* scenes, uint32_t n, tn_batch* b) {
+    std::vector<DevNode> nodes;
+    std::vector<uint32_t> refs, eids;
+    std::vector<float> ecdf;
+    std::vector<SceneRoot> roots(n);
+    b->device = scenes[0]->device;
+    b->cus = scenes[0]->cus;
+    b->nscenes = n;
+    uint64_t ntri = 0;
+    std::vector<uint64_t> tri_base(n);
+    for (uint32_t s = 0; s < n; ++s) {
+        const tn_scene* sc = scenes[s];
+        tri_base[s] = ntri;
+        if (ntri + sc->ntris >= TN_INVALID_ID || nodes.size() + sc->tree.nodes.size() >= (1ull << 30) ||
+            refs.size() + sc->tree.refs.size() >= (1ull << 32))
+            return set_error(TN_ERR_LIMIT, "batch exceeds 2^30 triangles or nodes");
+        roots[s].node = (uint32_t)nodes.size();
+        for (int k = 0; k < 3; ++k) {
+            roots[s].bmin[k] = sc->tree.box[k];
+            roots[s].bmax[k] = sc->tree.box[3 + k];
+        }
+        append_tree(sc->tree, (uint32_t)nodes.size(), (uint32_t)refs.size(), (uint32_t)ntri, nodes, refs);
+        ntri += sc->ntris;
+        b->emit_begin.push_back((uint32_t)eids.size());
+        b->nemit.push_back(sc->nemit);
+        b->emit_area.push_back(sc->emit_area);
+        if (sc->nemit) {
+            std::vector<uint32_t> ids(sc->nemit);
+            std::vector<float> cdf(sc->nemit);
+            hipError_t e = hipMemcpy(ids.data(), sc->d_emit_ids, sc->nemit * 4, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy(cdf.data(), sc->d_emit_cdf, sc->nemit * 4, hipMemcpyDeviceToHost);
+            if (e != hipSuccess) return hip_error(e, "hipMemcpy");
+            for (uint32_t& i : ids) i += (uint32_t)tri_base[s];
+            eids.insert(eids.end(), ids.begin(), ids.end());
+            ecdf.insert(ecdf.end(), cdf.begin(), cdf.end());
+        }
+    }
+    std::vector<Treelet> treelets;
+    for (SceneRoot& r : roots) r.treelet = append_treelets(nodes, r.node, treelets);
+    hipError_t e;
+    const size_t nt = std::max<uint64_t>(ntri, 1);
+    if ((e = hipMalloc(&b->nodes, std::max<size_t>(nodes.size(), 1) * 8)) != hipSuccess ||
+        (e = hipMalloc(&b->treelets, treelets.size() * sizeof(Treelet))) != hipSuccess ||
+        (e = hipMalloc(&b->refs, std::max<size_t>(refs.size(), 1) * 4)) != hipSuccess ||
+        (e = hipMalloc(&b->tris, nt * 64)) != hipSuccess || (e = hipMalloc(&b->normals, nt * 36)) != hipSuccess ||
+        (e = hipMalloc(&b->albedo, nt * 16)) != hipSuccess || (e = hipMalloc(&b->emission, nt * 16)) != hipSuccess ||
+        (e = hipMalloc(&b->emit_ids, std::max<size_t>(eids.size(), 1) * 4)) != hipSuccess ||
+        (e = hipMalloc(&b->emit_cdf, std::max<size_t>(ecdf.size(), 1) * 4)) != hipSuccess ||
+        (e = hipMalloc(&b->roots, n * sizeof(SceneRoot))) != hipSuccess ||
+        (e = hipMalloc(&b->status, 4 * sizeof(uint32_t))) != hipSuccess)
+        return hip_error(e, "hipMalloc");
+    if ((e = hipMemset(b->status, 0, 4 * sizeof(uint32_t))) != hipSuccess) return hip_error(e, "hipMemset");
+    if ((e = hipMemcpy(b->nodes, nodes.data(), nodes.size() * 8, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(b->treelets, treelets.data(), treelets.size() * sizeof(Treelet), hipMemcpyHostToDevice)) !=
+            hipSuccess ||
+        (e = hipMemcpy(b->refs, refs.data(), refs.size() * 4, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(b->roots, roots.data(), n * sizeof(SceneRoot), hipMemcpyHostToDevice)) != hipSuccess ||
+        (!eids.empty() &&
+         (e = hipMemcpy(b->emit_ids, eids.data(), eids.size() * 4, hipMemcpyHostToDevice)) != hipSuccess) ||
+        (!ecdf.empty() &&
+         (e = hipMemcpy(b->emit_cdf, ecdf.data(), ecdf.size() * 4, hipMemcpyHostToDevice)) != hipSuccess))
+        return hip_error(e, "hipMemcpy");
+    for (uint32_t s = 0; s < n; ++s) {
+        const tn_scene* sc = scenes[s];
+        const size_t t0 = tri_base[s], k = sc->ntris;
+        if ((e = hipMemcpy(b->tris + 4 * t0, sc->d_tris, k * 64, hipMemcpyDeviceToDevice)) != hipSuccess ||
+            (e = hipMemcpy(b->normals + 9 * t0, sc->d_normals, k * 36, hipMemcpyDeviceToDevice)) != hipSuccess ||
+            (e = hipMemcpy(b->albedo + t0, sc->d_albedo, k * 16, hipMemcpyDeviceToDevice)) != hipSuccess ||
+            (e = hipMemcpy(b->emission + t0, sc->d_emission, k * 16, hipMemcpyDeviceToDevice)) != hipSuccess)
+            return hip_error(e, "hipMemcpy");
+    }
+    b->nrefs = refs.size();
+    if ((e = hipMalloc(&b->lrec, std::max<size_t>(b->nrefs, 1) * 64)) != hipSuccess) return hip_error(e, "hipMalloc");
+    return gather_leaf_records(b->tris, b->refs, b->nrefs, b->lrec);
+}
+
 int batch_table(const tn_batch* b, const tn_batch_job* jobs, std::vector<SceneParams>& table, uint64_t& total,
                 uint64_t& pixels) {
     table.resize(b->nscenes);
@@ -2535,96 +2615,20 @@ int tn_batch_create(tn_scene* const* scenes, uint32_t n, tn_batch** out) {
     for (uint32_t s = 0; s < n; ++s)
         if (scenes[s]->device != dev) return set_error(TN_ERR_INVALID, "scenes live on different devices");
     TN_HIP(hipSetDevice(dev));
-    std::vector<DevNode> nodes;
-    std::vector<uint32_t> refs, eids;
-    std::vector<float> ecdf;
-    std::vector<SceneRoot> roots(n);
-    tn_batch* b = new tn_batch();
-    b->device = dev;
-    b->cus = scenes[0]->cus;
-    b->nscenes = n;
-    uint64_t ntri = 0;
-    std::vector<uint64_t> tri_base(n);
-    for (uint32_t s = 0; s < n; ++s) {
-        const tn_scene* sc = scenes[s];
-        tri_base[s] = ntri;
-        if (ntri + sc->ntris >= TN_INVALID_ID || nodes.size() + sc->tree.nodes.size() >= (1ull << 30) ||
-            refs.size() + sc->tree.refs.size() >= (1ull << 32)) {
-            delete b;
-            return set_error(TN_ERR_LIMIT, "batch exceeds 2^30 triangles or nodes");
-        }
-        roots[s].node = (uint32_t)nodes.size();
-        for (int k = 0; k < 3; ++k) {
-            roots[s].bmin[k] = sc->tree.box[k];
-            roots[s].bmax[k] = sc->tree.box[3 + k];
-        }
-        append_tree(sc->tree, (uint32_t)nodes.size(), (uint32_t)refs.size(), (uint32_t)ntri, nodes, refs);
-        ntri += sc->ntris;
-        b->emit_begin.push_back((uint32_t)eids.size());
-        b->nemit.push_back(sc->nemit);
-        b->emit_area.push_back(sc->emit_area);
-        if (sc->nemit) {
-            std::vector<uint32_t> ids(sc->nemit);
-            std::vector<float> cdf(sc->nemit);
-            hipError_t e = hipMemcpy(ids.data(), sc->d_emit_ids, sc->nemit * 4, hipMemcpyDeviceToHost);
-            if (e == hipSuccess) e = hipMemcpy(cdf.data(), sc->d_emit_cdf, sc->nemit * 4, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) {
-                delete b;
-                return hip_error(e, "hipMemcpy");
-            }
-            for (uint32_t& i : ids) i += (uint32_t)tri_base[s];
-            eids.insert(eids.end(), ids.begin(), ids.end());
-            ecdf.insert(ecdf.end(), cdf.begin(), cdf.end());
-        }
+    std::unique_ptr<tn_batch> b(new (std::nothrow) tn_batch());
+    if (!b) return set_error(TN_ERR_OOM, "host allocation failed");
+    int rc;
+    try {
+        rc = fill_batch(scenes, n, b.get());
+    } catch (const std::bad_alloc&) {
+        rc = set_error(TN_ERR_OOM, "host allocation failed");
     }
-    std::vector<Treelet> treelets;
-    for (SceneRoot& r : roots) r.treelet = append_treelets(nodes, r.node, treelets);
-    auto fail = [&](hipError_t e, const char* what) {
-        free_batch(b);
-        delete b;
-        return hip_error(e, what);
-    };
-    hipError_t e;
-    const size_t nt = std::max<uint64_t>(ntri, 1);
-    if ((e = hipMalloc(&b->nodes, std::max<size_t>(nodes.size(), 1) * 8)) != hipSuccess ||
-        (e = hipMalloc(&b->treelets, treelets.size() * sizeof(Treelet))) != hipSuccess ||
-        (e = hipMalloc(&b->refs, std::max<size_t>(refs.size(), 1) * 4)) != hipSuccess ||
-        (e = hipMalloc(&b->tris, nt * 64)) != hipSuccess || (e = hipMalloc(&b->normals, nt * 36)) != hipSuccess ||
-        (e = hipMalloc(&b->albedo, nt * 16)) != hipSuccess || (e = hipMalloc(&b->emission, nt * 16)) != hipSuccess ||
-        (e = hipMalloc(&b->emit_ids, std::max<size_t>(eids.size(), 1) * 4)) != hipSuccess ||
-        (e = hipMalloc(&b->emit_cdf, std::max<size_t>(ecdf.size(), 1) * 4)) != hipSuccess ||
-        (e = hipMalloc(&b->roots, n * sizeof(SceneRoot))) != hipSuccess ||
-        (e = hipMalloc(&b->status, 4 * sizeof(uint32_t))) != hipSuccess)
-        return fail(e, "hipMalloc");
-    if ((e = hipMemset(b->status, 0, 4 * sizeof(uint32_t))) != hipSuccess) return fail(e, "hipMemset");
-    if ((e = hipMemcpy(b->nodes, nodes.data(), nodes.size() * 8, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(b->treelets, treelets.data(), treelets.size() * sizeof(Treelet), hipMemcpyHostToDevice)) !=
-            hipSuccess ||
-        (e = hipMemcpy(b->refs, refs.data(), refs.size() * 4, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(b->roots, roots.data(), n * sizeof(SceneRoot), hipMemcpyHostToDevice)) != hipSuccess ||
-        (!eids.empty() &&
-         (e = hipMemcpy(b->emit_ids, eids.data(), eids.size() * 4, hipMemcpyHostToDevice)) != hipSuccess) ||
-        (!ecdf.empty() &&
-         (e = hipMemcpy(b->emit_cdf, ecdf.data(), ecdf.size() * 4, hipMemcpyHostToDevice)) != hipSuccess))
-        return fail(e, "hipMemcpy");
-    for (uint32_t s = 0; s < n; ++s) {
-        const tn_scene* sc = scenes[s];
-        const size_t t0 = tri_base[s], k = sc->ntris;
-        if ((e = hipMemcpy(b->tris + 4 * t0, sc->d_tris, k * 64, hipMemcpyDeviceToDevice)) != hipSuccess ||
-            (e = hipMemcpy(b->normals + 9 * t0, sc->d_normals, k * 36, hipMemcpyDeviceToDevice)) != hipSuccess ||
-            (e = hipMemcpy(b->albedo + t0, sc->d_albedo, k * 16, hipMemcpyDeviceToDevice)) != hipSuccess ||
-            (e = hipMemcpy(b->emission + t0, sc->d_emission, k * 16, hipMemcpyDeviceToDevice)) != hipSuccess)
-            return fail(e, "hipMemcpy");
-    }
-    b->nrefs = refs.size();
-    if ((e = hipMalloc(&b->lrec, std::max<size_t>(b->nrefs, 1) * 64)) != hipSuccess) return fail(e, "hipMalloc");
-    if (int rc = gather_leaf_records(b->tris, b->refs, b->nrefs, b->lrec)) {
-        free_batch(b);
-        delete b;
+    if (rc) {
+        free_batch(b.get());
         return rc;
     }
-    add_owner(b->device);
-    *out = b;
+    add_owner(dev);
+    *out = b.release();
     return TN_OK;
 }
 
