@@ -376,7 +376,6 @@ void free_device(tn_scene* sc) {
     (void)hipFree(sc->d_refs);
     (void)hipFree(sc->d_tris);
     (void)hipFree(sc->d_lrec);
-    (void)hipFree(sc->d_fnodes);
     (void)hipFree(sc->d_ftreelets);
     (void)hipFree(sc->d_frefs);
     (void)hipFree(sc->d_flrec);
@@ -433,8 +432,6 @@ int finish_scene(tn_scene* sc, const float* verts9, const float* normals9, const
     if (sc->refined) {
         refine_reference_tree(verts9, sc->tree.nodes, sc->tree.refs, sc->tree.box, sc->parallel_build,
                               sc->fnodes, sc->frefs, sc->fheight);
-        if ((rc = dev_upload(&sc->d_fnodes, reinterpret_cast<const uint2*>(sc->fnodes.data()), sc->fnodes.size())))
-            return rc;
         if ((rc = upload_treelets(&sc->d_ftreelets, sc->fnodes))) return rc;
         if ((rc = dev_upload(&sc->d_frefs, sc->frefs.data(), sc->frefs.size()))) return rc;
         if ((rc = dev_upload<float4>(&sc->d_flrec, nullptr, 4 * sc->frefs.size()))) return rc;

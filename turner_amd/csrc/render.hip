@@ -2282,7 +2282,6 @@ void append_tree(const HostTree& t, uint32_t node_base, uint32_t ref_base, uint3
 struct tn_batch {
     int device = 0, cus = 256;
     uint32_t nscenes = 0;
-    uint2* nodes = nullptr;
     uint4* treelets = nullptr;
     uint32_t* refs = nullptr;
     float4* tris = nullptr;
@@ -2309,7 +2308,7 @@ struct tn_batch {
 
     tn::RenderGeom geom() const {
         tn::RenderGeom g;
-        g.sv.nodes = nodes;
+        g.sv.nodes = nullptr;
         g.sv.treelets = treelets;
         g.sv.refs = refs;
         g.sv.tris = tris;
@@ -2334,7 +2333,7 @@ namespace tn {
 namespace {
 
 void free_batch(tn_batch* b) {
-    for (void* p : {(void*)b->nodes, (void*)b->treelets, (void*)b->refs, (void*)b->tris, (void*)b->lrec, (void*)b->normals,
+    for (void* p : {(void*)b->treelets, (void*)b->refs, (void*)b->tris, (void*)b->lrec, (void*)b->normals,
                     (void*)b->albedo,
                     (void*)b->emission, (void*)b->emit_ids, (void*)b->emit_cdf, (void*)b->roots,
                     (void*)b->status})
@@ -2348,6 +2347,7 @@ int fill_batch(tn_scene* const* scenes, uint32_t n, tn_batch* b) {
     std::vector<uint32_t> refs, eids;
     std::vector<float> ecdf;
     std::vector<SceneRoot> roots(n);
+    std::vector<uint32_t> first_node(n);
     b->device = scenes[0]->device;
     b->cus = scenes[0]->cus;
     b->nscenes = n;
@@ -2359,7 +2359,7 @@ int fill_batch(tn_scene* const* scenes, uint32_t n, tn_batch* b) {
         if (ntri + sc->ntris >= TN_INVALID_ID || nodes.size() + sc->tree.nodes.size() >= (1ull << 30) ||
             refs.size() + sc->tree.refs.size() >= (1ull << 32))
             return set_error(TN_ERR_LIMIT, "batch exceeds 2^30 triangles or nodes");
-        roots[s].node = (uint32_t)nodes.size();
+        first_node[s] = (uint32_t)nodes.size();
         for (int k = 0; k < 3; ++k) {
             roots[s].bmin[k] = sc->tree.box[k];
             roots[s].bmax[k] = sc->tree.box[3 + k];
@@ -2381,11 +2381,10 @@ int fill_batch(tn_scene* const* scenes, uint32_t n, tn_batch* b) {
         }
     }
     std::vector<Treelet> treelets;
-    for (SceneRoot& r : roots) r.treelet = append_treelets(nodes, r.node, treelets);
+    for (uint32_t s = 0; s < n; ++s) roots[s].treelet = append_treelets(nodes, first_node[s], treelets);
     hipError_t e;
     const size_t nt = std::max<uint64_t>(ntri, 1);
-    if ((e = hipMalloc(&b->nodes, std::max<size_t>(nodes.size(), 1) * 8)) != hipSuccess ||
-        (e = hipMalloc(&b->treelets, treelets.size() * sizeof(Treelet))) != hipSuccess ||
+    if ((e = hipMalloc(&b->treelets, treelets.size() * sizeof(Treelet))) != hipSuccess ||
         (e = hipMalloc(&b->refs, std::max<size_t>(refs.size(), 1) * 4)) != hipSuccess ||
         (e = hipMalloc(&b->tris, nt * 64)) != hipSuccess || (e = hipMalloc(&b->normals, nt * 36)) != hipSuccess ||
         (e = hipMalloc(&b->albedo, nt * 16)) != hipSuccess || (e = hipMalloc(&b->emission, nt * 16)) != hipSuccess ||
@@ -2395,8 +2394,7 @@ int fill_batch(tn_scene* const* scenes, uint32_t n, tn_batch* b) {
         (e = hipMalloc(&b->status, 4 * sizeof(uint32_t))) != hipSuccess)
         return hip_error(e, "hipMalloc");
     if ((e = hipMemset(b->status, 0, 4 * sizeof(uint32_t))) != hipSuccess) return hip_error(e, "hipMemset");
-    if ((e = hipMemcpy(b->nodes, nodes.data(), nodes.size() * 8, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(b->treelets, treelets.data(), treelets.size() * sizeof(Treelet), hipMemcpyHostToDevice)) !=
+    if ((e = hipMemcpy(b->treelets, treelets.data(), treelets.size() * sizeof(Treelet), hipMemcpyHostToDevice)) !=
             hipSuccess ||
         (e = hipMemcpy(b->refs, refs.data(), refs.size() * 4, hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipMemcpy(b->roots, roots.data(), n * sizeof(SceneRoot), hipMemcpyHostToDevice)) != hipSuccess ||

@@ -157,7 +157,6 @@ __host__ __device__ __forceinline__ uint16_t to_bf16(float x) {
     return (uint16_t)(u >> 16);
 #endif
 }
-__device__ __forceinline__ float from_bf16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 typedef __attribute__((ext_vector_type(8))) __bf16 g_bf8;
 

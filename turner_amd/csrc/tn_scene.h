@@ -35,7 +35,6 @@ struct tn_scene {
     std::vector<tn::DevNode> fnodes;
     std::vector<uint32_t> frefs;
     uint32_t fheight = 0;
-    uint2* d_fnodes = nullptr;
     uint4* d_ftreelets = nullptr;
     uint32_t* d_frefs = nullptr;
     float4* d_flrec = nullptr;
@@ -81,7 +80,7 @@ struct tn_scene {
     // the refined tree (TN_SCENE_REFINED scenes only)
     tn::SceneView fview() const {
         tn::SceneView v = view();
-        v.nodes = d_fnodes;
+        v.nodes = nullptr;  // the per-lane kernels walk the reference tree
         v.treelets = d_ftreelets;
         v.refs = d_frefs;
         v.lra = d_flrec;

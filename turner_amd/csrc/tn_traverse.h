@@ -51,16 +51,15 @@ constexpr int kMaxRestarts = 4096;
 constexpr uint32_t kMaxLeafVisits = 1u << 22;
 
 // Root of one tree in a packed forest (many scenes in one node / reference /
-// triangle allocation): its node and treelet indices and root box.
+// triangle allocation): its first treelet and root box.
 struct SceneRoot {
-    uint32_t node;
     float bmin[3];
     float bmax[3];
     uint32_t treelet;
 };
 
 struct SceneView {
-    const uint2* nodes;
+    const uint2* nodes;  // of a single tree, for the per-lane kernels (else null)
     const uint4* treelets;  // the same tree two levels at a time (Treelet of tn_host.h, 2 uint4 each)
     const uint32_t* refs;
     const float4* tris;  // 4 per triangle
@@ -84,7 +83,7 @@ struct TraversalCounters {
 struct Trav {
     float3 o, d, dinv;
     float tenter, texit, root_exit;
-    uint32_t node, root;
+    uint32_t node;
     uint32_t leaf_off, leaf_left;  // triangle references still to test in the current leaf
     int head, count, restarts;
     uint32_t visits;  // leaves visited
@@ -295,11 +294,10 @@ __device__ __forceinline__ bool trav_init(Trav& T, const SceneView& sc, float3 o
     T.d = d;
     float lo, hi;
     const bool inside = root_clip(sc, o, d, 0, T.dinv, lo, hi);
-    T.root = 0;
     T.tenter = lo;
     T.texit = hi;
     T.root_exit = hi;
-    T.node = T.root;
+    T.node = 0;
     T.leaf_off = 0;
     T.leaf_left = 0;
     T.head = 0;
@@ -384,7 +382,7 @@ __device__ __forceinline__ bool trav_step(Trav& T, const SceneView& sc, float tm
             cnt.incomplete = true;
             return true;
         }
-        T.node = T.root;
+        T.node = 0;
         T.tenter = texit;
         T.texit = T.root_exit;
         T.lost = false;
@@ -497,7 +495,7 @@ leaf_done : {
             cnt.incomplete = true;
             return true;
         }
-        T.node = T.root;
+        T.node = 0;
         T.tenter = texit;
         T.texit = T.root_exit;
         T.lost = false;
