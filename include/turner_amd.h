@@ -278,7 +278,8 @@ typedef struct {
     float exposure;        /* --exposure */
     float inverse_gamma;   /* --inverse-gamma */
     int32_t gamma_enabled; /* !--no-gamma-correction */
-    uint32_t chunk_paths;  /* primary samples per wavefront chunk (0: automatic) */
+    uint32_t chunk_paths;  /* primary samples per wavefront chunk (0: automatic); a call of one chunk and at
+                              least 2^20 samples runs as two halves of it */
     uint32_t sample_offset;/* first pixel-sample index (progressive rendering) */
     uint32_t renderer;     /* TN_RENDERER_*: which of the reference's trace() plugins */
     float max_visibility;  /* raycaster --max-visibility (reference default 2) */

@@ -533,10 +533,15 @@ int launch_rays(tn_scene* sc, const float* o3, const float* d3, const float* tma
     uint32_t waves = (uint32_t)(((uint64_t)n + chunk - 1) / chunk);
     // Large cooperative launches hand out chunks of about 1/32 of a wave's
     // share from a work slot of the scene, so waves that draw cheap
-    // rays take more of them and all finish together (6,000,000 visibility rays
-    // 997 us against 1027 in equal shares, 2,000,000 425 against 412, 500,001 227
-    // against 185).  Not under stream capture (the slot's reuse is ordered by an
-    // event recorded outside).
+    // rays take more of them and all finish together.  The line lies just below
+    // where that begins to pay.  Microseconds in chunks / equal shares, 82 k triangles,
+    // refined tree, closest hits (visibility): 500,001 rays (227 / 185), 1,900,000
+    // 946 / 927 (726 / 713), 2,300,000 1065 / 1081 (833 / 843), 3,400,000 1427 / 1475
+    // (1102 / 1132), 6,200,000 2375 / 2556 (1810 / 1948).  With 5 k or 1.31 M
+    // triangles chunks cost up to 6 % at 1,900,000 rays, 3 % at 2.8 to 4.2 million,
+    // and gain 3 to 5 % at 6,200,000 (closest hits on 1.31 M: equal).
+    // Not under stream capture (the slot's reuse is ordered by an event recorded
+    // outside).
     uint32_t* work = nullptr;
     int wslot = -1;
     std::unique_lock<std::mutex> work_lock;

@@ -13,8 +13,8 @@
 //
 //   trace : closest hit for every queued segment (lane-refill traversal);
 //   shade : miss / emission / next-event estimation (shadow queue) and m
-//           children per hit (next queue), pushed with wave-aggregated
-//           atomics (ballot + mbcnt prefix);
+//           children per hit (next queue), in slots that a block reserves for
+//           all of its waves with one atomic (ballot + mbcnt prefix);
 //   shadow: visibility of the shadow queue (reference predicate
 //           !hit || r > dist, pathtracer.cpp:53); unoccluded contributions
 //           are added to the pixel's FP32 accumulator.
@@ -1790,15 +1790,19 @@ struct ChunkPlan {
 // concurrently, so that one's launch tails (the slowest rays of a level) overlap
 // the other's work.  A render of one chunk is split evenly between them when the
 // halves still fill the chip.  With the path tracer that is from 2^19 samples or
-// 2^23 segments at the deepest level (Cornell box 819,200 samples 0.87 ms whole,
-// 0.81 split; m 1, depth 6: 524,176 samples 2.43 and 2.34, 262,144 2.02 and 1.98,
-// but a batch of six small scenes of about as many 0.85 and 0.88; m 4, depth 3:
-// 65,536 samples 2.48 and 2.56, 259,200 7.2 and 6.6), with the raytracer, whose
-// levels thin out, from 2^20 (262,144 samples 0.68 and 0.73 ms, 524,176 0.78 and
-// 0.82, 2,079,604 1.33 with two).  Several chunks are made equal so that both
-// pipelines end together.  Neither holds for chunks that the caller sizes, nor
-// (`plain` false) for training renders: which records those keep depends on their
-// chunks.
+// 2^23 segments at the deepest level, from where on it paid in every render
+// measured, batches too (milliseconds whole / split: Cornell box 819,200 samples
+// 0.87 / 0.81; m 1, depth 6, 524,176 samples 2.43 / 2.34; m 4, depth 3, 259,200
+// samples 7.2 / 6.6; batches of six small scenes, depth 3: m 1, 529,056 samples 1.04 /
+// 0.98, 993,408 1.47 / 1.42, m 2, 529,056 2.17 / 2.14, m 4, 239,760 4.42 / 4.15).
+// Below it depends on the scene: m 1, 262,144 samples 2.02 / 1.98, but a batch of
+// 280,000 0.85 / 0.88; m 2, 131,044 samples 1.74 / 1.67; m 4, 36,864 samples 1.94 /
+// 1.88, but 65,536 2.48 / 2.56.  With the raytracer, whose levels thin out, it is from
+// 2^20 (262,144 samples 0.68 / 0.73, 524,176 0.78 / 0.82, 2,079,604 1.33 with two).
+// Several chunks are made equal so that both pipelines end together.  Chunks that
+// the caller sizes and those of training renders (`plain` false; which records
+// these keep depends on their chunks) are not made equal, and a single one is
+// split from 2^20 samples on.
 constexpr uint64_t kSplitPaths = 1u << 19, kSplitOther = 1u << 20;
 constexpr double kSplitEntries = 8388608.0;
 int plan_chunks(const tn_render_params* P, uint32_t requested, uint32_t entries, uint64_t total, int npipes,
