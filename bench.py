@@ -262,7 +262,9 @@ def main():
             "kernel": "k_rays_coop<closest hit, refined tree> (tn_intersect, TN_ISECT_REFINED)",
             "note": ("the refined tree's traversal reads %.0f algorithmic bytes per ray against the reference "
                      "tree's %.0f (reference_tree_traversal), so it reaches a lower fraction of the HBM roofline "
-                     "at %.2fx the rays/s: its launch is bound by the latency of dependent node fetches"
+                     "at %.2fx the rays/s: no unit is full (vector issue in 82 %% of the cycles, half of the lanes "
+                     "active, memory at 5.2 of the 6.45 TB/s that the reference tree's launch draws; "
+                     "profiles/k_rays_intersect_refined_level8_2p24.md)"
                      % (alg_bytes / n, ref_bytes / n, value / (n / (ref_ms * 1e-3) / 1e6))),
         },
         "reference_tree_traversal": {

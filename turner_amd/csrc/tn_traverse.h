@@ -635,11 +635,12 @@ __device__ __forceinline__ NodeStep node_step(const CoopRay& R, uint32_t split, 
 // after its round's atomics leaves the barycentrics in the owner's entry, so
 // the owner reads nothing but its slot.
 //
-// What bounds the loop: on the 2^24-ray batch (1.31 M triangles) the lines it
-// reads (27 GB per launch, 5.2 TB/s against 4.7 of a large copy); elsewhere
-// VALU issue (SIMDs 96 % busy before the last of the changes below) and, for
-// launches that leave the chip idle, the chain of dependent reads of the
-// longest rays.  Four rules keep both short:
+// What bounds the loop: where the scene is cached, VALU issue; in launches that
+// leave the chip idle, the chain of dependent reads of the longest rays.  On the
+// 2^24-ray batch (1.31 M triangles, refined tree) no unit is full: SIMDs issue in
+// 82 % of the cycles, for 49 % of the lanes, and 25.4 GB in 4.9 ms are 5.2 TB/s,
+// where the reference tree's launch of the same kernel draws 6.45 (66 GB, SIMDs 66 %
+// busy: that one is bound by the lines it reads).  Four rules keep all three short:
 //   * a round's descent stops when at most a third of the wave's rays are
 //     still on their way (they go on in the next round): the last lanes of a
 //     round take most of its dependent node reads.  2^24 rays: 8.03 ms with
