@@ -395,9 +395,9 @@ void free_device(tn_scene* sc) {
         if (e) (void)hipEventDestroy(e);
 }
 
-int upload_treelets(uint4** dst, const std::vector<DevNode>& nodes) {
-    std::vector<Treelet> t;
-    append_treelets(nodes, 0, t);
+int upload_treelets(uint4** dst, const std::vector<DevNode>& nodes, uint32_t* count = nullptr) {
+    const std::vector<Treelet> t = make_treelets(nodes);
+    if (count) *count = (uint32_t)t.size();
     return dev_upload(dst, reinterpret_cast<const uint4*>(t.data()), 2 * t.size());
 }
 
@@ -414,7 +414,7 @@ int finish_scene(tn_scene* sc, const float* verts9, const float* normals9, const
     if ((rc = dev_upload(&sc->d_nodes, reinterpret_cast<const uint2*>(sc->tree.nodes.data()),
                          sc->tree.nodes.size())))
         return rc;
-    if ((rc = upload_treelets(&sc->d_treelets, sc->tree.nodes))) return rc;
+    if ((rc = upload_treelets(&sc->d_treelets, sc->tree.nodes, &sc->ntreelets))) return rc;
     if ((rc = dev_upload(&sc->d_refs, sc->tree.refs.data(), sc->tree.refs.size()))) return rc;
     // device record: (v0, uv) (n, vv) (u, uu) (v, denom), one 64-byte line per triangle
     std::vector<float4> rec((size_t)n * 4);

@@ -833,16 +833,19 @@ bool flat_to_device(const std::vector<uint64_t>& flat, uint32_t ntris, std::vect
     return true;
 }
 
-uint32_t append_treelets(const std::vector<DevNode>& nodes, uint32_t root, std::vector<Treelet>& out) {
+std::vector<Treelet> make_treelets(const std::vector<DevNode>& nodes) {
     struct Item {
         uint32_t node, treelet;
     };
+    std::vector<Treelet> out;
+    // two for the root (the second stays unused) and for every inner node at an odd
+    // depth: no more than nodes, but two of a lone leaf
+    out.reserve(nodes.size() + 1);
     auto pair = [&] {
-        out.resize(out.size() + (out.size() & 1) + 2);
+        out.resize(out.size() + 2);
         return (uint32_t)out.size() - 2;
     };
-    const uint32_t first = pair();  // the second of the pair stays unused
-    std::vector<Item> todo{{root, first}};
+    std::vector<Item> todo{{0, pair()}};
     while (!todo.empty()) {
         const Item it = todo.back();
         todo.pop_back();
@@ -870,7 +873,7 @@ uint32_t append_treelets(const std::vector<DevNode>& nodes, uint32_t root, std::
         }
         out[it.treelet] = t;
     }
-    return first;
+    return out;
 }
 
 }  // namespace tn

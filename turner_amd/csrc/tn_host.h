@@ -61,9 +61,8 @@ void refine_reference_tree(const float* verts9, const std::vector<DevNode>& rnod
 void build_device_tree(const float* verts9, uint32_t n, bool parallel, std::vector<DevNode>& nodes,
                        std::vector<uint32_t>& refs, float box6[6], uint32_t& height);
 
-// Appends the treelets of the tree at nodes[root] (right children anywhere in
-// `nodes`) to `out` and returns the index of the first one.  Sibling treelets
+// The treelets of the tree `nodes` (root first), the root's first.  Sibling treelets
 // share a 64-byte line.
-uint32_t append_treelets(const std::vector<DevNode>& nodes, uint32_t root, std::vector<Treelet>& out);
+std::vector<Treelet> make_treelets(const std::vector<DevNode>& nodes);
 
 }  // namespace tn

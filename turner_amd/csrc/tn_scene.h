@@ -25,6 +25,7 @@ struct tn_scene {
     // device buffers (owned)
     uint2* d_nodes = nullptr;
     uint4* d_treelets = nullptr;  // the same tree, two levels per 32 bytes
+    uint32_t ntreelets = 0;
     uint32_t* d_refs = nullptr;
     float4* d_tris = nullptr;
     float4* d_lrec = nullptr;    // records per reference: 2 x nrefs first halves, then second halves
