@@ -106,3 +106,31 @@ print(json.dumps([taken, kept, back, n == n2, bool(np.allclose(img, again, rtol=
     # beyond what may stay (2 x 2^23 entries), kept while a batch lives, then all of it back
     assert taken > 2 * 2**23 * 404 and kept > 2 * 2**23 * 404 and back <= 64 * MB
     assert same and close
+
+
+def test_scenes_of_several_threads(gpu):
+    """Each thread makes a scene, renders it and destroys it, while the others do."""
+    got = child.run(SETUP + """
+import threading
+want, rays = render(t, sc, 1024, 512, 1, 4, 3)
+t.close()
+failed = []
+
+def turns():
+    try:
+        for _ in range(4):
+            mine = T.KDTree(sc["verts"], sc["normals"], sc["albedo"], sc["emission"])
+            img, n = render(mine, sc, 1024, 512, 1, 4, 3)
+            assert n == rays and np.allclose(img, want, rtol=1e-5, atol=1e-6)
+            mine.close()
+    except Exception as e:
+        failed.append(repr(e))
+
+threads = [threading.Thread(target=turns) for _ in range(3)]
+for x in threads:
+    x.start()
+for x in threads:
+    x.join()
+print(json.dumps(failed))
+""")
+    assert got == []
